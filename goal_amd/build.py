@@ -56,6 +56,7 @@ SOURCES = [
     "goal_amg.cpp",
     "goal_capi.cpp",
     "goal_assembly.hip",
+    "goal_cluster.hip",
     "goal_util.hip",
     "goal_graph.hip",
     "goal_dwr.hip",

@@ -22,6 +22,7 @@
 
 #include "goal_amg.hpp"
 #include "goal_expr.hpp"
+#include "goal_cluster.hpp"
 #include "goal_kernels.hpp"
 #include "goal_mesh.hpp"
 #include "goal_meshio.hpp"
@@ -221,12 +222,24 @@ struct AmgHierarchy {
   int coarse_n = 0;
 };
 
+// Node clusters of a quadratic disc (goal_cluster.hpp), made when the first
+// neo-Hookean four-point mechanics on it is; no runs where a node has more
+// neighbours than a run takes blocks, or no element.
+struct ClusterPlan {
+  int64_t num_runs = 0;
+  DevBuf<int4> runs, chunks;
+  DevBuf<uint32_t> elems;
+  DevBuf<goal::ClusterLane> lanes;
+  DevBuf<int32_t> nodes, conn;
+};
+
 struct goal_disc_s {
   goal::HostMesh mesh;
   std::vector<int64_t> node_adj_ptr;
   std::vector<int32_t> node_adj;          // host copy, made on demand (host_node_adj)
   DevBuf<int32_t> node_adj_dev;           // the columns as built on the device
   std::unique_ptr<AmgHierarchy> amg;
+  std::unique_ptr<ClusterPlan> cluster;
   int max_degree = 0;
   int64_t num_dofs = 0, nnz = 0;
   // gather plan: runs of consecutive nodes whose CSR values fit `gather_cap`
@@ -334,6 +347,7 @@ void disc_build(goal_disc d) {
   const int npe = m.nodes_per_elem;
   const int64_t nn = m.num_nodes, ne = m.num_elems, ns = ne * npe, np = ns * npe;
   d->amg.reset();
+  d->cluster.reset();
   d->coords.upload(m.coords.data(), (int64_t)m.coords.size());
   d->conn.upload(m.conn.data(), (int64_t)m.conn.size());
   d->elem_set.upload(m.elem_set.data(), (int64_t)m.elem_set.size());
@@ -427,6 +441,66 @@ void disc_build(goal_disc d) {
     std::swap(d->node_adj_dev.n, adj.n);
   }
   sync();  // the graph buffers are released on return
+}
+
+// The disc's node clusters: ordered by key, sized, then filled, on the device.
+void cluster_build(goal_disc d) {
+  auto p = std::make_unique<ClusterPlan>();
+  const int64_t nn = d->mesh.num_nodes, ne = d->mesh.num_elems;
+  if (d->max_degree <= goal::kClusterSlots && ne > 0) {
+    size_t tb = 0;
+    HIPCHK(goal::cluster_temp_bytes(std::max(nn, 10 * ne), &tb));
+    DevBuf<uint8_t> temp;
+    temp.alloc((int64_t)tb + 256);
+    DevBuf<unsigned long long> box;
+    DevBuf<int32_t> keys, sorted, rank, place, nr, nx, nk, most, nlanes;
+    DevBuf<int64_t> seg;
+    DevBuf<int2> recs, spans;
+    keys.alloc(nn);
+    sorted.alloc(nn);
+    box.alloc(6);
+    rank.alloc(nn);
+    place.alloc(nn);
+    p->nodes.alloc(nn);
+    seg.alloc(nn + 1);
+    HIPCHK(goal::cluster_order(d->conn.p, d->coords.p, ne, nn, temp.p, tb, box.p, keys.p, sorted.p, rank.p, place.p,
+                               p->nodes.p, seg.p, stream()));
+    const goal::ClusterMesh m{p->nodes.p, d->inc_ptr.p, d->inc.p, d->row_ptr.p, d->posi.p, d->pos.p, d->cols.p, place.p};
+    nr.alloc(nn + 1);
+    nx.alloc(nn + 1);
+    nk.alloc(nn + 1);
+    most.alloc(1);
+    HIPCHK(hipMemsetAsync(most.p, 0, sizeof(int32_t), stream()));
+    HIPCHK(goal::cluster_count(m, seg.p, nn, temp.p, tb, nr.p, nx.p, nk.p, most.p, stream()));
+    int32_t runs = 0, more = 0, nb = 0, lanes = 0;
+    HIPCHK(hipMemcpyAsync(&runs, nr.p + nn, sizeof(int32_t), hipMemcpyDeviceToHost, stream()));
+    HIPCHK(hipMemcpyAsync(&more, nx.p + nn, sizeof(int32_t), hipMemcpyDeviceToHost, stream()));
+    most.download(&nb, 1);
+    if (nb <= goal::kClusterSlots && runs > 0) {
+      const int64_t chunks = (int64_t)runs + more;
+      p->runs.alloc(runs);
+      p->chunks.alloc(chunks);
+      p->elems.alloc(chunks * goal::kClusterElems);
+      spans.alloc(chunks);
+      recs.alloc(10 * ne);
+      HIPCHK(goal::cluster_fill(m, seg.p, nn, nr.p, nx.p, nk.p, runs, p->runs.p, p->chunks.p, spans.p, p->elems.p,
+                                recs.p, stream()));
+      nlanes.alloc(chunks + 1);
+      HIPCHK(hipMemsetAsync(nlanes.p + chunks, 0, sizeof(int32_t), stream()));
+      HIPCHK(goal::cluster_lanes(m, runs, chunks, p->runs.p, p->chunks.p, spans.p, p->elems.p, recs.p, nlanes.p, temp.p,
+                                 tb, nullptr, stream()));
+      HIPCHK(hipMemcpyAsync(&lanes, nlanes.p + chunks, sizeof(int32_t), hipMemcpyDeviceToHost, stream()));
+      sync();
+      p->lanes.alloc(lanes);
+      HIPCHK(goal::cluster_lanes(m, runs, chunks, p->runs.p, p->chunks.p, spans.p, p->elems.p, recs.p, nlanes.p, temp.p,
+                                 tb, p->lanes.p, stream()));
+      p->conn.alloc(chunks * goal::kClusterElems * 10);
+      HIPCHK(goal::cluster_conn(chunks, p->chunks.p, p->elems.p, d->conn.p, p->conn.p, stream()));
+      p->num_runs = runs;
+    }
+    sync();  // the work buffers are released on return
+  }
+  d->cluster = std::move(p);
 }
 
 // The node adjacency's column lists on the host (the multigrid aggregation
@@ -621,11 +695,61 @@ int64_t point_states(goal_mech m, int kind) {
   return goal::point_state_doubles(m->d->mesh.num_elems * m->st->nq, goal::point_stride(kind));
 }
 
+// Whether the element matrices of an assembly are summed where they are formed
+// (one kernel over node clusters) instead of going through memory.
+bool clustered(goal_mech m, bool want_vals) {
+  return want_vals && m->tangent == 64 && m->model == goal::MODEL_NEOHOOKEAN && m->quad_order == 2 && m->d->cluster &&
+         m->d->cluster->num_runs > 0;
+}
+
+void run_clustered(goal_mech m, goal_solinfo s, int kind, const goal::AsmArgs& a) {
+  goal_disc d = m->d;
+  const ClusterPlan& p = *d->cluster;
+  goal::ClusterArgs c{};
+  c.num_runs = p.num_runs;
+  c.num_elems = a.num_elems;
+  c.runs = p.runs.p;
+  c.chunks = p.chunks.p;
+  c.chunk_elems = p.elems.p;
+  c.chunk_conn = p.conn.p;
+  c.lanes = p.lanes.p;
+  c.nodes = p.nodes.p;
+  c.row_ptr = d->row_ptr.p;
+  c.coords = a.coords;
+  c.x = a.x;
+  c.elem_set = a.elem_set;
+  c.mats = a.mats;
+  c.sigma = a.sigma;
+  c.R = s->R.p;
+  c.vals = s->vals.p;
+  c.overwrite_R = s->zero_R ? 1 : 0;
+  c.overwrite_vals = s->zero_vals ? 1 : 0;
+  c.stabilization = a.stabilization;
+  c.save_state = a.save_state;
+  c.xcd_remap = a.xcd_remap;
+  if (m->timing) HIPCHK(hipEventRecord(m->ev[0], stream()));
+  if (s->zero_dMdu) {
+    HIPCHK(goal::launch_fill(s->dMdu.p, s->dMdu.n, 0.0, stream()));
+    s->zero_dMdu = false;
+  }
+  HIPCHK(goal::launch_cluster(kind == goal::ASM_ADJOINT, c, asm_blocks(m), stream()));
+  if (m->timing) {  // all of it counts as the element pass: there is no gather
+    HIPCHK(hipEventRecord(m->ev[1], stream()));
+    HIPCHK(hipEventRecord(m->ev[2], stream()));
+    m->timed = true;
+  }
+  s->zero_R = s->zero_vals = false;
+}
+
 // With emr_buf given (and pt_buf for J2) the assembly also stays in one pass
 // (the chunked path keeps a host-side table it builds on first use); the two
 // give the same bits.
 void run_assembly(goal_mech m, goal_solinfo s, int kind, goal::AsmArgs a, bool want_vals, double* emr_buf = nullptr,
                   double* em_buf = nullptr, double* pt_buf = nullptr) {
+  if (clustered(m, want_vals)) {
+    run_clustered(m, s, kind, a);
+    return;
+  }
   const bool own_buffers = emr_buf == nullptr;
   goal_disc d = m->d;
   const int64_t nd = 4 * (int64_t)d->mesh.nodes_per_elem;
@@ -1904,6 +2028,7 @@ int goal_mech_create(goal_disc d, goal_states st, int num_sets, const goal_mater
     m->status.alloc(1);
     HIPCHK(hipMemsetAsync(m->status.p, 0, sizeof(int), stream()));
     m->elem_value.alloc(d->mesh.num_elems);
+    if (m->model == GOAL_MODEL_NEOHOOKEAN && d->mesh.order == 2 && quad_order == 2 && !d->cluster) cluster_build(d);
     sync();
     *out = m.release();
     return GOAL_OK;

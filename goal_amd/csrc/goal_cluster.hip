@@ -1,0 +1,799 @@
+// One-kernel assembly of residual and Jacobian for neo-Hookean quadratic tets
+// with four points, FP64: a workgroup forms all CSR rows of one run of nodes
+// (goal_cluster.hpp) from the nodal values, so no element matrix goes through
+// memory.
+//
+// Tangent in spatial form.  With F^{-T} dN/dX = f and F dN/dX = h per node,
+// c = mu J^{-2/3}, P = c F + s F^{-T}, s = p J - c tr(F F^T) / 3,
+// s2 = p J + 2/9 c tr(F F^T), pi = F^{-T} grad p, t = tau J (the closed form of
+// goal_device.hpp contracted with node a's gradient G_a):
+//   K(ai,bk) = s2 f_ai f_bk - 2/3 c (h_ai f_bk + f_ai h_bk) - s f_ak f_bi + c d_ik G_a.G_b
+//   K(ai,b3) = N_b J f_ai
+//   K(a3,bk) = N_a beta f_bk + t (f_a.pi f_bk - pi_k f_a.f_b - f_ak f_b.pi)
+//   K(a3,b3) = N_a N_b / kappa + t f_a.f_b
+//   R(ai) = c h_ai + s f_ai,   R(a3) = N_a r1 + t f_a.pi     (all times w dv, summed over the points)
+//
+// One lane forms the two 4 x 4 CSR blocks of a pair of nodes: it runs over the
+// elements that hold both and sums the blocks over their points in registers.
+//
+// Measured on the P2 64^3 cube (1.57 M tets; 7.8 GB of CSR values): 5.6 ms
+// against 12.7 ms for the element pass and the gather, whose 20.6 GB of element
+// matrices were written and read once.  HBM traffic 10.5 GB instead of 51.
+// Leaving out the blocks' sums takes 1.0-1.6 ms off, the point states 1.6-1.9,
+// the stores 1.4-1.7, and all three leave 1.1 ms: with four workgroups per CU
+// (LDS) the phases' latencies add up, the vector ALUs are busy for 2.7 ms.
+// Also measured:
+//   - sums in LDS by FP64 atomics, one lane per (element, row): 8.2 ms; an
+//     LDS FP64 atomic of a wave takes 48 cycles, half of them conflicts
+//   - one lane per block instead of per pair of blocks: 7.9 ms
+//   - a persistent grid, with the next chunk's plan fetched ahead or its point
+//     states formed by waves of their own: 9.5-9.9 ms
+//   - four waves per workgroup and at most two visits a lane: 5.9 ms; three
+//     waves, two visits: 5.7; the blocks stored by one lane each: 5.7;
+//     nontemporal stores: 9.5 (L2 no longer joins the rows' 32-byte pieces)
+#include <hipcub/hipcub.hpp>
+
+#include <algorithm>
+
+#include "goal_cluster.hpp"
+#include "goal_device.hpp"
+#include "goal_kernels.hpp"
+
+namespace goal {
+namespace {
+
+// ------------------------------------------------------------------- plan
+constexpr int kBlock = 256;
+
+inline unsigned grid_for(int64_t n) { return (unsigned)std::min<int64_t>(std::max<int64_t>((n + kBlock - 1) / kBlock, 1), 65536); }
+
+__device__ inline int edge_lo(int k) { return k < 3 ? k : k - 3; }  // edges 01, 12, 20, 03, 13, 23
+__device__ inline int edge_hi(int k) { return k < 3 ? (k == 2 ? 0 : k + 1) : 3; }
+
+// A double's bits as an integer that orders as the double does.
+__device__ inline unsigned long long ordered_bits(double v) {
+  const unsigned long long u = (unsigned long long)__double_as_longlong(v);
+  return (u >> 63) ? ~u : (u | 0x8000000000000000ull);
+}
+__device__ inline double from_ordered(unsigned long long u) {
+  return __longlong_as_double((long long)((u >> 63) ? (u & 0x7fffffffffffffffull) : ~u));
+}
+
+// box[0..2], [3..5]: smallest and largest coordinates (ordered_bits), zero and ~0 before
+__global__ __launch_bounds__(kBlock) void cluster_box_kernel(const double* X, int64_t nn, unsigned long long* box) {
+  unsigned long long lo[3] = {~0ull, ~0ull, ~0ull}, hi[3] = {0, 0, 0};
+  for (int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x; i < nn; i += (int64_t)gridDim.x * kBlock)
+    for (int c = 0; c < 3; ++c) {
+      const unsigned long long u = ordered_bits(X[3 * i + c]);
+      lo[c] = min(lo[c], u);
+      hi[c] = max(hi[c], u);
+    }
+  for (int c = 0; c < 3; ++c) {
+    for (int off = 32; off > 0; off >>= 1) {
+      lo[c] = min(lo[c], (unsigned long long)__shfl_xor((long long)lo[c], off, 64));
+      hi[c] = max(hi[c], (unsigned long long)__shfl_xor((long long)hi[c], off, 64));
+    }
+    if ((threadIdx.x & 63) == 0) {
+      atomicMin(&box[c], lo[c]);
+      atomicMax(&box[3 + c], hi[c]);
+    }
+  }
+}
+
+__device__ inline uint32_t spread3(uint32_t v) {  // ten bits, three apart
+  v = (v | (v << 16)) & 0x030000ff;
+  v = (v | (v << 8)) & 0x0300f00f;
+  v = (v | (v << 4)) & 0x030c30c3;
+  return (v | (v << 2)) & 0x09249249;
+}
+
+// Each node's place on a Morton curve through the mesh's box (cubic cells).
+__global__ __launch_bounds__(kBlock) void cluster_morton_kernel(const double* X, int64_t nn,
+                                                                const unsigned long long* box, uint32_t* code,
+                                                                int32_t* iota) {
+  double lo[3], size = 0.0;
+  for (int c = 0; c < 3; ++c) {
+    lo[c] = from_ordered(box[c]);
+    size = fmax(size, from_ordered(box[3 + c]) - lo[c]);
+  }
+  const double scale = size > 0.0 ? 1024.0 / size : 0.0;
+  for (int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x; i < nn; i += (int64_t)gridDim.x * kBlock) {
+    uint32_t v = 0;
+    for (int c = 0; c < 3; ++c) v |= spread3((uint32_t)fmin(fmax((X[3 * i + c] - lo[c]) * scale, 0.0), 1023.0)) << c;
+    code[i] = v;
+    iota[i] = (int32_t)i;
+  }
+}
+
+// pass 0: every node its own rank; 1: edge nodes cleared; 2: edge nodes the
+// smaller rank of their edge's vertices
+__global__ __launch_bounds__(kBlock) void cluster_keys_kernel(const int32_t* conn, int64_t ne, int64_t nn, int pass,
+                                                              const int32_t* rank, int32_t* keys, int32_t* iota) {
+  const int64_t n = pass == 0 ? nn : 6 * ne;
+  for (int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x; i < n; i += (int64_t)gridDim.x * kBlock) {
+    if (pass == 0) {
+      keys[i] = rank[i];
+      iota[i] = (int32_t)i;
+      continue;
+    }
+    const int32_t* c = conn + 10 * (i / 6);
+    const int k = (int)(i % 6);
+    if (pass == 1) keys[c[4 + k]] = INT32_MAX;
+    else atomicMin(&keys[c[4 + k]], min(rank[c[edge_lo(k)]], rank[c[edge_hi(k)]]));
+  }
+}
+
+__global__ __launch_bounds__(kBlock) void cluster_segments_kernel(const int32_t* keys, int64_t nn, int64_t* seg) {
+  for (int64_t a = (int64_t)blockIdx.x * kBlock + threadIdx.x; a <= nn; a += (int64_t)gridDim.x * kBlock) {
+    int64_t lo = 0, hi = nn;
+    while (lo < hi) {
+      const int64_t mid = (lo + hi) >> 1;
+      if (keys[mid] < a) lo = mid + 1;
+      else hi = mid;
+    }
+    seg[a] = lo;
+  }
+}
+
+__global__ __launch_bounds__(kBlock) void cluster_place_kernel(const int32_t* nodes, int64_t nn, int32_t* place) {
+  for (int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x; i < nn; i += (int64_t)gridDim.x * kBlock)
+    place[nodes[i]] = (int32_t)i;
+}
+
+__global__ __launch_bounds__(kBlock) void cluster_count_kernel(ClusterMesh m, const int64_t* seg, int64_t nn,
+                                                               int32_t* runs, int32_t* more, int32_t* recs,
+                                                               int32_t* most) {
+  for (int64_t a = (int64_t)blockIdx.x * kBlock + threadIdx.x; a <= nn; a += (int64_t)gridDim.x * kBlock) {
+    ClusterCount c;
+    if (a < nn && seg[a] < seg[a + 1]) walk_cluster(m, seg[a], seg[a + 1], c);
+    runs[a] = c.runs;
+    more[a] = c.chunks > c.runs ? c.chunks - c.runs : 0;
+    recs[a] = c.recs;
+    if (c.most > *most) atomicMax(most, c.most);
+  }
+}
+
+__global__ __launch_bounds__(kBlock) void cluster_fill_kernel(ClusterMesh m, const int64_t* seg, int64_t nn,
+                                                              const int32_t* runs, const int32_t* more,
+                                                              const int32_t* recs, int64_t num_runs, int4* run_tab,
+                                                              int4* chunk_tab, int2* span_tab, uint32_t* elem_tab,
+                                                              int2* rec_tab) {
+  for (int64_t a = (int64_t)blockIdx.x * kBlock + threadIdx.x; a < nn; a += (int64_t)gridDim.x * kBlock) {
+    if (seg[a] == seg[a + 1]) continue;
+    ClusterFill f;
+    f.runs = run_tab;
+    f.chunks = chunk_tab;
+    f.spans = span_tab;
+    f.elems = elem_tab;
+    f.recs = rec_tab;
+    f.r = runs[a];
+    f.x = (int)num_runs + more[a];
+    f.k = recs[a];
+    walk_cluster(m, seg[a], seg[a + 1], f);
+  }
+}
+
+// One workgroup per run: the pairs of each of its chunks, one thread per
+// (row node, position), the visits of a pair in incidence order.
+__global__ __launch_bounds__(kBlock) void cluster_lanes_kernel(ClusterMesh m, const int4* run_tab, int4* chunk_tab,
+                                                               const int2* span_tab, const uint32_t* elem_tab,
+                                                               const int2* recs, int32_t* nlanes,
+                                                               ClusterLane* lanes) {
+  __shared__ int first[kClusterNodes + 1];               // first block of a node
+  __shared__ int rlo[kClusterNodes], rhi[kClusterNodes];  // a node's incidences in the chunk
+  __shared__ uint16_t cnt[kClusterSlots];
+  __shared__ int total;
+  const int tid = threadIdx.x;
+  const int4 run = run_tab[blockIdx.x];
+  const int nn = run.y - run.x;
+  if (tid == 0) {
+    int s = 0;
+    for (int i = 0; i < nn; ++i) {
+      const int64_t n = m.nodes[run.x + i];
+      first[i] = s;
+      s += (int)((m.row_ptr[4 * n + 1] - m.row_ptr[4 * n]) / 4);
+    }
+    first[nn] = s;
+  }
+  __syncthreads();
+  const int nb = first[nn];
+  for (int c = (int)blockIdx.x, nxt = run.z;; c = nxt++) {
+    const int2 span = span_tab[c];
+    if (tid < nn) rlo[tid] = rhi[tid] = 0;
+    if (tid == 0) total = 0;
+    __syncthreads();
+    for (int t = span.x + tid; t < span.y; t += kBlock) {
+      const int node = recs[t].y >> 16;
+      if (t == span.x || (recs[t - 1].y >> 16) != node) rlo[node] = t;
+      if (t + 1 == span.y || (recs[t + 1].y >> 16) != node) rhi[node] = t + 1;
+    }
+    __syncthreads();
+    for (int s = tid; s < nb; s += kBlock) {
+      int node = 0;
+      while (first[node + 1] <= s) ++node;
+      const int pos = s - first[node];
+      const int64_t ga = m.nodes[run.x + node], gb = m.cols[m.row_ptr[4 * ga] + 4 * pos] / 4;
+      int n = 0;
+      if (m.place[gb] >= m.place[ga])  // else the pair is b's run's
+        for (int t = rlo[node]; t < rhi[node]; ++t)
+          for (int b = 0; b < 10; ++b) n += m.posi[10 * (int64_t)recs[t].x + b] == pos;
+      cnt[s] = (uint16_t)n;
+      if (n) atomicAdd(&total, 1 << cluster_log_lanes(n));
+    }
+    __syncthreads();
+    if (!lanes) {
+      if (tid == 0) nlanes[c] = (total + 63) / 64 * 64;
+    } else {
+      const int base = nlanes[c], end = nlanes[c + 1];
+      if (tid == 0) {
+        chunk_tab[c].y = base;
+        chunk_tab[c].z = end;
+      }
+      for (int t = base + total + tid; t < end; t += kBlock) lanes[t] = ClusterLane{0, 0};  // idle lanes: no visits
+      for (int s = tid; s < nb; s += kBlock) {
+        const int n = cnt[s];
+        if (!n) continue;
+        const int rank = cluster_rank(n), lg = cluster_log_lanes(n);
+        int lane = 0;
+        for (int u = 0; u < nb; ++u) {
+          const int nu = cnt[u];
+          if (!nu) continue;
+          const int ru = cluster_rank(nu);
+          if (ru < rank || (ru == rank && u < s)) lane += 1 << cluster_log_lanes(nu);
+        }
+        int node = 0;
+        while (first[node + 1] <= s) ++node;
+        const int pos = s - first[node];
+        // an earlier chunk of the run that adds to this pair holds an earlier incidence of its node
+        const int64_t ga = m.nodes[run.x + node], gb = m.cols[m.row_ptr[4 * ga] + 4 * pos] / 4;
+        bool earlier = false;
+        for (int64_t k = m.inc_ptr[ga]; k < recs[rlo[node]].x; ++k)
+          for (int b = 0; b < 10; ++b) earlier |= m.posi[10 * k + b] == pos;
+        int pos_t = 0;
+        // lane j's visits, in incidence order
+        for (int j = 0; j < (1 << lg); ++j) {
+          uint64_t w = 0;
+          int at = 0, mine = 0;
+          for (int t = rlo[node]; t < rhi[node]; ++t) {
+            const int2 rec = recs[t];
+            const int a = (rec.y >> 8) & 255, el = rec.y & 31;
+            for (int b = 0; b < 10; ++b)
+              if (m.posi[10 * (int64_t)rec.x + b] == pos) {
+                const int64_t e = elem_tab[(int64_t)c * kClusterElems + el] & ~kClusterOwned;
+                pos_t = m.pos[(10 * e + b) * 10 + a];
+                if ((at++ & ((1 << lg) - 1)) == j) w |= (uint64_t)(el | (a << 5) | (b << 9)) << (13 * mine++);
+              }
+          }
+          ClusterLane o;
+          o.x = w | ((uint64_t)mine << kLaneCount) | ((uint64_t)pos << kLanePos) | ((uint64_t)node << kLaneNode) |
+                ((uint64_t)lg << kLaneLog) | (earlier ? 0 : kLaneFirst) | (ga == gb ? kLaneDiag : 0);
+          const int64_t rb = m.row_ptr[4 * gb];
+          o.y = (uint64_t)(rb / 16) | ((uint64_t)((m.row_ptr[4 * gb + 1] - rb) / 4) << kLaneDegT) |
+                ((uint64_t)pos_t << kLanePosT);
+          lanes[base + lane + j] = o;
+        }
+      }
+    }
+    __syncthreads();
+    if (nxt >= run.w) break;
+  }
+}
+
+__global__ __launch_bounds__(kBlock) void cluster_conn_kernel(int64_t num_chunks, const int4* chunk_tab,
+                                                              const uint32_t* elem_tab, const int32_t* conn,
+                                                              int32_t* chunk_conn) {
+  const int64_t n = num_chunks * kClusterElems * 10;
+  for (int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x; i < n; i += (int64_t)gridDim.x * kBlock) {
+    const int64_t s = i / 10, c = s / kClusterElems;
+    const bool live = s % kClusterElems < chunk_tab[c].x;
+    chunk_conn[i] = live ? conn[10 * (int64_t)(elem_tab[s] & ~kClusterOwned) + i % 10] : 0;
+  }
+}
+
+// --------------------------------------------------------------- assembly
+constexpr double kA = 0.5854101966249685, kB = 0.1381966011250105;  // lambda of the four points
+
+// LDS table of one element, per point: f_a = F^{-T} grad N_a of the ten nodes
+// (three each), dev(F F^T) (xx xy xz yy yz zz) and the scalars below (times
+// w dv: c, c tr(F F^T)/3, p J, J, beta, tau J, 1/kappa, r1; and pi).  Odd
+// strides spread the elements over the LDS banks.
+enum : int { oF = 0, oDev = 30, oC = 36, oCT, oPJ, oJ, oBeta, oT, oPi, oKap = oPi + 3, oR1, kPt };
+constexpr int kElemStride = 4 * kPt + 1;
+static_assert(kPt == 47 && kElemStride % 2 == 1, "odd strides");
+__device__ constexpr int sym(int i, int j) { return (i < j ? i : j) + (i > j ? i : j) + (i > 0 && j > 0 ? 1 : 0); }
+
+__device__ inline double lam_at(int v, int q) { return v == q ? kA : kB; }
+
+__device__ inline int64_t run_of(int64_t it, int64_t n, int remap) {
+  const int64_t nb = gridDim.x, b = blockIdx.x;
+  if (!remap || (nb & 7)) {
+    const int64_t g = b + it * nb;
+    return g < n ? g : -1;
+  }
+  // XCD x (workgroups go round the eight XCDs) takes the x-th eighth of the runs
+  const int64_t per = (n + 7) >> 3, g = (b >> 3) + it * (nb >> 3);
+  if (g >= per) return -1;
+  const int64_t r = (b & 7) * per + g;
+  return r < n ? r : -1;
+}
+
+// Stage ends: pin() forces a value here, stage_end() keeps later loads and
+// arithmetic behind.  Left alone, the compiler starts the loads of all stages
+// at once and spills at the 168 registers that three waves per SIMD leave
+// (13 spilled registers were 3 GB of scratch traffic per assembly; with the
+// stages apart the kernel takes 140 and spills none).
+__device__ __forceinline__ void pin(double& v) { asm volatile("" : "+v"(v)); }
+template <int N>
+__device__ __forceinline__ void pin(double (&v)[N]) {
+#pragma unroll
+  for (int k = 0; k < N; ++k) pin(v[k]);
+}
+__device__ __forceinline__ void stage_end() {
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_sched_barrier(0);
+}
+
+// The state of point q of element e (nodes ec), into its part of the element's
+// table.
+__device__ __forceinline__ void point_state(const ClusterArgs& a, int64_t e, const int32_t* ec, int q, bool owned,
+                                            double* pe) {
+  const MatParams mp = a.mats[a.elem_set ? a.elem_set[e] : 0];
+  double lam[4];
+#pragma unroll
+  for (int v = 0; v < 4; ++v) lam[v] = lam_at(v, q);
+  // U[v] = sum_n (dN_n / d lambda_v) x_n, so that grad x = sum_v U[v] grad lambda_v
+  double U[4][4], p = 0.0;
+#pragma unroll
+  for (int v = 0; v < 4; ++v) {
+    const double* xn = a.x + 4 * (int64_t)ec[v];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) U[v][i] = (4.0 * lam[v] - 1.0) * xn[i];
+    p += lam[v] * (2.0 * lam[v] - 1.0) * xn[3];
+  }
+#pragma unroll
+  for (int k = 0; k < 6; ++k) {
+    if (k == 2) stage_end();
+    const int i = k < 3 ? k : k - 3, j = k < 3 ? (k == 2 ? 0 : k + 1) : 3;
+    const double* xn = a.x + 4 * (int64_t)ec[4 + k];
+#pragma unroll
+    for (int d = 0; d < 4; ++d) {
+      U[i][d] += 4.0 * lam[j] * xn[d];
+      U[j][d] += 4.0 * lam[i] * xn[d];
+    }
+    p += 4.0 * lam[i] * lam[j] * xn[3];
+  }
+  // differences first (the four gradients sum to zero): a rigid part of x drops out exactly
+  double D[12];
+#pragma unroll
+  for (int v = 1; v < 4; ++v)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) D[4 * (v - 1) + i] = U[v][i] - U[0][i];
+  pin(D);
+  pin(p);
+  stage_end();
+  double F[9], gp[3], gl[4][3], tau, det;
+  {
+    double X[4][3];
+#pragma unroll
+    for (int v = 0; v < 4; ++v)
+#pragma unroll
+      for (int c = 0; c < 3; ++c) X[v][c] = a.coords[3 * (int64_t)ec[v] + c];
+    det = dev::tet_gradlambda(X, gl);
+    tau = a.stabilization ? dev::stab_tau(X, mp) : 0.0;
+  }
+#pragma unroll
+  for (int J = 0; J < 3; ++J) {
+#pragma unroll
+    for (int i = 0; i < 3; ++i)
+      F[3 * i + J] = (i == J ? 1.0 : 0.0) + (D[i] * gl[1][J] + D[4 + i] * gl[2][J] + D[8 + i] * gl[3][J]);
+    gp[J] = D[3] * gl[1][J] + D[7] * gl[2][J] + D[11] * gl[3][J];
+  }
+  pin(F);
+  pin(gp);
+  pin(tau);
+  pin(det);
+  stage_end();
+  double* o = pe + kPt * q;
+  const double J = dev::det3(F), iJ = 1.0 / J, W = det / 24.0;
+  {
+    double b[6];  // F F^T
+#pragma unroll
+    for (int i = 0; i < 3; ++i)
+#pragma unroll
+      for (int j = i; j < 3; ++j)
+        b[sym(i, j)] = F[3 * i] * F[3 * j] + F[3 * i + 1] * F[3 * j + 1] + F[3 * i + 2] * F[3 * j + 2];
+    const double trb = b[0] + b[3] + b[5], third = trb / 3.0;
+    b[0] -= third;
+    b[3] -= third;
+    b[5] -= third;
+    const double Jm13 = 1.0 / cbrt(J), Jm23 = Jm13 * Jm13;
+    if (owned) {
+      const double m = mp.mu * (Jm23 * Jm23 * Jm13);
+      double* sg = a.sigma + 4 * e + q;
+#pragma unroll
+      for (int k = 0; k < 9; ++k) sg[k * 4 * a.num_elems] = m * b[sym(k / 3, k % 3)] + (k % 4 == 0 ? p : 0.0);
+    }
+#pragma unroll
+    for (int k = 0; k < 6; ++k) o[oDev + k] = b[k];
+    const double C = W * (mp.mu * Jm23);
+    o[oC] = C;
+    o[oCT] = C * third;
+  }
+  o[oPJ] = W * (p * J);
+  o[oJ] = W * J;
+  o[oBeta] = W * (-0.5 * (J + iJ));
+  o[oT] = W * J * tau;
+  o[oKap] = W / mp.kappa;
+  o[oR1] = W * (p / mp.kappa - 0.5 * (J - iJ));
+  stage_end();
+  double Fi[9], phi[4][3];
+  dev::inv3(F, J, Fi);
+#pragma unroll
+  for (int k = 0; k < 3; ++k) o[oPi + k] = Fi[k] * gp[0] + Fi[3 + k] * gp[1] + Fi[6 + k] * gp[2];
+#pragma unroll
+  for (int v = 0; v < 4; ++v)
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+      phi[v][k] = Fi[k] * gl[v][0] + Fi[3 + k] * gl[v][1] + Fi[6 + k] * gl[v][2];
+      o[oF + 3 * v + k] = (4.0 * lam[v] - 1.0) * phi[v][k];
+    }
+#pragma unroll
+  for (int k = 0; k < 6; ++k) {
+    const int i = k < 3 ? k : k - 3, j = k < 3 ? (k == 2 ? 0 : k + 1) : 3;
+#pragma unroll
+    for (int d = 0; d < 3; ++d) o[oF + 12 + 3 * k + d] = 4.0 * (lam[i] * phi[j][d] + lam[j] * phi[i][d]);
+  }
+}
+
+// N_a at point q (vertices: lambda (2 lambda - 1), edges: 4 lambda_i lambda_j).
+__device__ inline double shape_at(int a, int q) {
+  if (a < 4) return lam_at(a, q) * (2.0 * lam_at(a, q) - 1.0);
+  return 4.0 * lam_at(edge_lo(a - 4), q) * lam_at(edge_hi(a - 4), q);
+}
+
+// The sums of a pair {a, b}: uu[3 i + k] = K(ai, bk) (= K(bk, ai)), pp = K(a3,
+// b3), and both blocks' pressure columns and rows; r: the residual of a = b.
+struct PairSum {
+  double uu[9], pp, ab_c[3], ab_r[3], ba_c[3], ba_r[3], r[4];
+  template <typename F>
+  __device__ __forceinline__ void each(F f) {
+#pragma unroll
+    for (int k = 0; k < 9; ++k) f(uu[k]);
+    f(pp);
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+      f(ab_c[k]);
+      f(ab_r[k]);
+      f(ba_c[k]);
+      f(ba_r[k]);
+    }
+#pragma unroll
+    for (int k = 0; k < 4; ++k) f(r[k]);
+  }
+};
+
+// Adds one visit: element table P, local nodes la and lb; shape[4 a + q] = N_a
+// at point q.
+__device__ __forceinline__ void visit(const double* P, const double* shape, int la, int lb, bool diag, PairSum& s) {
+#pragma unroll 1
+  for (int q = 0; q < 4; ++q) {
+    const double* p = P + kPt * q;
+    double fa[3], fb[3], ha[3], hb[3];
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+      fa[k] = p[oF + 3 * la + k];
+      fb[k] = p[oF + 3 * lb + k];
+    }
+    {
+      double dv[6];
+#pragma unroll
+      for (int k = 0; k < 6; ++k) dv[k] = p[oDev + k];
+#pragma unroll
+      for (int j = 0; j < 3; ++j) {
+        ha[j] = dv[sym(j, 0)] * fa[0] + dv[sym(j, 1)] * fa[1] + dv[sym(j, 2)] * fa[2];
+        hb[j] = dv[sym(j, 0)] * fb[0] + dv[sym(j, 1)] * fb[1] + dv[sym(j, 2)] * fb[2];
+      }
+    }
+    const double d = fa[0] * fb[0] + fa[1] * fb[1] + fa[2] * fb[2];
+    {
+      const double C = p[oC], CT = p[oCT], PJ = p[oPJ];
+      const double hd = ha[0] * fb[0] + ha[1] * fb[1] + ha[2] * fb[2];
+      const double m = (-2.0 / 3.0) * C, A = PJ - (2.0 / 3.0) * CT, S = CT - PJ, gg = C * hd + CT * d;
+      if (diag) {
+#pragma unroll
+        for (int i = 0; i < 3; ++i) s.r[i] += C * ha[i] + PJ * fa[i];
+      }
+#pragma unroll
+      for (int i = 0; i < 3; ++i) {
+        const double u = m * ha[i] + A * fa[i], v = m * fa[i], w = S * fb[i];
+#pragma unroll
+        for (int k = 0; k < 3; ++k) s.uu[3 * i + k] += u * fb[k] + v * hb[k] + w * fa[k];
+        s.uu[4 * i] += gg;
+      }
+    }
+    pin(s.uu);
+    stage_end();
+    const double Na = shape[4 * la + q], Nb = shape[4 * lb + q];
+    const double J = p[oJ], be = p[oBeta], t = p[oT];
+    const double pi[3] = {p[oPi], p[oPi + 1], p[oPi + 2]};
+    const double pa = pi[0] * fa[0] + pi[1] * fa[1] + pi[2] * fa[2];
+    const double pb = pi[0] * fb[0] + pi[1] * fb[1] + pi[2] * fb[2];
+    const double td = t * d, ta = t * pa, tb = t * pb;
+    const double ja = J * Na, jb = J * Nb, al = be * Na + ta, bl = be * Nb + tb;
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {
+      s.ab_c[i] += jb * fa[i];
+      s.ba_c[i] += ja * fb[i];
+      const double tp = td * pi[i];
+      s.ab_r[i] += al * fb[i] - tb * fa[i] - tp;
+      s.ba_r[i] += bl * fa[i] - ta * fb[i] - tp;
+    }
+    s.pp += td + p[oKap] * (Na * Nb);
+    if (diag) s.r[3] += p[oR1] * Na + ta;
+  }
+}
+
+// v + the partner's v for lanes that share a block, by step: 0: lane ^ 1, 1:
+// lane ^ 2, 2 and 3: the mirrored lane of 8 and of 16 (whose sums agree with
+// lane ^ 4 and ^ 8 by then).
+template <int STEP>
+__device__ inline double partner(double v) {
+  constexpr int ctrl = STEP == 0 ? 0xB1 : STEP == 1 ? 0x4E : STEP == 2 ? 0x141 : 0x140;
+  const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), ctrl, 0xF, 0xF, true);
+  const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), ctrl, 0xF, 0xF, true);
+  return __hiloint2double(hi, lo);
+}
+template <int STEP>
+__device__ __forceinline__ void join(int lg, PairSum& s) {
+  s.each([&](double& v) {
+    const double o = partner<STEP>(v);
+    if (lg > STEP) v += o;
+  });
+}
+
+// Where a lane's 4 x 4 block goes: rows len apart, 32-byte aligned; at = 0: none.
+struct BlockPlace {
+  uint64_t at;
+  int len, set;  // set: store, else add
+  __device__ __forceinline__ BlockPlace other() const {  // the neighbour lane's (lane ^ 1)
+    BlockPlace o;
+    const uint32_t lo = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)at, 0xB1, 0xF, 0xF, true);
+    const uint32_t hi = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)(at >> 32), 0xB1, 0xF, 0xF, true);
+    o.at = lo | ((uint64_t)hi << 32);
+    o.len = __builtin_amdgcn_update_dpp(0, len, 0xB1, 0xF, 0xF, true);
+    o.set = __builtin_amdgcn_update_dpp(0, set, 0xB1, 0xF, 0xF, true);
+    return o;
+  }
+  __device__ __forceinline__ void put(int i, int half, double2 v) const {
+    if (!at) return;
+    double2* o = reinterpret_cast<double2*>(at) + (int64_t)i * (len / 2) + half;
+    if (!set) {
+      const double2 w = *o;
+      v.x += w.x;
+      v.y += w.y;
+    }
+    *o = v;
+  }
+};
+
+// Stores the lanes' blocks, two lanes to a block: a row of a block is 32 bytes,
+// and one lane's two 16-byte stores reach L2 as two requests where the two
+// lanes' one store is a single one.
+__device__ __forceinline__ void put_block(const BlockPlace& mine, int half, const double* uu, bool transpose,
+                                          const double* col, const double* row, double pp) {
+  const BlockPlace other = mine.other();
+  const BlockPlace even = half ? other : mine, odd = half ? mine : other;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    double v[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+      v[k] = i < 3 ? (k < 3 ? (transpose ? uu[3 * k + i] : uu[3 * i + k]) : col[i]) : k < 3 ? row[k] : pp;
+    const double2 got = {partner<0>(half ? v[0] : v[2]), partner<0>(half ? v[1] : v[3])};
+    const double2 lo = {v[0], v[1]}, hi = {v[2], v[3]};
+    even.put(i, half, half ? got : lo);
+    odd.put(i, half, half ? hi : got);
+  }
+}
+
+constexpr int kClusterThreads = 192;
+static_assert(4 * kClusterElems <= kClusterThreads && kClusterNodes <= 64, "one thread per point, one per node");
+
+// A barrier for what the workgroup shares in LDS: __syncthreads() would also
+// wait until every store of the chunk's blocks has reached memory.
+__device__ __forceinline__ void lds_barrier() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
+// The chunks of a workgroup's runs, one after the other: chunk r is run r's
+// first, its further ones are r.z .. r.w.
+struct ClusterCursor {
+  int64_t it = 0, run, c;
+  int4 r;
+  int x;
+  __device__ __forceinline__ explicit ClusterCursor(const ClusterArgs& a) { load(a); }
+  __device__ __forceinline__ void load(const ClusterArgs& a) {
+    c = run = run_of(it, a.num_runs, a.xcd_remap);
+    if (run < 0) return;
+    r = a.runs[run];
+    x = r.z;
+  }
+  __device__ __forceinline__ bool valid() const { return run >= 0; }
+  __device__ __forceinline__ void next(const ClusterArgs& a) {
+    if (x < r.w) {
+      c = x++;
+      return;
+    }
+    ++it;
+    load(a);
+  }
+};
+
+template <bool TR>
+__global__ __launch_bounds__(kClusterThreads, 3) void cluster_kernel(ClusterArgs a) {
+  __shared__ double pe[kClusterElems * kElemStride];
+  __shared__ double shape[40];
+  __shared__ int64_t nbase[kClusterNodes];
+  __shared__ int32_t nid[kClusterNodes], nlen[kClusterNodes];
+  const int tid = threadIdx.x, lane = tid & 63, el = tid >> 2;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  if (tid < 40) shape[tid] = shape_at(tid >> 2, tid & 3);
+
+  ClusterCursor cur(a);
+  if (!cur.valid()) return;  // the whole workgroup
+  for (;;) {
+    const int4 ch = a.chunks[cur.c];
+    ClusterCursor nxt = cur;
+    nxt.next(a);
+    if (wave == 2 && lane < cur.r.y - cur.r.x) {  // the run's nodes: CSR base and row length
+      const int32_t n = a.nodes[cur.r.x + lane];
+      const int64_t b = a.row_ptr[4 * (int64_t)n];
+      nid[lane] = n;
+      nbase[lane] = b;
+      nlen[lane] = (int)(a.row_ptr[4 * (int64_t)n + 1] - b);
+    }
+    int q = tid & 3;
+    asm volatile("" : "+v"(q));  // what hangs on it is formed here, not kept in registers over the loop
+    if (el < ch.x) {
+      const int64_t s = cur.c * kClusterElems + el;
+      const uint32_t w = a.chunk_elems[s];
+      point_state(a, (int64_t)(w & ~kClusterOwned), a.chunk_conn + 10 * s, q, a.save_state && (w & kClusterOwned),
+                  pe + kElemStride * el);
+    }
+    lds_barrier();  // point states and node table are there
+    for (int g = ch.y + 64 * wave; g < ch.z; g += kClusterThreads) {
+      const ClusterLane e = a.lanes[g + lane];
+      const int n = (int)(e.x >> kLaneCount) & 3, lg = (int)(e.x >> kLaneLog) & 7;
+      const bool diag = e.x & kLaneDiag;
+      PairSum s;
+      s.each([](double& v) { v = 0.0; });
+      uint64_t code = e.x;
+      for (int v = 0; v < n; ++v, code >>= 13)
+        visit(pe + kElemStride * (int)(code & 31), shape, (int)(code >> 5) & 15, (int)(code >> 9) & 15, diag, s);
+      const int most = __builtin_amdgcn_readfirstlane(lg);  // the first lane's pair has the most lanes
+      if (most > 0) join<0>(lg, s);
+      if (most > 1) join<1>(lg, s);
+      if (most > 2) join<2>(lg, s);
+      if (most > 3) join<3>(lg, s);
+      const bool mine = n > 0 && !(lane & ((1 << lg) - 1));
+      const int nl = (int)(e.x >> kLaneNode) & 31;
+      const bool first = e.x & kLaneFirst;
+      BlockPlace ab = {0, nlen[nl], a.overwrite_vals && first}, ba = ab;
+      if (mine) ab.at = reinterpret_cast<uint64_t>(a.vals + nbase[nl] + 4 * ((int)(e.x >> kLanePos) & 511));
+      if (mine && !diag) {
+        ba.at = reinterpret_cast<uint64_t>(a.vals + 16 * (int64_t)(e.y & ((uint64_t(1) << kLaneDegT) - 1)) +
+                                           4 * (int64_t)(e.y >> kLanePosT));
+        ba.len = 4 * ((int)(e.y >> kLaneDegT) & 4095);
+      }
+      // block (a, b); of the transpose, what the matrix has at (b, a), transposed
+      put_block(ab, lane & 1, s.uu, false, TR ? s.ba_r : s.ab_c, TR ? s.ba_c : s.ab_r, s.pp);
+      put_block(ba, lane & 1, s.uu, true, TR ? s.ab_r : s.ba_c, TR ? s.ab_c : s.ba_r, s.pp);
+      if (mine && diag) {
+        double* o = a.R + 4 * (int64_t)nid[nl];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) o[i] = ((a.overwrite_R && first) ? 0.0 : o[i]) + s.r[i];
+      }
+    }
+    if (!nxt.valid()) break;
+    if (nxt.run == cur.run) __threadfence();  // the next chunk may add to this one's blocks
+    lds_barrier();                          // the point states are free
+    cur = nxt;
+  }
+}
+
+}  // namespace
+
+// scratch of the sort over n nodes and of scans over up to n + 1 entries
+hipError_t cluster_temp_bytes(int64_t nn, size_t* bytes) {
+  size_t a = 0, b = 0;
+  hipError_t err = hipcub::DeviceRadixSort::SortPairs(nullptr, a, (const int32_t*)nullptr, (int32_t*)nullptr,
+                                                      (const int32_t*)nullptr, (int32_t*)nullptr, (int)nn, 0, 31);
+  if (err != hipSuccess) return err;
+  err = hipcub::DeviceScan::ExclusiveSum(nullptr, b, (const int32_t*)nullptr, (int32_t*)nullptr, (int)(nn + 1));
+  *bytes = std::max(a, b);
+  return err;
+}
+
+hipError_t cluster_order(const int32_t* conn, const double* coords, int64_t ne, int64_t nn, void* temp,
+                         size_t temp_bytes, unsigned long long* box, int32_t* keys, int32_t* keys_sorted,
+                         int32_t* rank, int32_t* place, int32_t* nodes, int64_t* seg, hipStream_t s) {
+  hipError_t err = hipMemsetAsync(box, 0xff, 3 * sizeof(*box), s);
+  if (err == hipSuccess) err = hipMemsetAsync(box + 3, 0, 3 * sizeof(*box), s);
+  if (err != hipSuccess) return err;
+  hipLaunchKernelGGL(cluster_box_kernel, dim3(std::min(grid_for(nn), 1024u)), dim3(kBlock), 0, s, coords, nn, box);
+  uint32_t* code = reinterpret_cast<uint32_t*>(keys);
+  hipLaunchKernelGGL(cluster_morton_kernel, dim3(grid_for(nn)), dim3(kBlock), 0, s, coords, nn, box, code, place);
+  err = hipGetLastError();
+  if (err != hipSuccess) return err;
+  size_t tb = temp_bytes;
+  err = hipcub::DeviceRadixSort::SortPairs(temp, tb, code, reinterpret_cast<uint32_t*>(keys_sorted), place, nodes,
+                                           (int)nn, 0, 30, s);
+  if (err != hipSuccess) return err;
+  hipLaunchKernelGGL(cluster_place_kernel, dim3(grid_for(nn)), dim3(kBlock), 0, s, nodes, nn, rank);
+  for (int pass = 0; pass < 3; ++pass)
+    hipLaunchKernelGGL(cluster_keys_kernel, dim3(grid_for(pass == 0 ? nn : 6 * ne)), dim3(kBlock), 0, s, conn, ne, nn,
+                       pass, rank, keys, place);
+  err = hipGetLastError();
+  if (err != hipSuccess) return err;
+  tb = temp_bytes;
+  err = hipcub::DeviceRadixSort::SortPairs(temp, tb, keys, keys_sorted, place, nodes, (int)nn, 0, 31, s);
+  if (err != hipSuccess) return err;
+  hipLaunchKernelGGL(cluster_segments_kernel, dim3(grid_for(nn + 1)), dim3(kBlock), 0, s, keys_sorted, nn, seg);
+  hipLaunchKernelGGL(cluster_place_kernel, dim3(grid_for(nn)), dim3(kBlock), 0, s, nodes, nn, place);
+  return hipGetLastError();
+}
+
+hipError_t cluster_count(const ClusterMesh& m, const int64_t* seg, int64_t nn, void* temp, size_t temp_bytes,
+                         int32_t* runs, int32_t* more, int32_t* recs, int32_t* most, hipStream_t s) {
+  hipLaunchKernelGGL(cluster_count_kernel, dim3(grid_for(nn + 1)), dim3(kBlock), 0, s, m, seg, nn, runs, more, recs,
+                     most);
+  hipError_t err = hipGetLastError();
+  for (int32_t* v : {runs, more, recs}) {
+    if (err != hipSuccess) return err;
+    size_t tb = temp_bytes;
+    err = hipcub::DeviceScan::ExclusiveSum(temp, tb, v, v, (int)(nn + 1), s);
+  }
+  return err;
+}
+
+hipError_t cluster_fill(const ClusterMesh& m, const int64_t* seg, int64_t nn, const int32_t* runs,
+                        const int32_t* more, const int32_t* recs, int64_t num_runs, int4* run_tab, int4* chunk_tab,
+                        int2* span_tab, uint32_t* elem_tab, int2* rec_tab, hipStream_t s) {
+  hipLaunchKernelGGL(cluster_fill_kernel, dim3(grid_for(nn)), dim3(kBlock), 0, s, m, seg, nn, runs, more, recs,
+                     num_runs, run_tab, chunk_tab, span_tab, elem_tab, rec_tab);
+  return hipGetLastError();
+}
+
+hipError_t cluster_lanes(const ClusterMesh& m, int64_t num_runs, int64_t num_chunks, const int4* run_tab,
+                         int4* chunk_tab, const int2* span_tab, const uint32_t* elem_tab, const int2* rec_tab,
+                         int32_t* nlanes, void* temp, size_t temp_bytes, ClusterLane* lanes, hipStream_t s) {
+  if (num_runs == 0) return hipSuccess;
+  hipLaunchKernelGGL(cluster_lanes_kernel, dim3((unsigned)num_runs), dim3(kBlock), 0, s, m, run_tab, chunk_tab,
+                     span_tab, elem_tab, rec_tab, nlanes, lanes);
+  hipError_t err = hipGetLastError();
+  if (err != hipSuccess || lanes) return err;
+  return hipcub::DeviceScan::ExclusiveSum(temp, temp_bytes, nlanes, nlanes, (int)(num_chunks + 1), s);
+}
+
+hipError_t cluster_conn(int64_t num_chunks, const int4* chunk_tab, const uint32_t* elem_tab, const int32_t* conn,
+                        int32_t* chunk_conn, hipStream_t s) {
+  hipLaunchKernelGGL(cluster_conn_kernel, dim3(grid_for(num_chunks * kClusterElems * 10)), dim3(kBlock), 0, s,
+                     num_chunks, chunk_tab, elem_tab, conn, chunk_conn);
+  return hipGetLastError();
+}
+
+hipError_t launch_cluster(bool transpose, const ClusterArgs& a, int blocks, hipStream_t s) {
+  if (a.num_runs == 0) return hipSuccess;
+  // One workgroup per run unless told otherwise (a multiple of 8 for the XCD
+  // slabs).  Not a persistent grid: loads and stores share a wait counter, so a
+  // workgroup's next run would begin by waiting for all stores of the last one
+  // (P2 64^3 cube: 9.5 ms against 6.0).
+  if (blocks <= 0) blocks = (int)std::min<int64_t>((a.num_runs + 7) / 8 * 8, int64_t(1) << 30);
+  if (transpose) hipLaunchKernelGGL((cluster_kernel<true>), dim3(blocks), dim3(kClusterThreads), 0, s, a);
+  else hipLaunchKernelGGL((cluster_kernel<false>), dim3(blocks), dim3(kClusterThreads), 0, s, a);
+  return hipGetLastError();
+}
+
+}  // namespace goal

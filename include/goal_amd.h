@@ -256,7 +256,9 @@ int goal_mech_destroy(goal_mech m);
  * "overlap" (neo-Hookean only: 2..1024 runs the element pass in this many
  * chunks and gathers each finished chunk's node ranges on a second stream,
  * bitwise equal to one pass; 0 off; -1, the default, is one pass; not used
- * under stream capture),
+ * under stream capture, nor by the FP64 Jacobians of ten-node four-point tets,
+ * which one kernel forms without a gather: goal_mech_timing counts all of it
+ * as the element pass),
  * "overlap_blocks" (element workgroups per chunk, 0 = 5/6 of the resident
  * grid). */
 int goal_mech_set_option(goal_mech m, const char* key, int64_t value);
