@@ -450,53 +450,60 @@ void cluster_build(goal_disc d) {
   if (d->max_degree <= goal::kClusterSlots && ne > 0) {
     size_t tb = 0;
     HIPCHK(goal::cluster_temp_bytes(std::max(nn, 10 * ne), &tb));
-    DevBuf<uint8_t> temp;
-    temp.alloc((int64_t)tb + 256);
-    DevBuf<unsigned long long> box;
-    DevBuf<int32_t> keys, sorted, rank, place, nr, nx, nk, most, nlanes;
-    DevBuf<int64_t> seg;
-    DevBuf<int2> recs, spans;
-    keys.alloc(nn);
-    sorted.alloc(nn);
-    box.alloc(6);
-    rank.alloc(nn);
-    place.alloc(nn);
+    // one work buffer: sort and scan scratch, then the arrays over nodes and incidences
+    DevBuf<uint8_t> work;
+    size_t at = 0;
+    auto reserve = [&](int64_t bytes) {
+      const size_t o = at;
+      at += ((size_t)bytes + 255) / 256 * 256;
+      return o;
+    };
+    const size_t o_temp = reserve((int64_t)tb), o_box = reserve(48), o_most = reserve(4), o_seg = reserve(8 * (nn + 1));
+    size_t o_n[7];
+    for (size_t& o : o_n) o = reserve(4 * (nn + 1));
+    const size_t o_recs = reserve(8 * 10 * ne);
+    work.alloc((int64_t)at);
+    auto ints = [&](size_t o) { return reinterpret_cast<int32_t*>(work.p + o); };
+    void* temp = work.p + o_temp;
+    int64_t* seg = reinterpret_cast<int64_t*>(work.p + o_seg);
+    int32_t *keys = ints(o_n[0]), *sorted = ints(o_n[1]), *rank = ints(o_n[2]), *place = ints(o_n[3]),
+            *nr = ints(o_n[4]), *nx = ints(o_n[5]), *nk = ints(o_n[6]), *most = ints(o_most);
+    int2* recs = reinterpret_cast<int2*>(work.p + o_recs);
     p->nodes.alloc(nn);
-    seg.alloc(nn + 1);
-    HIPCHK(goal::cluster_order(d->conn.p, d->coords.p, ne, nn, temp.p, tb, box.p, keys.p, sorted.p, rank.p, place.p,
-                               p->nodes.p, seg.p, stream()));
-    const goal::ClusterMesh m{p->nodes.p, d->inc_ptr.p, d->inc.p, d->row_ptr.p, d->posi.p, d->pos.p, d->cols.p, place.p};
-    nr.alloc(nn + 1);
-    nx.alloc(nn + 1);
-    nk.alloc(nn + 1);
-    most.alloc(1);
-    HIPCHK(hipMemsetAsync(most.p, 0, sizeof(int32_t), stream()));
-    HIPCHK(goal::cluster_count(m, seg.p, nn, temp.p, tb, nr.p, nx.p, nk.p, most.p, stream()));
+    HIPCHK(goal::cluster_order(d->conn.p, d->coords.p, ne, nn, temp, tb,
+                               reinterpret_cast<unsigned long long*>(work.p + o_box), keys, sorted, rank, place,
+                               p->nodes.p, seg, stream()));
+    const goal::ClusterMesh m{p->nodes.p, d->inc_ptr.p, d->inc.p, d->row_ptr.p, d->posi.p, d->pos.p, d->cols.p, place};
+    HIPCHK(hipMemsetAsync(most, 0, sizeof(int32_t), stream()));
+    HIPCHK(goal::cluster_count(m, seg, nn, temp, tb, nr, nx, nk, most, stream()));
     int32_t runs = 0, more = 0, nb = 0, lanes = 0;
-    HIPCHK(hipMemcpyAsync(&runs, nr.p + nn, sizeof(int32_t), hipMemcpyDeviceToHost, stream()));
-    HIPCHK(hipMemcpyAsync(&more, nx.p + nn, sizeof(int32_t), hipMemcpyDeviceToHost, stream()));
-    most.download(&nb, 1);
+    HIPCHK(hipMemcpyAsync(&runs, nr + nn, sizeof(int32_t), hipMemcpyDeviceToHost, stream()));
+    HIPCHK(hipMemcpyAsync(&more, nx + nn, sizeof(int32_t), hipMemcpyDeviceToHost, stream()));
+    HIPCHK(hipMemcpyAsync(&nb, most, sizeof(int32_t), hipMemcpyDeviceToHost, stream()));
+    sync();
     if (nb <= goal::kClusterSlots && runs > 0) {
       const int64_t chunks = (int64_t)runs + more;
       p->runs.alloc(runs);
       p->chunks.alloc(chunks);
       p->elems.alloc(chunks * goal::kClusterElems);
-      spans.alloc(chunks);
-      recs.alloc(10 * ne);
-      HIPCHK(goal::cluster_fill(m, seg.p, nn, nr.p, nx.p, nk.p, runs, p->runs.p, p->chunks.p, spans.p, p->elems.p,
-                                recs.p, stream()));
-      nlanes.alloc(chunks + 1);
-      HIPCHK(hipMemsetAsync(nlanes.p + chunks, 0, sizeof(int32_t), stream()));
-      HIPCHK(goal::cluster_lanes(m, runs, chunks, p->runs.p, p->chunks.p, spans.p, p->elems.p, recs.p, nlanes.p, temp.p,
-                                 tb, nullptr, stream()));
-      HIPCHK(hipMemcpyAsync(&lanes, nlanes.p + chunks, sizeof(int32_t), hipMemcpyDeviceToHost, stream()));
+      p->conn.alloc(chunks * goal::kClusterElems * 10);
+      DevBuf<int32_t> sizes;  // lanes of every chunk, then its incidences
+      sizes.alloc(3 * chunks + 2);
+      int32_t* nlanes = sizes.p;
+      int2* spans = reinterpret_cast<int2*>(sizes.p + (chunks + 2) / 2 * 2);
+      HIPCHK(goal::cluster_fill(m, seg, nn, nr, nx, nk, runs, p->runs.p, p->chunks.p, spans, p->elems.p, recs,
+                                stream()));
+      HIPCHK(hipMemsetAsync(nlanes + chunks, 0, sizeof(int32_t), stream()));
+      HIPCHK(goal::cluster_lanes(m, runs, chunks, p->runs.p, p->chunks.p, spans, p->elems.p, recs, nlanes, temp, tb,
+                                 nullptr, stream()));
+      HIPCHK(hipMemcpyAsync(&lanes, nlanes + chunks, sizeof(int32_t), hipMemcpyDeviceToHost, stream()));
       sync();
       p->lanes.alloc(lanes);
-      HIPCHK(goal::cluster_lanes(m, runs, chunks, p->runs.p, p->chunks.p, spans.p, p->elems.p, recs.p, nlanes.p, temp.p,
-                                 tb, p->lanes.p, stream()));
-      p->conn.alloc(chunks * goal::kClusterElems * 10);
+      HIPCHK(goal::cluster_lanes(m, runs, chunks, p->runs.p, p->chunks.p, spans, p->elems.p, recs, nlanes, temp, tb,
+                                 p->lanes.p, stream()));
       HIPCHK(goal::cluster_conn(chunks, p->chunks.p, p->elems.p, d->conn.p, p->conn.p, stream()));
       p->num_runs = runs;
+      sync();  // the work buffers are released here and on return
     }
     sync();  // the work buffers are released on return
   }

@@ -179,46 +179,53 @@ __global__ __launch_bounds__(kBlock) void cluster_lanes_kernel(ClusterMesh m, co
                                                                const int2* span_tab, const uint32_t* elem_tab,
                                                                const int2* recs, int32_t* nlanes,
                                                                ClusterLane* lanes) {
-  __shared__ int first[kClusterNodes + 1];               // first block of a node
-  __shared__ int rlo[kClusterNodes], rhi[kClusterNodes];  // a node's incidences in the chunk
-  __shared__ uint16_t cnt[kClusterSlots];
+  constexpr int kRecs = 10 * kClusterElems;                // a chunk's incidences, at most
+  __shared__ int first[kClusterNodes + 1];                 // first block of a node
+  __shared__ int rlo[kClusterNodes], rhi[kClusterNodes];   // a node's incidences in the chunk
+  __shared__ uint16_t rpos[kRecs * 10];                    // their positions
+  __shared__ int rinfo[kRecs];                             // element slot | local node << 8 | run-local node << 16
+  __shared__ int cnt[kClusterSlots];                       // visits of a block's pair
+  __shared__ __align__(4) uint8_t rank[kClusterSlots + 4];
   __shared__ int total;
   const int tid = threadIdx.x;
   const int4 run = run_tab[blockIdx.x];
   const int nn = run.y - run.x;
-  if (tid == 0) {
-    int s = 0;
-    for (int i = 0; i < nn; ++i) {
-      const int64_t n = m.nodes[run.x + i];
-      first[i] = s;
-      s += (int)((m.row_ptr[4 * n + 1] - m.row_ptr[4 * n]) / 4);
-    }
-    first[nn] = s;
+  if (tid < nn) {
+    const int64_t n = m.nodes[run.x + tid];
+    first[tid + 1] = (int)((m.row_ptr[4 * n + 1] - m.row_ptr[4 * n]) / 4);
   }
+  if (tid == 0) first[0] = 0;
   __syncthreads();
-  const int nb = first[nn];
+  if (tid == 0)
+    for (int i = 0; i < nn; ++i) first[i + 1] += first[i];
+  __syncthreads();
+  const int nb = first[nn], nb4 = (nb + 3) / 4 * 4;
   for (int c = (int)blockIdx.x, nxt = run.z;; c = nxt++) {
     const int2 span = span_tab[c];
+    const int nr = span.y - span.x;
     if (tid < nn) rlo[tid] = rhi[tid] = 0;
     if (tid == 0) total = 0;
+    for (int s = tid; s < nb; s += kBlock) cnt[s] = 0;
+    for (int t = tid; t < nr; t += kBlock) rinfo[t] = recs[span.x + t].y;
+    for (int t = tid; t < 10 * nr; t += kBlock) rpos[t] = m.posi[10 * (int64_t)recs[span.x + t / 10].x + t % 10];
     __syncthreads();
-    for (int t = span.x + tid; t < span.y; t += kBlock) {
-      const int node = recs[t].y >> 16;
-      if (t == span.x || (recs[t - 1].y >> 16) != node) rlo[node] = t;
-      if (t + 1 == span.y || (recs[t + 1].y >> 16) != node) rhi[node] = t + 1;
+    for (int t = tid; t < nr; t += kBlock) {
+      const int node = rinfo[t] >> 16;
+      if (t == 0 || (rinfo[t - 1] >> 16) != node) rlo[node] = t;
+      if (t + 1 == nr || (rinfo[t + 1] >> 16) != node) rhi[node] = t + 1;
     }
+    for (int t = tid; t < 10 * nr; t += kBlock) atomicAdd(&cnt[first[rinfo[t / 10] >> 16] + rpos[t]], 1);
     __syncthreads();
-    for (int s = tid; s < nb; s += kBlock) {
-      int node = 0;
-      while (first[node + 1] <= s) ++node;
-      const int pos = s - first[node];
-      const int64_t ga = m.nodes[run.x + node], gb = m.cols[m.row_ptr[4 * ga] + 4 * pos] / 4;
-      int n = 0;
-      if (m.place[gb] >= m.place[ga])  // else the pair is b's run's
-        for (int t = rlo[node]; t < rhi[node]; ++t)
-          for (int b = 0; b < 10; ++b) n += m.posi[10 * (int64_t)recs[t].x + b] == pos;
-      cnt[s] = (uint16_t)n;
-      if (n) atomicAdd(&total, 1 << cluster_log_lanes(n));
+    for (int s = tid; s < nb4; s += kBlock) {
+      int n = s < nb ? cnt[s] : 0;
+      if (n) {
+        int node = 0;
+        while (first[node + 1] <= s) ++node;
+        const int64_t ga = m.nodes[run.x + node], gb = m.cols[m.row_ptr[4 * ga] + 4 * (s - first[node])] / 4;
+        if (m.place[gb] < m.place[ga]) n = cnt[s] = 0;  // the pair is b's run's
+        else atomicAdd(&total, 1 << cluster_log_lanes(n));
+      }
+      rank[s] = (uint8_t)cluster_rank(n);
     }
     __syncthreads();
     if (!lanes) {
@@ -233,43 +240,42 @@ __global__ __launch_bounds__(kBlock) void cluster_lanes_kernel(ClusterMesh m, co
       for (int s = tid; s < nb; s += kBlock) {
         const int n = cnt[s];
         if (!n) continue;
-        const int rank = cluster_rank(n), lg = cluster_log_lanes(n);
-        int lane = 0;
-        for (int u = 0; u < nb; ++u) {
-          const int nu = cnt[u];
-          if (!nu) continue;
-          const int ru = cluster_rank(nu);
-          if (ru < rank || (ru == rank && u < s)) lane += 1 << cluster_log_lanes(nu);
+        const int mine = rank[s], lg = cluster_log_lanes(n);
+        int lane = 0;  // lanes of the pairs before this one
+        for (int u = 0; u < nb; u += 4) {
+          const uint32_t four = *reinterpret_cast<const uint32_t*>(rank + u);
+#pragma unroll
+          for (int k = 0; k < 4; ++k) {
+            const int ru = (four >> (8 * k)) & 255;
+            if (ru < mine || (ru == mine && u + k < s)) lane += ru < 4 ? 16 >> ru : 1;
+          }
         }
         int node = 0;
         while (first[node + 1] <= s) ++node;
         const int pos = s - first[node];
-        // an earlier chunk of the run that adds to this pair holds an earlier incidence of its node
         const int64_t ga = m.nodes[run.x + node], gb = m.cols[m.row_ptr[4 * ga] + 4 * pos] / 4;
+        // an earlier chunk of the run that adds to this pair holds an earlier incidence of its node
         bool earlier = false;
-        for (int64_t k = m.inc_ptr[ga]; k < recs[rlo[node]].x; ++k)
+        for (int64_t k = m.inc_ptr[ga]; k < recs[span.x + rlo[node]].x; ++k)
           for (int b = 0; b < 10; ++b) earlier |= m.posi[10 * k + b] == pos;
-        int pos_t = 0;
-        // lane j's visits, in incidence order
-        for (int j = 0; j < (1 << lg); ++j) {
+        uint16_t code[kClusterElems];
+        int at = 0;
+        for (int t = rlo[node]; t < rhi[node]; ++t)
+          for (int b = 0; b < 10; ++b)
+            if (rpos[10 * t + b] == pos && at < kClusterElems)
+              code[at++] = (uint16_t)((rinfo[t] & 31) | (((rinfo[t] >> 8) & 15) << 5) | (b << 9));
+        const int64_t e = elem_tab[(int64_t)c * kClusterElems + (code[0] & 31)] & ~kClusterOwned;
+        const int pos_t = m.pos[(10 * e + (code[0] >> 9)) * 10 + ((code[0] >> 5) & 15)];
+        const int64_t rb = m.row_ptr[4 * gb];
+        ClusterLane o;
+        o.y = (uint64_t)(rb / 16) | ((uint64_t)((m.row_ptr[4 * gb + 1] - rb) / 4) << kLaneDegT) |
+              ((uint64_t)pos_t << kLanePosT);
+        for (int j = 0; j < (1 << lg); ++j) {  // lane j's visits, in incidence order
           uint64_t w = 0;
-          int at = 0, mine = 0;
-          for (int t = rlo[node]; t < rhi[node]; ++t) {
-            const int2 rec = recs[t];
-            const int a = (rec.y >> 8) & 255, el = rec.y & 31;
-            for (int b = 0; b < 10; ++b)
-              if (m.posi[10 * (int64_t)rec.x + b] == pos) {
-                const int64_t e = elem_tab[(int64_t)c * kClusterElems + el] & ~kClusterOwned;
-                pos_t = m.pos[(10 * e + b) * 10 + a];
-                if ((at++ & ((1 << lg) - 1)) == j) w |= (uint64_t)(el | (a << 5) | (b << 9)) << (13 * mine++);
-              }
-          }
-          ClusterLane o;
-          o.x = w | ((uint64_t)mine << kLaneCount) | ((uint64_t)pos << kLanePos) | ((uint64_t)node << kLaneNode) |
+          int k = 0;
+          for (int v = j; v < at; v += 1 << lg) w |= (uint64_t)code[v] << (13 * k++);
+          o.x = w | ((uint64_t)k << kLaneCount) | ((uint64_t)pos << kLanePos) | ((uint64_t)node << kLaneNode) |
                 ((uint64_t)lg << kLaneLog) | (earlier ? 0 : kLaneFirst) | (ga == gb ? kLaneDiag : 0);
-          const int64_t rb = m.row_ptr[4 * gb];
-          o.y = (uint64_t)(rb / 16) | ((uint64_t)((m.row_ptr[4 * gb + 1] - rb) / 4) << kLaneDegT) |
-                ((uint64_t)pos_t << kLanePosT);
           lanes[base + lane + j] = o;
         }
       }
