@@ -237,7 +237,7 @@ struct goal_disc_s {
   goal::HostMesh mesh;
   std::vector<int64_t> node_adj_ptr;
   std::vector<int32_t> node_adj;          // host copy, made on demand (host_node_adj)
-  DevBuf<int32_t> node_adj_dev;           // the columns as built on the device
+  DevBuf<int32_t> node_adj_dev;           // the nodes' neighbours on the device
   std::unique_ptr<AmgHierarchy> amg;
   std::unique_ptr<ClusterPlan> cluster;
   int max_degree = 0;
@@ -435,7 +435,7 @@ void disc_build(goal_disc d) {
   HIPCHK(goal::launch_expand_csr(adj_ptr.p, adj.p, nn, d->row_ptr.p, d->cols.p, stream()));
   d->x.alloc(d->num_dofs);
   HIPCHK(goal::launch_fill(d->x.p, d->num_dofs, 0.0, stream()));
-  if (d->node_adj.empty() && adj.n > 0) {  // keep the columns on the device for the multigrid set-up
+  {  // the neighbours stay on the device: the solver's products and the multigrid set-up read them
     d->node_adj_dev.release();
     std::swap(d->node_adj_dev.p, adj.p);
     std::swap(d->node_adj_dev.n, adj.n);
@@ -897,16 +897,14 @@ void amg_build_structure(goal_disc d) {
   d->amg = std::move(h);
 }
 
-// y = b - A_l x, or y = A_l x without b (finest level: the solve's CSR).
-void amg_residual(goal_solinfo s, AmgHierarchy& h, int l, const double* x, const double* b, double* y) {
-  AmgLevel& L = *h.lv[l];
+// The solve's matrix, and level l's.
+goal::MatrixRef fine_matrix(goal_solinfo s) {
   goal_disc d = s->d;
-  if (l == 0) {
-    if (b) HIPCHK(goal::launch_spmv_resid(4 * L.nn, d->row_ptr.p, d->cols.p, s->vals.p, x, b, y, stream()));
-    else HIPCHK(goal::launch_spmv(4 * L.nn, d->row_ptr.p, d->cols.p, s->vals.p, x, y, stream()));
-  } else {
-    HIPCHK(goal::launch_bsr_spmv(L.nn, L.bptr.p, L.bcol.p, L.bval.p, x, b, y, stream()));
-  }
+  return {d->mesh.num_nodes, d->nnz, d->row_ptr.p, d->node_adj_dev.p, nullptr, s->vals.p};
+}
+goal::MatrixRef amg_matrix(goal_solinfo s, AmgHierarchy& h, int l) {
+  AmgLevel& L = *h.lv[l];
+  return l == 0 ? fine_matrix(s) : goal::MatrixRef{L.nn, 0, L.bptr.p, nullptr, L.bcol.p, L.bval.p};
 }
 
 // Values of the hierarchy for the solve's current matrix.
@@ -948,7 +946,7 @@ void amg_setup(goal_solinfo s, int* status) {
     int steps = 0;
     for (int j = 0; j < M; ++j) {
       double* w = Q + (int64_t)(j + 1) * nv;
-      amg_residual(s, h, l, Q + (int64_t)j * nv, nullptr, L.r.p);
+      HIPCHK(goal::launch_product(amg_matrix(s, h, l), Q + (int64_t)j * nv, nullptr, L.r.p, stream()));
       HIPCHK(goal::launch_block_apply(L.nn, L.binv.p, L.r.p, w, stream()));
       for (int pass = 0; pass < 2; ++pass) {
         HIPCHK(goal::launch_multi_dot(nv, j + 1, Q, nv, w, s->partial.p, s->h1.p, stream()));
@@ -1002,7 +1000,8 @@ void amg_setup(goal_solinfo s, int* status) {
   sync();
 }
 
-// x = Chebyshev smoothing of A_l x = b (from x = 0 when zero).
+// x = Chebyshev smoothing of A_l x = b (from x = 0 when zero).  A step reads x
+// and writes the other of x and L.r, so that x is where the last one lands.
 void amg_smooth(goal_solinfo s, AmgHierarchy& h, int l, const double* b, double* x, bool zero) {
   AmgLevel& L = *h.lv[l];
   // Chebyshev iteration for the ellipse with centre theta and foci
@@ -1010,20 +1009,17 @@ void amg_smooth(goal_solinfo s, AmgHierarchy& h, int l, const double* b, double*
   // 1 / (2 theta - c2 kappa_k), d_0 = kappa_0 Binv r_0 and d_{k+1} =
   // c2 kappa_{k+1} kappa_k d_k + 2 kappa_{k+1} Binv r_{k+1}, all real also
   // when the foci are imaginary (c2 < 0)
+  static_assert(kAmgDegree % 2 == 0, "an even number of steps ends where it began");
+  const goal::MatrixRef A = amg_matrix(s, h, l);
   const double th = L.theta, c2 = L.c2;
   double k0 = 1.0 / th;
-  const double* r = b;
-  if (zero) {
-    HIPCHK(goal::launch_fill(x, 4 * L.nn, 0.0, stream()));
-  } else {
-    amg_residual(s, h, l, x, b, L.r.p);
-    r = L.r.p;
-  }
-  HIPCHK(goal::launch_cheb(L.nn, L.binv.p, r, 0.0, k0, L.d.p, x, stream()));
+  double *from = x, *to = L.r.p;
+  if (zero) HIPCHK(goal::launch_smooth_start(L.nn, L.binv.p, b, k0, L.d.p, to, stream()));
+  else HIPCHK(goal::launch_smooth(A, L.binv.p, b, from, 0.0, k0, L.d.p, to, stream()));
   for (int k = 1; k < kAmgDegree; ++k) {
+    std::swap(from, to);
     const double k1 = 1.0 / (2.0 * th - c2 * k0);
-    amg_residual(s, h, l, x, b, L.r.p);
-    HIPCHK(goal::launch_cheb(L.nn, L.binv.p, L.r.p, c2 * k1 * k0, 2.0 * k1, L.d.p, x, stream()));
+    HIPCHK(goal::launch_smooth(A, L.binv.p, b, from, c2 * k1 * k0, 2.0 * k1, L.d.p, to, stream()));
     k0 = k1;
   }
 }
@@ -1037,7 +1033,7 @@ void amg_vcycle(goal_solinfo s, AmgHierarchy& h, int l, const double* b, double*
   }
   AmgLevel& C = *h.lv[l + 1];
   amg_smooth(s, h, l, b, x, true);
-  amg_residual(s, h, l, x, b, L.r.p);
+  HIPCHK(goal::launch_product(amg_matrix(s, h, l), x, b, L.r.p, stream()));
   HIPCHK(goal::launch_restrict(L.nc, L.aptr.p, L.amem.p, L.r.p, C.b.p, stream()));
   amg_vcycle(s, h, l + 1, C.b.p, C.x.p);
   HIPCHK(goal::launch_prolong(L.nn, L.agg.p, C.x.p, x, stream()));
@@ -1877,6 +1873,7 @@ int goal_linear_solve_pc(goal_solinfo s, const double* b, double* x, double rtol
     const int64_t* rp = d->row_ptr.p;
     const int32_t* cols = d->cols.p;
     const double* A = s->vals.p;
+    const goal::MatrixRef fine = fine_matrix(s);
     double* V = s->V.p;
     double* t = s->t.p;
     double* z = s->z.p;
@@ -1901,8 +1898,7 @@ int goal_linear_solve_pc(goal_solinfo s, const double* b, double* x, double rtol
     for (;;) {
       // residual r = b - A x into V_0 (right preconditioning: the Krylov
       // space is that of A M^{-1}, and the residual GMRES minimizes is b - A x)
-      HIPCHK(goal::launch_spmv(n, rp, cols, A, x, V, stream()));
-      HIPCHK(goal::launch_rsub(n, b, V, stream()));
+      HIPCHK(goal::launch_product(fine, x, b, V, stream()));
       const double beta = norm2(V);
       if (beta0 < 0.0) beta0 = beta;
       relres = beta0 > 0.0 ? beta / beta0 : 0.0;
@@ -1915,7 +1911,7 @@ int goal_linear_solve_pc(goal_solinfo s, const double* b, double* x, double rtol
       while (j < m && total < max_iters) {
         double* w = V + (int64_t)(j + 1) * n;
         prec(V + (int64_t)j * n, t);
-        HIPCHK(goal::launch_spmv(n, rp, cols, A, t, w, stream()));
+        HIPCHK(goal::launch_product(fine, t, nullptr, w, stream()));
         // classical Gram-Schmidt with the DGKS test (the reference's Belos
         // orthogonalization, src/goal_linear_solve.cpp:53-90): a second pass
         // only when the first removed more than 1 - 1/sqrt(2) of the norm

@@ -140,25 +140,33 @@ int element_resident_grid(int kind, int order, int quad_order, int model, bool f
 
 // Utility kernels (goal_util.hip)
 // Device linear solve (goal_solve.hip).
-hipError_t launch_spmv(int64_t nrows, const int64_t* rp, const int32_t* cols, const double* vals, const double* x,
-                       double* y, hipStream_t s);
+// A matrix of 4 x 4 node blocks: the finest level's scalar CSR (adj: the nodes'
+// neighbours, ptr: four rows per node, each neighbour four columns), or, with
+// adj null, block CSR (ptr, bcol, 16 values per block, row-major).
+struct MatrixRef {
+  int64_t nn, nnz;
+  const int64_t* ptr;
+  const int32_t *adj, *bcol;
+  const double* vals;
+};
+hipError_t launch_product(const MatrixRef& A, const double* x, const double* b, double* y,
+                          hipStream_t s);  // y = A x, or b - A x with b
+// Chebyshev step: d = c1 d + c2 Binv (b - A x), y = x + d (y != x; d unread with c1 = 0)
+hipError_t launch_smooth(const MatrixRef& A, const double* binv, const double* b, const double* x, double c1,
+                         double c2, double* d, double* y, hipStream_t s);
+hipError_t launch_smooth_start(int64_t nn, const double* binv, const double* b, double c2, double* d, double* x,
+                               hipStream_t s);  // from x = 0: d = x = c2 Binv b
 hipError_t launch_block_inverse(int64_t nn, const int64_t* rp, const int32_t* cols, const double* vals,
                                 double* binv, int* status, hipStream_t s);
 hipError_t launch_block_apply(int64_t nn, const double* binv, const double* x, double* y, hipStream_t s);
 // aggregation multigrid: BSR (4x4 node blocks) levels, Galerkin sums, transfers, smoother
 hipError_t launch_bsr_block_inverse(int64_t nb, const int64_t* bptr, const int32_t* bcol, const double* bval,
                                     double* binv, int* status, hipStream_t s);
-hipError_t launch_bsr_spmv(int64_t nb, const int64_t* bptr, const int32_t* bcol, const double* bval, const double* x,
-                           const double* b, double* y, hipStream_t s);  // y = A x, or b - A x with b
-hipError_t launch_spmv_resid(int64_t nrows, const int64_t* rp, const int32_t* cols, const double* vals,
-                             const double* x, const double* b, double* y, hipStream_t s);  // y = b - A x
 hipError_t launch_galerkin(int64_t ncb, const int64_t* gptr, const int64_t* gidx, const int32_t* brow,
                            const int64_t* rp, const double* fvals, double* cvals, hipStream_t s);
 hipError_t launch_restrict(int64_t nc, const int64_t* aptr, const int32_t* amem, const double* r, double* bc,
                            hipStream_t s);
 hipError_t launch_prolong(int64_t nf, const int32_t* agg, const double* xc, double* x, hipStream_t s);
-hipError_t launch_cheb(int64_t nn, const double* binv, const double* r, double c1, double c2, double* d, double* x,
-                       hipStream_t s);
 hipError_t launch_dense_matvec(int n, const double* M, const double* x, double* y, hipStream_t s);
 // out[j] = V_j . w (j < k); partial holds k * multi_dot_blocks(n) doubles
 int multi_dot_blocks(int64_t n);
@@ -167,7 +175,6 @@ hipError_t launch_multi_dot(int64_t n, int k, const double* V, int64_t ldv, cons
 hipError_t launch_multi_axpy(int64_t n, int k, const double* V, int64_t ldv, const double* c, double sign, double* w,
                              hipStream_t s);
 hipError_t launch_scale(int64_t n, double a, const double* x, double* y, hipStream_t s);
-hipError_t launch_rsub(int64_t n, const double* b, double* y, hipStream_t s);
 
 hipError_t launch_fill(double* p, int64_t n, double v, hipStream_t s);
 hipError_t launch_copy(double* dst, const double* src, int64_t n, hipStream_t s);

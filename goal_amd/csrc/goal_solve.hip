@@ -10,16 +10,92 @@ namespace {
 
 constexpr int kSolveThreads = 256;
 
-// y = A x for a CSR matrix, one wavefront per row.
-__global__ __launch_bounds__(kSolveThreads) void spmv_kernel(int64_t nrows, const int64_t* rp, const int32_t* cols,
-                                                             const double* vals, const double* x, double* y) {
-  const int lane = threadIdx.x & 63;
-  const int64_t row = (int64_t)blockIdx.x * (kSolveThreads / 64) + (threadIdx.x >> 6);
-  if (row >= nrows) return;  // uniform per wave
-  double s = 0.0;
-  for (int64_t k = rp[row] + lane; k < rp[row + 1]; k += 64) s += vals[k] * x[cols[k]];
-  for (int off = 32; off > 0; off >>= 1) s += __shfl_down(s, off, 64);
-  if (lane == 0) y[row] = s;
+// ------------------------------------------------- products with a matrix
+// What a product is for: y = A x, y = b - A x, or a Chebyshev step of the
+// block-Jacobi smoother, r = b - A x, d = c1 d + c2 Binv r, y = x + d (y other
+// than x: other rows still read x; with c1 = 0 d is not read).
+enum ProductKind { PRODUCT, RESIDUAL, SMOOTH };
+struct ProductArgs {
+  const double *x, *b, *binv;
+  double c1, c2;
+  double *d, *y;
+};
+
+// What a lane that ends row i of a node needs beside the sums; loaded before
+// them, so that the loads' latency is not added to the matrix's (SMOOTH on the
+// P2 24^3 cube: 96 -> 91 us).
+template <int KIND>
+struct RowEnd {
+  double b = 0.0, x = 0.0, d = 0.0, B[4] = {0.0, 0.0, 0.0, 0.0};
+  __device__ inline void load(const ProductArgs& a, int64_t node, int i) {
+    const int64_t k = 4 * node + i;
+    if constexpr (KIND != PRODUCT) b = a.b[k];
+    if constexpr (KIND == SMOOTH) {
+      x = a.x[k];
+      if (a.c1 != 0.0) d = a.d[k];
+      for (int j = 0; j < 4; ++j) B[j] = a.binv[4 * k + j];
+    }
+  }
+  // r: A x, b - A x or, of all four rows, the residual
+  __device__ inline void store(const ProductArgs& a, int64_t node, int i, const double* r) const {
+    const int64_t k = 4 * node + i;
+    if constexpr (KIND == SMOOTH) {
+      const double z = B[0] * r[0] + B[1] * r[1] + B[2] * r[2] + B[3] * r[3];
+      const double dn = a.c1 * d + a.c2 * z;
+      a.d[k] = dn;
+      a.y[k] = x + dn;
+    } else {
+      a.y[k] = r[0];
+    }
+  }
+};
+
+// The finest level: scalar CSR whose rows come four to a node with the same
+// columns, four to a neighbour.  L lanes take a node: each reads two columns of
+// all four rows (four 16-byte loads in flight, every one coalesced) and two
+// values of x; the neighbour's id comes from the node adjacency (4 bytes per
+// 4 x 4 block).  Bound by HBM: the matrix is read once.  One wavefront per
+// scalar row with the columns of every row took 230 us per product of the
+// P2 24^3 cube (51 M values) against 75.
+template <int L, int KIND>
+__global__ __launch_bounds__(kSolveThreads) void node_product_kernel(int64_t nn, const int64_t* rp,
+                                                                     const int32_t* adj, const double* vals,
+                                                                     ProductArgs a) {
+  const int l = threadIdx.x % L;
+  const int64_t node = (int64_t)blockIdx.x * (kSolveThreads / L) + threadIdx.x / L;
+  if (node >= nn) return;  // uniform per group of L lanes
+  const int64_t base = rp[4 * node];
+  const int len = (int)(rp[4 * node + 1] - base);
+  const double* v = vals + base;
+  const int32_t* nb = adj + base / 16;
+  const int i = l / (L / 4);  // the row this lane holds in the end
+  RowEnd<KIND> end;
+  if (l % (L / 4) == 0) end.load(a, node, i);
+  double s0 = 0.0, s1 = 0.0, s2 = 0.0, s3 = 0.0;
+  for (int p = l; p < len / 2; p += L) {
+    const double2 xc = *reinterpret_cast<const double2*>(a.x + 4 * (int64_t)nb[p >> 1] + 2 * (p & 1));
+    const double2 v0 = *reinterpret_cast<const double2*>(v + 2 * p);
+    const double2 v1 = *reinterpret_cast<const double2*>(v + len + 2 * p);
+    const double2 v2 = *reinterpret_cast<const double2*>(v + 2 * len + 2 * p);
+    const double2 v3 = *reinterpret_cast<const double2*>(v + 3 * (int64_t)len + 2 * p);
+    s0 += v0.x * xc.x + v0.y * xc.y;
+    s1 += v1.x * xc.x + v1.y * xc.y;
+    s2 += v2.x * xc.x + v2.y * xc.y;
+    s3 += v3.x * xc.x + v3.y * xc.y;
+  }
+  // four sums over L lanes: halve the rows a lane holds twice, then the lanes
+  const bool h = l & (L / 2), q = l & (L / 4);
+  double t0 = h ? s2 : s0, t1 = h ? s3 : s1;
+  t0 += __shfl_xor(h ? s0 : s2, L / 2, 64);
+  t1 += __shfl_xor(h ? s1 : s3, L / 2, 64);
+  double t = q ? t1 : t0;
+  t += __shfl_xor(q ? t0 : t1, L / 4, 64);
+  for (int off = L / 8; off > 0; off >>= 1) t += __shfl_xor(t, off, 64);
+  double r[4] = {t, 0.0, 0.0, 0.0};
+  if constexpr (KIND != PRODUCT) r[0] = t = end.b - t;
+  if constexpr (KIND == SMOOTH)
+    for (int j = 0; j < 4; ++j) r[j] = __shfl(t, (threadIdx.x & 63) / L * L + j * (L / 4), 64);
+  if (l % (L / 4) == 0) end.store(a, node, i, r);
 }
 
 // Gauss-Jordan inverse with partial pivoting of the 4x4 block in M[:, 0:4]
@@ -106,34 +182,31 @@ __global__ __launch_bounds__(kSolveThreads) void bsr_block_inverse_kernel(int64_
   invert4(M, binv + 16 * a, status);
 }
 
-// y = A x, or y = b - A x when b is given; one thread per scalar row.
-__global__ __launch_bounds__(kSolveThreads) void bsr_spmv_kernel(int64_t nb, const int64_t* bptr,
-                                                                 const int32_t* bcol, const double* bval,
-                                                                 const double* x, const double* b, double* y) {
-  const int64_t r = (int64_t)blockIdx.x * kSolveThreads + threadIdx.x;
-  if (r >= 4 * nb) return;
-  const int64_t a = r >> 2;
-  const int i = (int)(r & 3);
-  double s = 0.0;
-  for (int64_t k = bptr[a]; k < bptr[a + 1]; ++k) {
-    const double* v = bval + 16 * k + 4 * i;
-    const double* xc = x + 4 * (int64_t)bcol[k];
-    s += v[0] * xc[0] + v[1] * xc[1] + v[2] * xc[2] + v[3] * xc[3];
+// Coarse levels: 16 lanes take a block row, lane 4 k + i the row i of every
+// fourth block.
+template <int KIND>
+__global__ __launch_bounds__(kSolveThreads) void bsr_product_kernel(int64_t nb, const int64_t* bptr,
+                                                                    const int32_t* bcol, const double* bval,
+                                                                    ProductArgs a) {
+  const int l = threadIdx.x & 15, i = l & 3;
+  const int64_t node = (int64_t)blockIdx.x * (kSolveThreads / 16) + threadIdx.x / 16;
+  if (node >= nb) return;  // uniform per group of 16 lanes
+  RowEnd<KIND> end;
+  if (l < 4) end.load(a, node, i);
+  double t = 0.0;
+  for (int64_t k = bptr[node] + (l >> 2); k < bptr[node + 1]; k += 4) {
+    const double2* v = reinterpret_cast<const double2*>(bval + 16 * k + 4 * i);
+    const double2* xc = reinterpret_cast<const double2*>(a.x + 4 * (int64_t)bcol[k]);
+    const double2 v0 = v[0], v1 = v[1], x0 = xc[0], x1 = xc[1];
+    t += v0.x * x0.x + v0.y * x0.y + v1.x * x1.x + v1.y * x1.y;
   }
-  y[r] = b ? b[r] - s : s;
-}
-
-// y = b - A x for the scalar CSR of the finest level, one wavefront per row.
-__global__ __launch_bounds__(kSolveThreads) void spmv_resid_kernel(int64_t nrows, const int64_t* rp,
-                                                                   const int32_t* cols, const double* vals,
-                                                                   const double* x, const double* b, double* y) {
-  const int lane = threadIdx.x & 63;
-  const int64_t row = (int64_t)blockIdx.x * (kSolveThreads / 64) + (threadIdx.x >> 6);
-  if (row >= nrows) return;  // uniform per wave
-  double s = 0.0;
-  for (int64_t k = rp[row] + lane; k < rp[row + 1]; k += 64) s += vals[k] * x[cols[k]];
-  for (int off = 32; off > 0; off >>= 1) s += __shfl_down(s, off, 64);
-  if (lane == 0) y[row] = b[row] - s;
+  t += __shfl_xor(t, 4, 64);
+  t += __shfl_xor(t, 8, 64);
+  double r[4] = {t, 0.0, 0.0, 0.0};
+  if constexpr (KIND != PRODUCT) r[0] = t = end.b - t;
+  if constexpr (KIND == SMOOTH)
+    for (int j = 0; j < 4; ++j) r[j] = __shfl(t, (threadIdx.x & 48) + j, 64);
+  if (l < 4) end.store(a, node, i, r);
 }
 
 // Galerkin sum P^T A P of the plain-aggregation prolongator: coarse block s,
@@ -163,17 +236,19 @@ __global__ __launch_bounds__(kSolveThreads) void galerkin_kernel(int64_t ncb, co
   cvals[16 * sidx + e] = sum;
 }
 
-// bc[A] = sum of r over the aggregate's nodes (P^T r), one thread per (A, i).
+// bc[A] = sum of r over the aggregate's nodes (P^T r): 16 lanes per aggregate,
+// lane 4 k + i entry i of every fourth node.
 __global__ __launch_bounds__(kSolveThreads) void restrict_kernel(int64_t nc, const int64_t* aptr,
                                                                  const int32_t* amem, const double* r,
                                                                  double* bc) {
-  const int64_t t = (int64_t)blockIdx.x * kSolveThreads + threadIdx.x;
-  if (t >= 4 * nc) return;
-  const int64_t A = t >> 2;
-  const int i = (int)(t & 3);
+  const int l = threadIdx.x & 15, i = l & 3;
+  const int64_t A = (int64_t)blockIdx.x * (kSolveThreads / 16) + threadIdx.x / 16;
+  if (A >= nc) return;  // uniform per group of 16 lanes
   double s = 0.0;
-  for (int64_t m = aptr[A]; m < aptr[A + 1]; ++m) s += r[4 * (int64_t)amem[m] + i];
-  bc[t] = s;
+  for (int64_t m = aptr[A] + (l >> 2); m < aptr[A + 1]; m += 4) s += r[4 * (int64_t)amem[m] + i];
+  s += __shfl_xor(s, 4, 64);
+  s += __shfl_xor(s, 8, 64);
+  if (l < 4) bc[4 * A + i] = s;
 }
 
 // x += P xc: each node takes its aggregate's correction.
@@ -184,30 +259,28 @@ __global__ __launch_bounds__(kSolveThreads) void prolong_kernel(int64_t nf, cons
   x[t] += xc[4 * (int64_t)agg[t >> 2] + (t & 3)];
 }
 
-// One Chebyshev step with the block-Jacobi preconditioner, node by node:
-// d = c1 d + c2 Binv r;  x += d.
-__global__ __launch_bounds__(kSolveThreads) void cheb_kernel(int64_t nn, const double* binv, const double* r,
-                                                             double c1, double c2, double* d, double* x) {
-  const int64_t a = (int64_t)blockIdx.x * kSolveThreads + threadIdx.x;
-  if (a >= nn) return;
-  const double* B = binv + 16 * a;
-  const double r0 = r[4 * a], r1 = r[4 * a + 1], r2 = r[4 * a + 2], r3 = r[4 * a + 3];
-  for (int i = 0; i < 4; ++i) {
-    const double z = B[4 * i] * r0 + B[4 * i + 1] * r1 + B[4 * i + 2] * r2 + B[4 * i + 3] * r3;
-    const double dn = c1 * d[4 * a + i] + c2 * z;
-    d[4 * a + i] = dn;
-    x[4 * a + i] += dn;
-  }
+// The first Chebyshev step from x = 0: d = x = c2 Binv b.
+__global__ __launch_bounds__(kSolveThreads) void smooth_start_kernel(int64_t nn, const double* binv, const double* b,
+                                                                     double c2, double* d, double* x) {
+  const int64_t k = (int64_t)blockIdx.x * kSolveThreads + threadIdx.x;
+  if (k >= 4 * nn) return;
+  const double* B = binv + 4 * k;
+  const double* r = b + k / 4 * 4;
+  const double v = c2 * (B[0] * r[0] + B[1] * r[1] + B[2] * r[2] + B[3] * r[3]);
+  d[k] = v;
+  x[k] = v;
 }
 
-// y = M x for a dense row-major n x n matrix (the coarsest level's inverse).
+// y = M x for a dense row-major n x n matrix (the coarsest level's inverse),
+// one wavefront per row.
 __global__ __launch_bounds__(kSolveThreads) void dense_matvec_kernel(int n, const double* M, const double* x,
                                                                      double* y) {
-  const int i = blockIdx.x * kSolveThreads + threadIdx.x;
-  if (i >= n) return;
+  const int lane = threadIdx.x & 63, i = blockIdx.x * (kSolveThreads / 64) + (threadIdx.x >> 6);
+  if (i >= n) return;  // uniform per wave
   double s = 0.0;
-  for (int j = 0; j < n; ++j) s += M[(int64_t)i * n + j] * x[j];
-  y[i] = s;
+  for (int j = lane; j < n; j += 64) s += M[(int64_t)i * n + j] * x[j];
+  for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off, 64);
+  if (lane == 0) y[i] = s;
 }
 
 // y = Binv x, node by node.
@@ -221,8 +294,9 @@ __global__ __launch_bounds__(kSolveThreads) void block_apply_kernel(int64_t nn, 
 }
 
 // partial[j][block] = sum over the block's slice of V_j . w, j < k.  The
-// vectors go eight at a time: each row's w is read once per eight vectors and
-// the eight loads of a row are independent.
+// vectors go eight at a time, one group of eight per grid row: each row's w is
+// read once per eight vectors, the eight loads of a row are independent, and
+// the groups run beside each other.
 constexpr int kDotGroup = 8;
 
 __global__ __launch_bounds__(kSolveThreads) void multi_dot_partial_kernel(int64_t n, int k, const double* V,
@@ -231,30 +305,27 @@ __global__ __launch_bounds__(kSolveThreads) void multi_dot_partial_kernel(int64_
   __shared__ double red[kSolveThreads / 64][kDotGroup];
   const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
   const int64_t stride = (int64_t)gridDim.x * kSolveThreads;
-  for (int j0 = 0; j0 < k; j0 += kDotGroup) {
-    const int nj = min(kDotGroup, k - j0);
-    double s[kDotGroup];
+  const int j0 = blockIdx.y * kDotGroup, nj = min(kDotGroup, k - j0);
+  double s[kDotGroup];
 #pragma unroll
-    for (int jj = 0; jj < kDotGroup; ++jj) s[jj] = 0.0;
-    for (int64_t i = (int64_t)blockIdx.x * kSolveThreads + tid; i < n; i += stride) {
-      const double wi = w[i];
+  for (int jj = 0; jj < kDotGroup; ++jj) s[jj] = 0.0;
+  for (int64_t i = (int64_t)blockIdx.x * kSolveThreads + tid; i < n; i += stride) {
+    const double wi = w[i];
 #pragma unroll
-      for (int jj = 0; jj < kDotGroup; ++jj)
-        if (jj < nj) s[jj] += V[(int64_t)(j0 + jj) * ldv + i] * wi;
-    }
+    for (int jj = 0; jj < kDotGroup; ++jj)
+      if (jj < nj) s[jj] += V[(int64_t)(j0 + jj) * ldv + i] * wi;
+  }
 #pragma unroll
-    for (int jj = 0; jj < kDotGroup; ++jj) {
-      double t = s[jj];
-      for (int off = 32; off > 0; off >>= 1) t += __shfl_down(t, off, 64);
-      if (lane == 0) red[wv][jj] = t;
-    }
-    __syncthreads();
-    if (tid < nj) {
-      double t = 0.0;
-      for (int q = 0; q < kSolveThreads / 64; ++q) t += red[q][tid];
-      partial[(int64_t)(j0 + tid) * gridDim.x + blockIdx.x] = t;
-    }
-    __syncthreads();
+  for (int jj = 0; jj < kDotGroup; ++jj) {
+    double t = s[jj];
+    for (int off = 32; off > 0; off >>= 1) t += __shfl_down(t, off, 64);
+    if (lane == 0) red[wv][jj] = t;
+  }
+  __syncthreads();
+  if (tid < nj) {
+    double t = 0.0;
+    for (int q = 0; q < kSolveThreads / 64; ++q) t += red[q][tid];
+    partial[(int64_t)(j0 + tid) * gridDim.x + blockIdx.x] = t;
   }
 }
 
@@ -290,26 +361,59 @@ __global__ __launch_bounds__(kSolveThreads) void scale_kernel(int64_t n, double 
   if (i < n) y[i] = a * x[i];
 }
 
-// y = b - y
-__global__ __launch_bounds__(kSolveThreads) void rsub_kernel(int64_t n, const double* b, double* y) {
-  const int64_t i = (int64_t)blockIdx.x * kSolveThreads + threadIdx.x;
-  if (i < n) y[i] = b[i] - y[i];
-}
-
 dim3 grid_for(int64_t n) { return dim3((unsigned)((n + kSolveThreads - 1) / kSolveThreads)); }
 
 }  // namespace
 
 int multi_dot_blocks(int64_t n) {
-  const int64_t b = (n + kSolveThreads - 1) / kSolveThreads;
+  const int64_t b = (n + 4 * kSolveThreads - 1) / (4 * kSolveThreads);  // four rows a thread and more
   return (int)std::min<int64_t>(std::max<int64_t>(b, 1), 1024);
 }
 
-hipError_t launch_spmv(int64_t nrows, const int64_t* rp, const int32_t* cols, const double* vals, const double* x,
-                       double* y, hipStream_t s) {
-  if (nrows == 0) return hipSuccess;
-  const int64_t blocks = (nrows + kSolveThreads / 64 - 1) / (kSolveThreads / 64);
-  hipLaunchKernelGGL(spmv_kernel, dim3((unsigned)blocks), dim3(kSolveThreads), 0, s, nrows, rp, cols, vals, x, y);
+namespace {
+// Lanes per node: a node's row pairs fit the group for most nodes (P1: 15
+// neighbours, 30 pairs; P2: 28 on average, 57).
+template <int KIND>
+hipError_t node_product(int64_t nn, int64_t nnz, const int64_t* rp, const int32_t* adj, const double* vals,
+                        const ProductArgs& a, hipStream_t s) {
+  if (nn == 0) return hipSuccess;
+  if (nnz / (8 * nn) <= 40) {
+    hipLaunchKernelGGL((node_product_kernel<32, KIND>), dim3((unsigned)((nn + kSolveThreads / 32 - 1) / (kSolveThreads / 32))),
+                       dim3(kSolveThreads), 0, s, nn, rp, adj, vals, a);
+  } else {
+    hipLaunchKernelGGL((node_product_kernel<64, KIND>), dim3((unsigned)((nn + kSolveThreads / 64 - 1) / (kSolveThreads / 64))),
+                       dim3(kSolveThreads), 0, s, nn, rp, adj, vals, a);
+  }
+  return hipGetLastError();
+}
+template <int KIND>
+hipError_t bsr_product(int64_t nb, const int64_t* bptr, const int32_t* bcol, const double* bval, const ProductArgs& a,
+                       hipStream_t s) {
+  if (nb == 0) return hipSuccess;
+  hipLaunchKernelGGL(bsr_product_kernel<KIND>, grid_for(16 * nb), dim3(kSolveThreads), 0, s, nb, bptr, bcol, bval, a);
+  return hipGetLastError();
+}
+}  // namespace
+
+hipError_t launch_product(const MatrixRef& A, const double* x, const double* b, double* y, hipStream_t s) {
+  const ProductArgs a{x, b, nullptr, 0.0, 0.0, nullptr, y};
+  if (A.adj) return b ? node_product<RESIDUAL>(A.nn, A.nnz, A.ptr, A.adj, A.vals, a, s)
+                      : node_product<PRODUCT>(A.nn, A.nnz, A.ptr, A.adj, A.vals, a, s);
+  return b ? bsr_product<RESIDUAL>(A.nn, A.ptr, A.bcol, A.vals, a, s)
+           : bsr_product<PRODUCT>(A.nn, A.ptr, A.bcol, A.vals, a, s);
+}
+
+hipError_t launch_smooth(const MatrixRef& A, const double* binv, const double* b, const double* x, double c1,
+                         double c2, double* d, double* y, hipStream_t s) {
+  const ProductArgs a{x, b, binv, c1, c2, d, y};
+  return A.adj ? node_product<SMOOTH>(A.nn, A.nnz, A.ptr, A.adj, A.vals, a, s)
+               : bsr_product<SMOOTH>(A.nn, A.ptr, A.bcol, A.vals, a, s);
+}
+
+hipError_t launch_smooth_start(int64_t nn, const double* binv, const double* b, double c2, double* d, double* x,
+                               hipStream_t s) {
+  if (nn == 0) return hipSuccess;
+  hipLaunchKernelGGL(smooth_start_kernel, grid_for(4 * nn), dim3(kSolveThreads), 0, s, nn, binv, b, c2, d, x);
   return hipGetLastError();
 }
 
@@ -328,22 +432,6 @@ hipError_t launch_bsr_block_inverse(int64_t nb, const int64_t* bptr, const int32
   return hipGetLastError();
 }
 
-hipError_t launch_bsr_spmv(int64_t nb, const int64_t* bptr, const int32_t* bcol, const double* bval, const double* x,
-                           const double* b, double* y, hipStream_t s) {
-  if (nb == 0) return hipSuccess;
-  hipLaunchKernelGGL(bsr_spmv_kernel, grid_for(4 * nb), dim3(kSolveThreads), 0, s, nb, bptr, bcol, bval, x, b, y);
-  return hipGetLastError();
-}
-
-hipError_t launch_spmv_resid(int64_t nrows, const int64_t* rp, const int32_t* cols, const double* vals,
-                             const double* x, const double* b, double* y, hipStream_t s) {
-  if (nrows == 0) return hipSuccess;
-  const int64_t blocks = (nrows + kSolveThreads / 64 - 1) / (kSolveThreads / 64);
-  hipLaunchKernelGGL(spmv_resid_kernel, dim3((unsigned)blocks), dim3(kSolveThreads), 0, s, nrows, rp, cols, vals, x,
-                     b, y);
-  return hipGetLastError();
-}
-
 hipError_t launch_galerkin(int64_t ncb, const int64_t* gptr, const int64_t* gidx, const int32_t* brow,
                            const int64_t* rp, const double* fvals, double* cvals, hipStream_t s) {
   if (ncb == 0) return hipSuccess;
@@ -355,7 +443,7 @@ hipError_t launch_galerkin(int64_t ncb, const int64_t* gptr, const int64_t* gidx
 hipError_t launch_restrict(int64_t nc, const int64_t* aptr, const int32_t* amem, const double* r, double* bc,
                            hipStream_t s) {
   if (nc == 0) return hipSuccess;
-  hipLaunchKernelGGL(restrict_kernel, grid_for(4 * nc), dim3(kSolveThreads), 0, s, nc, aptr, amem, r, bc);
+  hipLaunchKernelGGL(restrict_kernel, grid_for(16 * nc), dim3(kSolveThreads), 0, s, nc, aptr, amem, r, bc);
   return hipGetLastError();
 }
 
@@ -365,16 +453,9 @@ hipError_t launch_prolong(int64_t nf, const int32_t* agg, const double* xc, doub
   return hipGetLastError();
 }
 
-hipError_t launch_cheb(int64_t nn, const double* binv, const double* r, double c1, double c2, double* d, double* x,
-                       hipStream_t s) {
-  if (nn == 0) return hipSuccess;
-  hipLaunchKernelGGL(cheb_kernel, grid_for(nn), dim3(kSolveThreads), 0, s, nn, binv, r, c1, c2, d, x);
-  return hipGetLastError();
-}
-
 hipError_t launch_dense_matvec(int n, const double* M, const double* x, double* y, hipStream_t s) {
   if (n == 0) return hipSuccess;
-  hipLaunchKernelGGL(dense_matvec_kernel, grid_for(n), dim3(kSolveThreads), 0, s, n, M, x, y);
+  hipLaunchKernelGGL(dense_matvec_kernel, grid_for(64 * (int64_t)n), dim3(kSolveThreads), 0, s, n, M, x, y);
   return hipGetLastError();
 }
 
@@ -388,7 +469,7 @@ hipError_t launch_multi_dot(int64_t n, int k, const double* V, int64_t ldv, cons
                             double* out, hipStream_t s) {
   if (k == 0) return hipSuccess;
   const int nb = multi_dot_blocks(n);
-  hipLaunchKernelGGL(multi_dot_partial_kernel, dim3(nb), dim3(kSolveThreads), 0, s, n, k, V, ldv, w, partial);
+  hipLaunchKernelGGL(multi_dot_partial_kernel, dim3(nb, (k + kDotGroup - 1) / kDotGroup), dim3(kSolveThreads), 0, s, n, k, V, ldv, w, partial);
   hipLaunchKernelGGL(multi_dot_final_kernel, dim3(k), dim3(kSolveThreads), 0, s, nb, partial, out);
   return hipGetLastError();
 }
@@ -403,12 +484,6 @@ hipError_t launch_multi_axpy(int64_t n, int k, const double* V, int64_t ldv, con
 hipError_t launch_scale(int64_t n, double a, const double* x, double* y, hipStream_t s) {
   if (n == 0) return hipSuccess;
   hipLaunchKernelGGL(scale_kernel, grid_for(n), dim3(kSolveThreads), 0, s, n, a, x, y);
-  return hipGetLastError();
-}
-
-hipError_t launch_rsub(int64_t n, const double* b, double* y, hipStream_t s) {
-  if (n == 0) return hipSuccess;
-  hipLaunchKernelGGL(rsub_kernel, grid_for(n), dim3(kSolveThreads), 0, s, n, b, y);
   return hipGetLastError();
 }
 
