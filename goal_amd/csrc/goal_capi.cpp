@@ -2492,8 +2492,8 @@ int goal_mlp_gradient(goal_mlp m, const float* x_dev, const float* y_dev, const 
   return guard([&]() -> int {
     require(m && x_dev && y_dev && idx_dev && n > 0, "goal_mlp_gradient: bad arguments");
     mlp_workspace(m, n);
-    HIPCHK(goal::launch_mlp_grad(m->args(), x_dev, y_dev, idx_dev, n, m->partial.p, m->partial_loss.p, m->grad.p,
-                                 m->loss.p, stream()));
+    HIPCHK(goal::launch_mlp_grad(m->args(), x_dev, y_dev, idx_dev, n, m->partial.p, m->partial_loss.p, 0, 0.0f,
+                                 m->grad.p, m->loss.p, stream()));
     if (grad) m->grad.download(grad, goal::kMlpParams);
     if (loss) m->loss.download(loss, 1);
     sync();
@@ -2508,8 +2508,7 @@ int goal_mlp_train(goal_mlp m, const float* x_dev, const float* y_dev, const int
     mlp_workspace(m, batch);
     for (int k = 0; k < steps; ++k) {
       HIPCHK(goal::launch_mlp_grad(m->args(), x_dev, y_dev, idx_dev + (int64_t)k * batch, batch, m->partial.p,
-                                   m->partial_loss.p, m->grad.p, m->loss.p, stream()));
-      HIPCHK(goal::launch_mlp_adam(m->args(), m->grad.p, ++m->step, lr, stream()));
+                                   m->partial_loss.p, ++m->step, lr, m->grad.p, m->loss.p, stream()));
     }
     if (last_loss) m->loss.download(last_loss, 1);
     sync();

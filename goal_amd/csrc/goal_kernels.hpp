@@ -281,9 +281,10 @@ hipError_t launch_mlp_forward(const MlpArgs& a, const float* x, int64_t n, float
 // Blocks of the gradient kernel for a batch of B rows (partial holds that many
 // kMlpParams rows and partial_loss that many floats).
 int mlp_grad_blocks(int64_t B);
+// step > 0: an Adam step (its number, counted from one) with the gradient
 hipError_t launch_mlp_grad(const MlpArgs& a, const float* x, const float* y, const int32_t* idx, int64_t B,
-                           float* partial, float* partial_loss, float* grad, float* loss, hipStream_t s);
-hipError_t launch_mlp_adam(const MlpArgs& a, const float* grad, int step, float lr, hipStream_t s);
+                           float* partial, float* partial_loss, int step, float lr, float* grad, float* loss,
+                           hipStream_t s);
 hipError_t launch_mlp_round(const MlpArgs& a, hipStream_t s);
 
 }  // namespace goal

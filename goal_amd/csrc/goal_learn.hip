@@ -176,34 +176,6 @@ __device__ inline uint16_t f32_to_bf16(float f) {
   return (uint16_t)(u >> 16);
 }
 
-// Network parameters staged in LDS as FP32: weights from their BF16 copy,
-// biases from the FP32 master.
-struct SharedNet {
-  float w1[kHid * kIn], b1[kHid], w2[kHid * kHid], b2[kHid], w3[kHid], b3;
-  float mu[kIn], is[kIn], mu_y, s_y, c;
-};
-
-__device__ void stage_net(SharedNet& S, const MlpArgs& a) {
-  for (int i = threadIdx.x; i < kHid * kIn; i += blockDim.x) S.w1[i] = bf16_to_f32(a.wq[oW1 + i]);
-  for (int i = threadIdx.x; i < kHid * kHid; i += blockDim.x) S.w2[i] = bf16_to_f32(a.wq[oW2 + i]);
-  for (int i = threadIdx.x; i < kHid; i += blockDim.x) {
-    S.w3[i] = bf16_to_f32(a.wq[oW3 + i]);
-    S.b1[i] = a.params[oB1 + i];
-    S.b2[i] = a.params[oB2 + i];
-  }
-  for (int i = threadIdx.x; i < kIn; i += blockDim.x) {
-    S.mu[i] = a.norms[i];
-    S.is[i] = a.norms[kIn + i];
-  }
-  if (threadIdx.x == 0) {
-    S.b3 = a.params[oB3];
-    S.mu_y = a.norms[2 * kIn];
-    S.s_y = a.norms[2 * kIn + 1];
-    S.c = a.norms[kMlpOffC];
-  }
-  __syncthreads();
-}
-
 __device__ inline float round_bf16(float f) { return bf16_to_f32(f32_to_bf16(f)); }
 
 // ---------------------------------------------------------- forward (MFMA)
@@ -317,145 +289,189 @@ __global__ __launch_bounds__(kFwdThreads) void mlp_forward_kernel(MlpArgs a, con
 }
 
 // Gradient of L = (1/B) sum_i (net(x_i) - t_i)^2, t_i = (y_i - mu_y - c x_i0)/s_y, over
-// rows idx[0..B).  A block takes tiles of kTile rows: wave 0 runs the forward
-// and back-propagation of its rows into LDS, then all threads accumulate the
-// parameter gradients of the tile into registers.  Each block writes its sums
-// to partial[block][kP] and its loss sum to partial_loss[block].
-constexpr int kTile = 64, kGradThreads = 256, kPad = kHid + 1;
+// rows idx[0..B), on the matrix cores in FP32 (v_mfma_f32_16x16x4_f32) with the
+// samples in tiles of 16.  For lane l, r = l % 16 and q = l / 16:
+//   A operand  lane holds A[r][q],  B operand  B[q][r],
+//   C/D        lane holds D[4q + i][r]      i = 0..3
+// Wave w of four owns the 16 hidden units 16 w ..: its rows of both layers, of
+// both deltas and of all parameter gradients, whose sums stay in its registers
+// over the block's tiles.  Activations and deltas pass between the waves
+// through LDS ([unit][sample], one word of padding).  Each block writes its
+// sums to partial[block][kP] and its loss sum to partial_loss[block].
+// Bound by the latency of its few products and barriers, not by their number:
+// 16 samples per block instead of 64 put 256 blocks on the chip at a batch of
+// 4096, and all four waves work instead of one (116 -> 11 us; with the
+// reduction and Adam in one kernel a step takes 15 us instead of 140).
+constexpr int kTile = 16, kGradThreads = 256, kPad = kTile + 1;
 
-struct SharedTile {
-  float xs[kTile][kIn + 1];
-  float h1[kTile][kPad], h2[kTile][kPad], d2[kTile][kPad], d1[kTile][kPad];
-  float d3[kTile];
-};
+__device__ inline f32x4 mfma4(float a, float b, f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
 
 __global__ __launch_bounds__(kGradThreads) void mlp_grad_kernel(MlpArgs a, const float* x, const float* y,
                                                                 const int32_t* idx, int64_t B, float* partial,
                                                                 float* partial_loss) {
-  __shared__ SharedNet S;
-  __shared__ SharedTile T;
-  stage_net(S, a);
-  const int tid = threadIdx.x;
-  // parameter ownership: W2 entries tid + 256 r (r < 16), W1 entries tid + 256 r
-  // (r < 3), and for tid < 193 one of W3 / b1 / b2 / b3
-  float g2[16], g1[3], g3 = 0.0f;
-  for (int r = 0; r < 16; ++r) g2[r] = 0.0f;
-  for (int r = 0; r < 3; ++r) g1[r] = 0.0f;
-  float loss = 0.0f;
+  __shared__ uint16_t sw[kP + 1];
+  __shared__ float xs[kTile][kIn + 1], tgt[kTile], os[4][kTile];
+  __shared__ float h1s[kHid][kPad], d2s[kHid][kPad], d1s[kHid][kPad];
+  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, r = lane & 15, q = lane >> 4;
+  for (int i = tid; i < kP; i += kGradThreads) sw[i] = a.wq[i];
+  __syncthreads();
+  // operand fragments: W1 and W2 by rows of this wave's units, W2 by columns
+  float A1[3], A2[16], A2t[16], b1[4], b2[4], w3[4];
+  for (int k = 0; k < 3; ++k) A1[k] = bf16_to_f32(sw[oW1 + (16 * w + r) * kIn + 4 * k + q]);
+  for (int k = 0; k < 16; ++k) {
+    A2[k] = bf16_to_f32(sw[oW2 + (16 * w + r) * kHid + 4 * k + q]);
+    A2t[k] = bf16_to_f32(sw[oW2 + (4 * k + q) * kHid + 16 * w + r]);
+  }
+  for (int i = 0; i < 4; ++i) {
+    const int unit = 16 * w + 4 * q + i;
+    b1[i] = a.params[oB1 + unit];
+    b2[i] = a.params[oB2 + unit];
+    w3[i] = bf16_to_f32(sw[oW3 + unit]);
+  }
+  const float b3 = a.params[oB3], mu_y = a.norms[2 * kIn], s_y = a.norms[2 * kIn + 1], cx = a.norms[kMlpOffC];
   const float invB = 1.0f / (float)B;
+  const f32x4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
+  f32x4 g2[4] = {zero, zero, zero, zero}, g1 = zero;
+  float gw3[4] = {0, 0, 0, 0}, gb1[4] = {0, 0, 0, 0}, gb2[4] = {0, 0, 0, 0}, gb3 = 0.0f, loss = 0.0f;
   const int64_t tiles = (B + kTile - 1) / kTile;
   for (int64_t tile = blockIdx.x; tile < tiles; tile += gridDim.x) {
-    if (tid < kTile) {
-      const int64_t row = tile * kTile + tid;
-      const bool live = row < B;
-      float xs[kIn];
-      float t = 0.0f;
-      if (live) {
-        const int64_t r = idx[row];
-        for (int k = 0; k < kIn; ++k) xs[k] = round_bf16((x[r * kIn + k] - S.mu[k]) * S.is[k]);
-        t = (y[r] - S.mu_y - S.c * x[r * kIn]) / S.s_y;
-      } else {
-        for (int k = 0; k < kIn; ++k) xs[k] = 0.0f;
+    if (tid < kTile * kIn) {
+      const int s = tid / kIn, k = tid % kIn;
+      const int64_t row = tile * kTile + s;
+      float v = 0.0f;
+      if (row < B) {
+        const int64_t g = idx[row];
+        const float raw = x[g * kIn + k];
+        v = round_bf16((raw - a.norms[k]) * a.norms[kIn + k]);
+        if (k == 0) tgt[s] = (y[g] - mu_y - cx * raw) / s_y;
       }
-      for (int k = 0; k < kIn; ++k) T.xs[tid][k] = xs[k];
-      // Each thread works on its own padded LDS rows, which keeps register
-      // use low; the odd row stride makes the 64 rows conflict-free.
-      for (int j = 0; j < kHid; ++j) {
-        float s = S.b1[j];
-#pragma unroll
-        for (int k = 0; k < kIn; ++k) s += S.w1[j * kIn + k] * xs[k];
-        T.h1[tid][j] = round_bf16(fmaxf(s, 0.0f));
-      }
-      float o = S.b3;
-      for (int jj = 0; jj < kHid; ++jj) {
-        float s = S.b2[jj];
-        for (int j = 0; j < kHid; ++j) s += S.w2[jj * kHid + j] * T.h1[tid][j];
-        const float h = fmaxf(s, 0.0f);
-        T.h2[tid][jj] = h;
-        o += S.w3[jj] * h;
-      }
-      const float r = live ? o - t : 0.0f;
-      loss += r * r;
-      const float d3 = 2.0f * r * invB;
-      T.d3[tid] = d3;
-      for (int jj = 0; jj < kHid; ++jj) T.d2[tid][jj] = T.h2[tid][jj] > 0.0f ? d3 * S.w3[jj] : 0.0f;
-      for (int j = 0; j < kHid; ++j) {
-        float s = 0.0f;
-        for (int jj = 0; jj < kHid; ++jj) s += S.w2[jj * kHid + j] * T.d2[tid][jj];
-        T.d1[tid][j] = T.h1[tid][j] > 0.0f ? s : 0.0f;
-      }
+      xs[s][k] = v;
     }
     __syncthreads();
-    // W2 entry tid + 256 r is (row tid / 64 + 4 r, column tid % 64)
-    {
-      const int j = tid % kHid, jj0 = tid / kHid;
-      int j1[3], k1[3];
-      for (int r = 0; r < 3; ++r) {
-        j1[r] = (tid + kGradThreads * r) / kIn;
-        k1[r] = (tid + kGradThreads * r) % kIn;
-      }
-      const int sel = tid / kHid, col = tid % kHid;  // W3 / b1 / b2 slot for tid < 192
-#pragma unroll 2
-      for (int q = 0; q < kTile; ++q) {
-        const float h = T.h1[q][j];
-#pragma unroll
-        for (int r = 0; r < 16; ++r) g2[r] += T.d2[q][jj0 + 4 * r] * h;
-#pragma unroll
-        for (int r = 0; r < 3; ++r) g1[r] += T.d1[q][j1[r]] * T.xs[q][k1[r]];
-        if (sel == 0) g3 += T.d3[q] * T.h2[q][col];
-        else if (sel == 1) g3 += T.d1[q][col];
-        else if (sel == 2) g3 += T.d2[q][col];
-        else if (tid == 3 * kHid) g3 += T.d3[q];
-      }
+    // layer 1
+    f32x4 z = zero;
+    for (int k = 0; k < 3; ++k) z = mfma4(A1[k], xs[r][4 * k + q], z);
+    float h1[4], h2[4];
+    for (int i = 0; i < 4; ++i) {
+      h1[i] = round_bf16(fmaxf(z[i] + b1[i], 0.0f));
+      h1s[16 * w + 4 * q + i][r] = h1[i];
     }
     __syncthreads();
+    // layer 2 and the output
+    z = zero;
+    for (int k = 0; k < 16; ++k) z = mfma4(A2[k], h1s[4 * k + q][r], z);
+    float o = 0.0f;
+    for (int i = 0; i < 4; ++i) {
+      h2[i] = fmaxf(z[i] + b2[i], 0.0f);
+      o += w3[i] * h2[i];
+    }
+    o += __shfl_xor(o, 16, 64);
+    o += __shfl_xor(o, 32, 64);
+    if (q == 0) os[w][r] = o;
+    __syncthreads();
+    const bool live = tile * kTile + r < B;
+    const float res = live ? (os[0][r] + os[1][r]) + (os[2][r] + os[3][r]) + b3 - tgt[r] : 0.0f;
+    const float d3 = 2.0f * res * invB;
+    if (tid < kTile) {  // once per sample
+      loss += res * res;
+      gb3 += d3;
+    }
+    for (int i = 0; i < 4; ++i) {
+      const float d2 = h2[i] > 0.0f ? d3 * w3[i] : 0.0f;
+      d2s[16 * w + 4 * q + i][r] = d2;
+      gb2[i] += d2;
+      gw3[i] += d3 * h2[i];
+    }
+    __syncthreads();
+    // d1 = W2^T d2 where the unit is active
+    z = zero;
+    for (int k = 0; k < 16; ++k) z = mfma4(A2t[k], d2s[4 * k + q][r], z);
+    for (int i = 0; i < 4; ++i) {
+      const float d1 = h1[i] > 0.0f ? z[i] : 0.0f;
+      d1s[16 * w + 4 * q + i][r] = d1;
+      gb1[i] += d1;
+    }
+    for (int k = 0; k < 4; ++k) {  // samples 4 k ..
+      const float d = d2s[16 * w + r][4 * k + q];
+      for (int b = 0; b < 4; ++b) g2[b] = mfma4(d, h1s[16 * b + r][4 * k + q], g2[b]);
+    }
+    __syncthreads();  // d1s is there
+    for (int k = 0; k < 4; ++k) g1 = mfma4(d1s[16 * w + r][4 * k + q], r < kIn ? xs[4 * k + q][r] : 0.0f, g1);
+    __syncthreads();  // the next tile overwrites xs, h1s and d2s
   }
   float* out = partial + (int64_t)blockIdx.x * kP;
-  for (int r = 0; r < 16; ++r) out[oW2 + tid + kGradThreads * r] = g2[r];
-  for (int r = 0; r < 3; ++r) out[oW1 + tid + kGradThreads * r] = g1[r];
-  if (tid < kHid) out[oW3 + tid] = g3;
-  else if (tid < 2 * kHid) out[oB1 + tid - kHid] = g3;
-  else if (tid < 3 * kHid) out[oB2 + tid - 2 * kHid] = g3;
-  else if (tid == 3 * kHid) out[oB3] = g3;
-  if (tid < kTile) {
-    // wave 0 holds the tile losses: fixed-order wave sum
-    for (int off = 32; off > 0; off >>= 1) loss += __shfl_down(loss, off, 64);
-    if (tid == 0) partial_loss[blockIdx.x] = loss;
+  for (int i = 0; i < 4; ++i) {
+    const int unit = 16 * w + 4 * q + i;
+    for (int b = 0; b < 4; ++b) out[oW2 + unit * kHid + 16 * b + r] = g2[b][i];
+    if (r < kIn) out[oW1 + unit * kIn + r] = g1[i];
+    for (int off = 8; off > 0; off >>= 1) {  // over the samples
+      gw3[i] += __shfl_xor(gw3[i], off, 64);
+      gb1[i] += __shfl_xor(gb1[i], off, 64);
+      gb2[i] += __shfl_xor(gb2[i], off, 64);
+    }
+    if (r == 0) {
+      out[oW3 + unit] = gw3[i];
+      out[oB1 + unit] = gb1[i];
+      out[oB2 + unit] = gb2[i];
+    }
+  }
+  if (w == 0) {
+    for (int off = 8; off > 0; off >>= 1) {
+      gb3 += __shfl_xor(gb3, off, 64);
+      loss += __shfl_xor(loss, off, 64);
+    }
+    if (lane == 0) {
+      out[oB3] = gb3;
+      partial_loss[blockIdx.x] = loss;
+    }
   }
 }
 
-// grad[p] = sum_b partial[b][p]; loss = sum_b partial_loss[b] / B.
-__global__ void mlp_grad_reduce_kernel(const float* partial, const float* partial_loss, int nb, int64_t B,
-                                       float* grad, float* loss) {
-  const int p = blockIdx.x * blockDim.x + threadIdx.x;
-  if (p < kP) {
-    float s = 0.0f;
-    for (int b = 0; b < nb; ++b) s += partial[(int64_t)b * kP + p];
-    grad[p] = s;
-  }
-  if (p == 0) {
-    float s = 0.0f;
-    for (int b = 0; b < nb; ++b) s += partial_loss[b];
-    *loss = s / (float)B;
-  }
-}
+struct AdamArgs {
+  int step;  // 0: leave the parameters alone
+  float lr, beta1, beta2, eps;
+};
 
-// Adam (Kingma & Ba 2015, algorithm 1) on the FP32 master; weight entries
-// are re-rounded into the BF16 copy.
-__global__ void mlp_adam_kernel(MlpArgs a, const float* grad, int step, float lr, float beta1, float beta2,
-                                float eps) {
-  const int p = blockIdx.x * blockDim.x + threadIdx.x;
-  if (p >= kP) return;
-  const float g = grad[p];
-  const float m = beta1 * a.adam_m[p] + (1.0f - beta1) * g;
-  const float v = beta2 * a.adam_v[p] + (1.0f - beta2) * g * g;
-  a.adam_m[p] = m;
-  a.adam_v[p] = v;
-  const float mh = m / (1.0f - powf(beta1, (float)step));
-  const float vh = v / (1.0f - powf(beta2, (float)step));
-  const float w = a.params[p] - lr * mh / (sqrtf(vh) + eps);
-  a.params[p] = w;
-  a.wq[p] = f32_to_bf16(w);
+// grad[p] = sum_b partial[b][p]; loss = sum_b partial_loss[b] / B; and, for a
+// training step, Adam (Kingma & Ba 2015, algorithm 1) on the FP32 master, the
+// weight entries re-rounded into the BF16 copy.  A block takes 64 parameters,
+// its 16 waves each every 16th row of partial: the rows' latencies overlap
+// where one thread per parameter took them one after the other.
+constexpr int kReduceSlices = 16;
+__global__ __launch_bounds__(64 * kReduceSlices) void mlp_grad_reduce_kernel(MlpArgs a, const float* partial,
+                                                                             const float* partial_loss, int nb,
+                                                                             int64_t B, AdamArgs adam, float* grad,
+                                                                             float* loss) {
+  __shared__ float part[kReduceSlices][64];
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, p = blockIdx.x * 64 + lane;
+  float s = 0.0f;
+  if (p < kP)
+#pragma unroll 4
+    for (int b = w; b < nb; b += kReduceSlices) s += partial[(int64_t)b * kP + p];
+  part[w][lane] = s;
+  __syncthreads();
+  if (w == 0 && p < kP) {
+    float g = 0.0f;
+    for (int k = 0; k < kReduceSlices; ++k) g += part[k][lane];
+    grad[p] = g;
+    if (adam.step > 0) {
+      const float m = adam.beta1 * a.adam_m[p] + (1.0f - adam.beta1) * g;
+      const float v = adam.beta2 * a.adam_v[p] + (1.0f - adam.beta2) * g * g;
+      a.adam_m[p] = m;
+      a.adam_v[p] = v;
+      const float mh = m / (1.0f - powf(adam.beta1, (float)adam.step));
+      const float vh = v / (1.0f - powf(adam.beta2, (float)adam.step));
+      const float q = a.params[p] - adam.lr * mh / (sqrtf(vh) + adam.eps);
+      a.params[p] = q;
+      a.wq[p] = f32_to_bf16(q);
+    }
+  }
+  if (blockIdx.x == 0 && w == 1) {
+    float t = 0.0f;
+    for (int b = lane; b < nb; b += 64) t += partial_loss[b];
+    for (int off = 32; off > 0; off >>= 1) t += __shfl_xor(t, off, 64);
+    if (lane == 0) *loss = t / (float)B;
+  }
 }
 
 __global__ void mlp_round_kernel(MlpArgs a) {
@@ -467,7 +483,7 @@ __global__ void mlp_round_kernel(MlpArgs a) {
 
 int mlp_grad_blocks(int64_t B) {
   const int64_t tiles = (B + kTile - 1) / kTile;
-  return (int)std::min<int64_t>(std::max<int64_t>(tiles, 1), 512);
+  return (int)std::min<int64_t>(std::max<int64_t>(tiles, 1), 256);
 }
 
 hipError_t launch_features(const FeatureArgs& a, hipStream_t s) {
@@ -504,18 +520,13 @@ hipError_t launch_mlp_forward(const MlpArgs& a, const float* x, int64_t n, float
 }
 
 hipError_t launch_mlp_grad(const MlpArgs& a, const float* x, const float* y, const int32_t* idx, int64_t B,
-                           float* partial, float* partial_loss, float* grad, float* loss, hipStream_t s) {
+                           float* partial, float* partial_loss, int step, float lr, float* grad, float* loss,
+                           hipStream_t s) {
   if (B <= 0) return hipErrorInvalidValue;
   const int nb = mlp_grad_blocks(B);
   hipLaunchKernelGGL(mlp_grad_kernel, dim3(nb), dim3(kGradThreads), 0, s, a, x, y, idx, B, partial, partial_loss);
-  hipLaunchKernelGGL(mlp_grad_reduce_kernel, dim3((kP + 255) / 256), dim3(256), 0, s, partial, partial_loss, nb, B,
-                     grad, loss);
-  return hipGetLastError();
-}
-
-hipError_t launch_mlp_adam(const MlpArgs& a, const float* grad, int step, float lr, hipStream_t s) {
-  hipLaunchKernelGGL(mlp_adam_kernel, dim3((kP + 255) / 256), dim3(256), 0, s, a, grad, step, lr, 0.9f, 0.999f,
-                     1e-8f);
+  hipLaunchKernelGGL(mlp_grad_reduce_kernel, dim3((kP + 63) / 64), dim3(64 * kReduceSlices), 0, s, a, partial,
+                     partial_loss, nb, B, AdamArgs{step, lr, 0.9f, 0.999f, 1e-8f}, grad, loss);
   return hipGetLastError();
 }
 
