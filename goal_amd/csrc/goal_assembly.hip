@@ -145,16 +145,6 @@ template <int NQ, int G, typename S>
 struct SJac<NQ, MODEL_NEOHOOKEAN, G, S> {
   QPStore<MODEL_NEOHOOKEAN, S> qs[G][NQ];
 };
-template <int NN, int NQ, int G>
-struct SLoc {
-  double zq[G][NQ][4];      // z_diff (u,p) at qp
-  double zgq[G][NQ][4][3];  // grad z_diff
-  double zcq[G][NQ][4];     // z_coarse p and its gradient
-  double zd[G][4 * NN];
-  double zc[G][NN];
-};
-struct SNone {};
-
 // neo-Hookean: the next group's phase-A data, fetched by wave 1 while wave 0
 // computes the point states (phase C1)
 template <int NN, int G>
@@ -169,13 +159,13 @@ struct SNoPrefetch {};
 // precision; the vector-ALU FP32-tangent kernels measured slightly slower
 // with it, 10.50 -> 10.55 ms, chunked beside the gather)
 template <int NN, int NQ, int MODEL, int KIND, typename TE>
-constexpr bool kPrefetch = MODEL == MODEL_NEOHOOKEAN && KIND != ASM_LOCALIZE && Layout<NN, NQ, MODEL>::T >= 128 &&
+constexpr bool kPrefetch = MODEL == MODEL_NEOHOOKEAN && Layout<NN, NQ, MODEL>::T >= 128 &&
                            (std::is_same<TE, double>::value || Layout<NN, NQ, MODEL>::MF);
 
-// J2 assemblies other than the localization take their point states from the
-// thread-per-point pass (j2_point_kernel) instead of phases C1 and C2.
+// J2 assemblies take their point states from the thread-per-point pass
+// (j2_point_kernel) instead of phases C1 and C2.
 template <int MODEL, int KIND>
-constexpr bool kPointPass = MODEL == MODEL_J2 && KIND != ASM_LOCALIZE;
+constexpr bool kPointPass = MODEL == MODEL_J2;
 template <int NQ, int G>
 struct SJacD {
   double D[G][NQ][13][13];
@@ -183,12 +173,7 @@ struct SJacD {
 
 template <int NN, int NQ, int MODEL, int KIND, int G, typename TE = double>
 struct Smem : std::conditional<kPrefetch<NN, NQ, MODEL, KIND, TE>, SPrefetch<NN, G>, SNoPrefetch>::type {
-  static constexpr bool JK = KIND == ASM_JACOBIAN || KIND == ASM_ADJOINT;
-  using Ext = typename std::conditional<
-      JK && kPointPass<MODEL, KIND>, SJacD<NQ, G>,
-      typename std::conditional<
-          JK, SJac<NQ, MODEL, G, TE>,
-          typename std::conditional<KIND == ASM_LOCALIZE, SLoc<NN, NQ, G>, SNone>::type>::type>::type;
+  using Ext = typename std::conditional<kPointPass<MODEL, KIND>, SJacD<NQ, G>, SJac<NQ, MODEL, G, TE>>::type;
   SBase<NN, NQ, G> b;
   Ext ext;
 };
@@ -522,8 +507,7 @@ __global__ __launch_bounds__((Layout<NN, NQ, MODEL>::T), (elem_waves<NN, NQ, MOD
   using Lay = Layout<NN, NQ, MODEL>;
   using M = typename ModelOf<MODEL>::type;
   constexpr int G = Lay::G, ND = Lay::ND, T = Lay::T;
-  constexpr bool JAC = (KIND == ASM_JACOBIAN || KIND == ASM_ADJOINT);
-  constexpr bool LOC = (KIND == ASM_LOCALIZE);
+  static_assert(KIND == ASM_JACOBIAN || KIND == ASM_ADJOINT, "residuals have a kernel of their own");
   __shared__ Smem<NN, NQ, MODEL, KIND, G, TE> sm;
   auto& s = sm.b;
   const int tid = threadIdx.x;
@@ -541,7 +525,7 @@ __global__ __launch_bounds__((Layout<NN, NQ, MODEL>::T), (elem_waves<NN, NQ, MOD
   // registers one group ahead, so the loads are in flight during the previous
   // group's phases (ten-node tets have no registers to spare for it)
   constexpr bool PP = kPointPass<MODEL, KIND>;
-  constexpr int PPS = PP ? (JAC ? kPointTangent : kPointStress) : 1;
+  constexpr int PPS = PP ? kPointTangent : 1;
   constexpr int NPF = PP ? (G * NQ * PPS + T - 1) / T : 1;
   constexpr bool PPF = PP && NN == 4 && NQ == 1;
   double pf[PPF ? NPF : 1];
@@ -557,7 +541,7 @@ __global__ __launch_bounds__((Layout<NN, NQ, MODEL>::T), (elem_waves<NN, NQ, MOD
     }
   };
   if constexpr (PPF) fetch_points(0);
-  if constexpr (kPointPass<MODEL, KIND> && JAC) {
+  if constexpr (kPointPass<MODEL, KIND>) {
     // the point tangent's structural zeros (s3 rows of the p column, P and r1
     // rows of the grad-p columns): never stored, never overwritten
     for (int t = tid; t < G * NQ * 33; t += T) {
@@ -602,10 +586,7 @@ __global__ __launch_bounds__((Layout<NN, NQ, MODEL>::T), (elem_waves<NN, NQ, MOD
         const int el = t / ND, k = t % ND;
         const int64_t dof = 4 * (int64_t)s.conn[el][k >> 2] + (k & 3);
         s.x[el][k] = a.x[dof];
-        if constexpr (LOC) sm.ext.zd[el][k] = a.z_diff[dof];
       }
-    if constexpr (LOC)
-      for (int t = tid; t < nv * NN; t += T) sm.ext.zc[t / NN][t % NN] = a.z_coarse[4 * (int64_t)s.conn[t / NN][t % NN] + 3];
     }
     __syncthreads();
 
@@ -713,7 +694,7 @@ __global__ __launch_bounds__((Layout<NN, NQ, MODEL>::T), (elem_waves<NN, NQ, MOD
         const int r = t / npq, pq = t % npq;  // consecutive lanes: consecutive points
         if (r < 13) {
           s.sig[pq / NQ][pq % NQ][r] = v;
-        } else if constexpr (JAC) {
+        } else {
           auto& D = sm.ext.D[pq / NQ][pq % NQ];
           if (r < 130) D[(r - 13) % 13][(r - 13) / 13] = v;
           else if (r < 140) D[r - 130][9] = v;
@@ -757,22 +738,7 @@ __global__ __launch_bounds__((Layout<NN, NQ, MODEL>::T), (elem_waves<NN, NQ, MOD
         const double wdv = s.wdv[el][q];
         const int64_t sidx = e * NQ + q;
         M m;
-        if constexpr (MODEL == MODEL_J2) {
-          double Fpo[9];
-          for (int k = 0; k < 9; ++k) Fpo[k] = a.Fp_old[k * nqtot + sidx];
-          m.init(qp, mp, Fpo, a.eqps_old[sidx]);
-          if (m.failed()) atomicOr(a.status, 1);
-          if (a.save_state) {
-            a.eqps[sidx] = m.alpha;
-            if (m.plastic) {
-              double Fpn[9];
-              m.new_Fp(Fpo, Fpn);
-              for (int k = 0; k < 9; ++k) a.Fp[k * nqtot + sidx] = Fpn[k];
-            }
-          }
-        } else {
-          m.init(qp, mp);
-        }
+        m.init(qp, mp);
         if (a.save_state)
           for (int k = 0; k < 9; ++k) a.sigma[k * nqtot + sidx] = m.sig[k];
         for (int k = 0; k < 9; ++k) s.sig[el][q][k] = m.P[k] * wdv;
@@ -780,9 +746,9 @@ __global__ __launch_bounds__((Layout<NN, NQ, MODEL>::T), (elem_waves<NN, NQ, MOD
         double s3[3];
         st.value(s3);
         for (int j = 0; j < 3; ++j) s.sig[el][q][10 + j] = s3[j] * wdv;
-        if constexpr (JAC && MODEL == MODEL_NEOHOOKEAN) {
+        if constexpr (MODEL == MODEL_NEOHOOKEAN) {
           dev::nh_base(qp, m, st, sm.ext.qs[el][q].b);
-        } else if constexpr (JAC) {
+        } else {
           auto& D = sm.ext.D[el][q];
           sm.ext.qs[el][q].qp = qp;
           sm.ext.qs[el][q].st = st;
@@ -807,32 +773,12 @@ __global__ __launch_bounds__((Layout<NN, NQ, MODEL>::T), (elem_waves<NN, NQ, MOD
             for (int j = 0; j < 3; ++j) D[10 + j][10 + I] = ds3[j] * wdv;
           }
         }
-        if constexpr (LOC) {
-          for (int i = 0; i < 4; ++i) {
-            double z = 0.0, zg[3] = {0.0, 0.0, 0.0};
-            for (int n = 0; n < NN; ++n) {
-              const double zn = sm.ext.zd[el][4 * n + i];
-              z += zn * s.sh[el][q][n][0];
-              for (int j = 0; j < 3; ++j) zg[j] += zn * s.sh[el][q][n][1 + j];
-            }
-            sm.ext.zq[el][q][i] = z;
-            for (int j = 0; j < 3; ++j) sm.ext.zgq[el][q][i][j] = zg[j];
-          }
-          double z = 0.0, zg[3] = {0.0, 0.0, 0.0};
-          for (int n = 0; n < NN; ++n) {
-            const double zn = sm.ext.zc[el][n];
-            z += zn * s.sh[el][q][n][0];
-            for (int j = 0; j < 3; ++j) zg[j] += zn * s.sh[el][q][n][1 + j];
-          }
-          sm.ext.zcq[el][q][0] = z;
-          for (int j = 0; j < 3; ++j) sm.ext.zcq[el][q][1 + j] = zg[j];
-        }
       }
     }
     __syncthreads();
 
     // ---- C2: tangent columns d sig / d F_kL, one (element, point, direction) per lane
-    if constexpr (JAC && MODEL != MODEL_NEOHOOKEAN && !kPointPass<MODEL, KIND>) {
+    if constexpr (MODEL != MODEL_NEOHOOKEAN && !kPointPass<MODEL, KIND>) {
       for (int t = tid; t < nv * NQ * 9; t += T) {
         const int el = t / (NQ * 9), r = t % (NQ * 9);
         const int q = r / 9, c = r % 9;
@@ -858,22 +804,8 @@ __global__ __launch_bounds__((Layout<NN, NQ, MODEL>::T), (elem_waves<NN, NQ, MOD
       for (int q = 0; q < NQ; ++q) {
         const double* sg = s.sig[el][q];
         const double* sh = s.sh[el][q][n];
-        if constexpr (!LOC) {
-          if (i < 3) r += sg[3 * i] * sh[1] + sg[3 * i + 1] * sh[2] + sg[3 * i + 2] * sh[3];
-          else r += sg[9] * sh[0] + sg[10] * sh[1] + sg[11] * sh[2] + sg[12] * sh[3];
-        } else {
-          // DisplacementAdjoint / PressureAdjoint weights
-          // (src/goal_displacement_adjoint.cpp:37-53, src/goal_pressure_adjoint.cpp:38-49)
-          if (i < 3) {
-            const double z = sm.ext.zq[el][q][i];
-            const double* zg = sm.ext.zgq[el][q][i];
-            for (int J = 0; J < 3; ++J) r += sg[3 * i + J] * (zg[J] * sh[0] + z * sh[1 + J]);
-          } else {
-            r += sg[9] * sm.ext.zq[el][q][3] * sh[0];
-            const double zc = sm.ext.zcq[el][q][0];
-            for (int J = 0; J < 3; ++J) r += sg[10 + J] * (sm.ext.zcq[el][q][1 + J] * sh[0] + zc * sh[1 + J]);
-          }
-        }
+        if (i < 3) r += sg[3 * i] * sh[1] + sg[3 * i + 1] * sh[2] + sg[3 * i + 2] * sh[3];
+        else r += sg[9] * sh[0] + sg[10] * sh[1] + sg[11] * sh[2] + sg[12] * sh[3];
       }
       a.emr[(int64_t)s.rec[el][n] * 4 + i] = r;
     }
@@ -883,7 +815,7 @@ __global__ __launch_bounds__((Layout<NN, NQ, MODEL>::T), (elem_waves<NN, NQ, MOD
     TE* em;
     if constexpr (std::is_same<TE, float>::value) em = a.em32;
     else em = a.em;
-    if constexpr (JAC && MODEL == MODEL_NEOHOOKEAN && Lay::MF) {
+    if constexpr (MODEL == MODEL_NEOHOOKEAN && Lay::MF) {
       if constexpr (GOAL_MF_PIPE && std::is_same<TE, float>::value) {
         // matrix cores, pipelined: wave w takes elements w, w + 4, ... and
         // forms each tile's columns during the previous tile's products
@@ -912,7 +844,7 @@ __global__ __launch_bounds__((Layout<NN, NQ, MODEL>::T), (elem_waves<NN, NQ, MOD
           emit_tile_mfma<NN, TR, TE>(s.sh[el], s.wdv[el], sm.ext.qs[el], s.rec[el], em, tid & 63, task % NTL);
         }
       }
-    } else if constexpr (JAC && MODEL == MODEL_NEOHOOKEAN) {
+    } else if constexpr (MODEL == MODEL_NEOHOOKEAN) {
       if constexpr (T == 256 && G * NN <= 64 && std::is_same<TE, double>::value) {
         // displacement columns on waves 0-2, pressure columns on wave 3: the
         // closed-form column takes a different (shorter) path for pressure,
@@ -934,7 +866,7 @@ __global__ __launch_bounds__((Layout<NN, NQ, MODEL>::T), (elem_waves<NN, NQ, MOD
           emit_column_nh<NN, NQ, TR, TE>(s.sh[el], s.wdv[el], sm.ext.qs[el], col, s.rec[el], em);
         }
       }
-    } else if constexpr (JAC) {
+    } else {
       for (int t = tid; t < nv * ND; t += T) {
         const int el = t / ND, col = t % ND;
         emit_column<NN, NQ, TR, TE>(s.sh[el], sm.ext.D[el], col, s.rec[el], em);
@@ -1117,9 +1049,9 @@ __global__ __launch_bounds__(kGatherThreads) void gather_kernel(GatherArgs g) {
 // budget of the return map; here every lane takes a point and no barrier
 // holds it.  The arithmetic is that of phases B, C1 and C2, in the same order.
 template <int NN, int NQ>
-__global__ __launch_bounds__(256, 2) void j2_point_kernel(AsmArgs a, int jac) {
+__global__ __launch_bounds__(256, 2) void j2_point_kernel(AsmArgs a) {
   const int64_t npts = a.num_elems * NQ, nqtot = npts;
-  const int PS = jac ? kPointTangent : kPointStress;
+  constexpr int PS = kPointTangent;
   for (int64_t sidx = (int64_t)blockIdx.x * 256 + threadIdx.x; sidx < npts; sidx += (int64_t)gridDim.x * 256) {
     const int64_t e = sidx / NQ;
     const int q = (int)(sidx % NQ);
@@ -1177,7 +1109,6 @@ __global__ __launch_bounds__(256, 2) void j2_point_kernel(AsmArgs a, int jac) {
     double s3[3];
     st.value(s3);
     for (int j = 0; j < 3; ++j) o[64 * (10 + j)] = s3[j] * wdv;
-    if (!jac) continue;
     // p column: dsigma/dp = I (Mixed); grad-p columns: stabilization only
     for (int i = 0; i < 3; ++i)
       for (int jj = 0; jj < 3; ++jj) o[64 * (130 + 3 * i + jj)] = (qp.J * qp.Fi[3 * jj + i]) * wdv;
@@ -1239,8 +1170,7 @@ hipError_t launch4(const AsmArgs& a, int blocks, hipStream_t s) {
     if (!a.pt) return hipErrorInvalidValue;
     const int64_t npts = a.num_elems * NQ;
     const int pb = (int)std::min<int64_t>((npts + 255) / 256, 65536);
-    hipLaunchKernelGGL((j2_point_kernel<NN, NQ>), dim3(pb), dim3(256), 0, s, a,
-                       (KIND == ASM_JACOBIAN || KIND == ASM_ADJOINT) ? 1 : 0);
+    hipLaunchKernelGGL((j2_point_kernel<NN, NQ>), dim3(pb), dim3(256), 0, s, a);
   }
   if (blocks <= 0) blocks = resident_grid<NN, NQ, MODEL, KIND, TE>(a.num_elems);
   hipLaunchKernelGGL((element_kernel<NN, NQ, MODEL, KIND, TE>), dim3(blocks), dim3(Layout<NN, NQ, MODEL>::T), 0, s,
@@ -1253,14 +1183,12 @@ template <int NN, int NQ, int MODEL>
 hipError_t launch3(int kind, const AsmArgs& a, int blocks, hipStream_t s) {
   const bool f32 = a.em32 != nullptr;
   switch (kind) {
-    case ASM_RESIDUAL: return launch4<NN, NQ, MODEL, ASM_RESIDUAL, double>(a, blocks, s);
     case ASM_JACOBIAN:
       return f32 ? launch4<NN, NQ, MODEL, ASM_JACOBIAN, float>(a, blocks, s)
                  : launch4<NN, NQ, MODEL, ASM_JACOBIAN, double>(a, blocks, s);
     case ASM_ADJOINT:
       return f32 ? launch4<NN, NQ, MODEL, ASM_ADJOINT, float>(a, blocks, s)
                  : launch4<NN, NQ, MODEL, ASM_ADJOINT, double>(a, blocks, s);
-    case ASM_LOCALIZE: return launch4<NN, NQ, MODEL, ASM_LOCALIZE, double>(a, blocks, s);
     default: return hipErrorInvalidValue;
   }
 }
@@ -1428,8 +1356,6 @@ int group_size_of(int model) {
 }
 }  // namespace
 
-int point_stride(int kind) { return (kind == ASM_JACOBIAN || kind == ASM_ADJOINT) ? kPointTangent : kPointStress; }
-bool uses_point_pass(int model, int kind) { return model == MODEL_J2 && kind != ASM_LOCALIZE; }
 
 int element_group_size(int order, int quad_order, int model) {
   const int nq = quad_order == 1 ? 1 : 4;
@@ -1440,16 +1366,11 @@ int element_group_size(int order, int quad_order, int model) {
 namespace {
 template <int NN, int NQ, int MODEL>
 int resident_of_kind(int kind, bool f32, int64_t ne) {
-  const bool jac = kind == ASM_JACOBIAN || kind == ASM_ADJOINT;
-  if (jac && f32)
+  if (f32)
     return kind == ASM_JACOBIAN ? resident_grid<NN, NQ, MODEL, ASM_JACOBIAN, float>(ne)
                                 : resident_grid<NN, NQ, MODEL, ASM_ADJOINT, float>(ne);
-  switch (kind) {
-    case ASM_RESIDUAL: return resident_grid<NN, NQ, MODEL, ASM_RESIDUAL, double>(ne);
-    case ASM_JACOBIAN: return resident_grid<NN, NQ, MODEL, ASM_JACOBIAN, double>(ne);
-    case ASM_ADJOINT: return resident_grid<NN, NQ, MODEL, ASM_ADJOINT, double>(ne);
-    default: return resident_grid<NN, NQ, MODEL, ASM_LOCALIZE, double>(ne);
-  }
+  return kind == ASM_JACOBIAN ? resident_grid<NN, NQ, MODEL, ASM_JACOBIAN, double>(ne)
+                              : resident_grid<NN, NQ, MODEL, ASM_ADJOINT, double>(ne);
 }
 }  // namespace
 

@@ -608,19 +608,16 @@ void materialize(goal_solinfo s) {
 // 9.56 ms in one pass, 9.84 ms in 32 chunks), so the automatic setting is
 // one pass.
 // Same kernels and the same arithmetic as one pass: results are bitwise equal.
-int chunks_of(goal_mech m, bool want_vals) {
-  (void)want_vals;
-  return m->overlap >= 0 ? m->overlap : 0;
-}
+int chunks_of(goal_mech m) { return m->overlap >= 0 ? m->overlap : 0; }
 
-bool chunked(goal_mech m, bool want_vals) {
-  if (chunks_of(m, want_vals) < 2 || m->model != goal::MODEL_NEOHOOKEAN) return false;
+bool chunked(goal_mech m) {
+  if (chunks_of(m) < 2 || m->model != goal::MODEL_NEOHOOKEAN) return false;
   hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
   HIPCHK(hipStreamIsCapturing(stream(), &cs));
   return cs == hipStreamCaptureStatusNone;  // graphs keep the one-stream order
 }
 
-void run_chunked(goal_mech m, goal_solinfo s, int kind, goal::AsmArgs a, bool want_vals) {
+void run_chunked(goal_mech m, goal_solinfo s, int kind, goal::AsmArgs a) {
   goal_disc d = m->d;
   const int64_t ne = d->mesh.num_elems, nr = d->num_ranges;
   if (d->range_last_elem.empty()) {
@@ -635,7 +632,7 @@ void run_chunked(goal_mech m, goal_solinfo s, int kind, goal::AsmArgs a, bool wa
   }
   const int G = goal::element_group_size(d->mesh.order, m->quad_order, m->model);
   const int64_t ngroups = (ne + G - 1) / G;
-  const int K = (int)std::min<int64_t>(chunks_of(m, want_vals), ngroups);
+  const int K = (int)std::min<int64_t>(chunks_of(m), ngroups);
   int blocks = m->overlap_blocks;
   if (blocks <= 0) {
     const int full = goal::element_resident_grid(kind, d->mesh.order, m->quad_order, m->model, a.em32 != nullptr, ne);
@@ -646,10 +643,6 @@ void run_chunked(goal_mech m, goal_solinfo s, int kind, goal::AsmArgs a, bool wa
     HIPCHK(goal::launch_fill(s->dMdu.p, s->dMdu.n, 0.0, stream()));
     s->zero_dMdu = false;
   }
-  if (!want_vals && s->zero_vals) {
-    HIPCHK(goal::launch_fill(s->vals.p, s->vals.n, 0.0, stream()));
-    s->zero_vals = false;
-  }
   goal::GatherArgs g{};
   g.cap = d->gather_cap;
   g.inc_ptr = d->inc_ptr.p;
@@ -659,9 +652,9 @@ void run_chunked(goal_mech m, goal_solinfo s, int kind, goal::AsmArgs a, bool wa
   g.em = a.em;
   g.em32 = a.em32;
   g.R = s->R.p;
-  g.vals = want_vals ? s->vals.p : nullptr;
+  g.vals = s->vals.p;
   g.overwrite_R = s->zero_R ? 1 : 0;
-  g.overwrite_vals = (want_vals && s->zero_vals) ? 1 : 0;
+  g.overwrite_vals = s->zero_vals ? 1 : 0;
   int64_t r0 = 0;
   for (int c = 0; c < K; ++c) {
     a.group_lo = ngroups * c / K;
@@ -690,22 +683,21 @@ void run_chunked(goal_mech m, goal_solinfo s, int kind, goal::AsmArgs a, bool wa
     HIPCHK(hipEventRecord(m->ev[2], stream()));
     m->timed = true;
   }
-  s->zero_R = false;
-  if (want_vals) s->zero_vals = false;
+  s->zero_R = s->zero_vals = false;
 }
 
 // Element buffers between the two passes: the mechanics' own (allocated on
 // first use), or, with emr_buf/em_buf given, the caller's.
 // Doubles of J2 point states an assembly of this kind needs (0: none).
-int64_t point_states(goal_mech m, int kind) {
-  if (!goal::uses_point_pass(m->model, kind)) return 0;
-  return goal::point_state_doubles(m->d->mesh.num_elems * m->st->nq, goal::point_stride(kind));
+int64_t point_states(goal_mech m) {
+  if (m->model != goal::MODEL_J2) return 0;
+  return goal::point_state_doubles(m->d->mesh.num_elems * m->st->nq, goal::kPointTangent);
 }
 
 // Whether the element matrices of an assembly are summed where they are formed
 // (one kernel over node clusters) instead of going through memory.
-bool clustered(goal_mech m, bool want_vals) {
-  return want_vals && m->tangent == 64 && m->model == goal::MODEL_NEOHOOKEAN && m->quad_order == 2 && m->d->cluster &&
+bool clustered(goal_mech m) {
+  return m->tangent == 64 && m->model == goal::MODEL_NEOHOOKEAN && m->quad_order == 2 && m->d->cluster &&
          m->d->cluster->num_runs > 0;
 }
 
@@ -748,12 +740,43 @@ void run_clustered(goal_mech m, goal_solinfo s, int kind, const goal::AsmArgs& a
   s->zero_R = s->zero_vals = false;
 }
 
-// With emr_buf given (and pt_buf for J2) the assembly also stays in one pass
-// (the chunked path keeps a host-side table it builds on first use); the two
-// give the same bits.
-void run_assembly(goal_mech m, goal_solinfo s, int kind, goal::AsmArgs a, bool want_vals, double* emr_buf = nullptr,
+// Element residuals between the passes: the mechanics' own, allocated on first use.
+double* element_residuals(goal_mech m) {
+  const int64_t n = m->d->mesh.num_elems * 4 * (int64_t)m->d->mesh.nodes_per_elem;
+  if (m->emr.n < n) m->emr.alloc(n);
+  return m->emr.p;
+}
+
+// R (+)= the residuals of a residual kind.
+void run_residual(goal_mech m, goal_solinfo s, int kind, goal::AsmArgs a) {
+  goal_disc d = m->d;
+  a.emr = element_residuals(m);
+  a.rec = d->rec.p;
+  if (m->timing) HIPCHK(hipEventRecord(m->ev[0], stream()));
+  HIPCHK(goal::launch_residual(kind, d->mesh.order, m->quad_order, a, stream()));
+  if (m->timing) HIPCHK(hipEventRecord(m->ev[1], stream()));
+  HIPCHK(goal::launch_node_sum(d->mesh.num_nodes, d->inc_ptr.p, a.emr, s->zero_R ? 1 : 0, s->R.p, stream()));
+  s->zero_R = false;
+  if (s->zero_dMdu) {
+    HIPCHK(goal::launch_fill(s->dMdu.p, s->dMdu.n, 0.0, stream()));
+    s->zero_dMdu = false;
+  }
+  if (s->zero_vals) {
+    HIPCHK(goal::launch_fill(s->vals.p, s->vals.n, 0.0, stream()));
+    s->zero_vals = false;
+  }
+  if (m->timing) {
+    HIPCHK(hipEventRecord(m->ev[2], stream()));
+    m->timed = true;
+  }
+}
+
+// Residual and Jacobian.  With emr_buf given (and pt_buf for J2) the assembly
+// also stays in one pass (the chunked path keeps a host-side table it builds on
+// first use); the two give the same bits.
+void run_assembly(goal_mech m, goal_solinfo s, int kind, goal::AsmArgs a, double* emr_buf = nullptr,
                   double* em_buf = nullptr, double* pt_buf = nullptr) {
-  if (clustered(m, want_vals)) {
+  if (clustered(m)) {
     run_clustered(m, s, kind, a);
     return;
   }
@@ -761,23 +784,22 @@ void run_assembly(goal_mech m, goal_solinfo s, int kind, goal::AsmArgs a, bool w
   goal_disc d = m->d;
   const int64_t nd = 4 * (int64_t)d->mesh.nodes_per_elem;
   if (!emr_buf) {
-    if (m->emr.n < d->mesh.num_elems * nd) m->emr.alloc(d->mesh.num_elems * nd);
-    if (want_vals && m->em.n < d->mesh.num_elems * nd * nd) m->em.alloc(d->mesh.num_elems * nd * nd);
-    const int64_t np = point_states(m, kind);
+    emr_buf = element_residuals(m);
+    if (m->em.n < d->mesh.num_elems * nd * nd) m->em.alloc(d->mesh.num_elems * nd * nd);
+    const int64_t np = point_states(m);
     if (m->pt.n < np) m->pt.alloc(np);
-    emr_buf = m->emr.p;
     em_buf = m->em.p;
     pt_buf = m->pt.p;
   }
   a.pt = pt_buf;
   a.rec = d->rec.p;
   a.emr = emr_buf;
-  const bool f32 = want_vals && m->tangent == 32;
-  a.em = (want_vals && !f32) ? em_buf : nullptr;
+  const bool f32 = m->tangent == 32;
+  a.em = f32 ? nullptr : em_buf;
   a.em32 = f32 ? reinterpret_cast<float*>(em_buf) : nullptr;
   if (m->timing) HIPCHK(hipEventRecord(m->ev[0], stream()));
-  if (own_buffers && chunked(m, want_vals)) {
-    run_chunked(m, s, kind, a, want_vals);
+  if (own_buffers && chunked(m)) {
+    run_chunked(m, s, kind, a);
     return;
   }
   HIPCHK(goal::launch_element(kind, d->mesh.order, m->quad_order, a, asm_blocks(m), stream()));
@@ -785,10 +807,6 @@ void run_assembly(goal_mech m, goal_solinfo s, int kind, goal::AsmArgs a, bool w
   if (s->zero_dMdu) {
     HIPCHK(goal::launch_fill(s->dMdu.p, s->dMdu.n, 0.0, stream()));
     s->zero_dMdu = false;
-  }
-  if (!want_vals && s->zero_vals) {
-    HIPCHK(goal::launch_fill(s->vals.p, s->vals.n, 0.0, stream()));
-    s->zero_vals = false;
   }
   goal::GatherArgs g{};
   g.num_ranges = d->num_ranges;
@@ -801,9 +819,9 @@ void run_assembly(goal_mech m, goal_solinfo s, int kind, goal::AsmArgs a, bool w
   g.em = a.em;
   g.em32 = a.em32;
   g.R = s->R.p;
-  g.vals = want_vals ? s->vals.p : nullptr;
+  g.vals = s->vals.p;
   g.overwrite_R = s->zero_R ? 1 : 0;
-  g.overwrite_vals = (want_vals && s->zero_vals) ? 1 : 0;
+  g.overwrite_vals = s->zero_vals ? 1 : 0;
   HIPCHK(goal::launch_gather(d->mesh.order, g,
                              goal::gather_grid(d->mesh.order, g.em32 != nullptr, d->gather_cap, d->num_ranges),
                              stream()));
@@ -811,8 +829,7 @@ void run_assembly(goal_mech m, goal_solinfo s, int kind, goal::AsmArgs a, bool w
     HIPCHK(hipEventRecord(m->ev[2], stream()));
     m->timed = true;
   }
-  s->zero_R = false;
-  if (want_vals) s->zero_vals = false;
+  s->zero_R = s->zero_vals = false;
 }
 
 // ------------------------------------------------- multigrid preconditioner
@@ -2109,7 +2126,7 @@ int goal_asm_residual(goal_mech m, goal_solinfo s, int save_states) {
     require(m && s && s->d == m->d, "goal_asm_residual: bad arguments");
     goal::AsmArgs a = asm_args(m);
     a.save_state = save_states ? 1 : 0;
-    run_assembly(m, s, goal::ASM_RESIDUAL, a, false);
+    run_residual(m, s, goal::ASM_RESIDUAL, a);
     return finish_assembly(m);
   });
 }
@@ -2119,7 +2136,7 @@ int goal_asm_jacobian(goal_mech m, goal_solinfo s, int adjoint, int save_states)
     require(m && s && s->d == m->d, "goal_asm_jacobian: bad arguments");
     goal::AsmArgs a = asm_args(m);
     a.save_state = save_states ? 1 : 0;
-    run_assembly(m, s, adjoint ? goal::ASM_ADJOINT : goal::ASM_JACOBIAN, a, true);
+    run_assembly(m, s, adjoint ? goal::ASM_ADJOINT : goal::ASM_JACOBIAN, a);
     return finish_assembly(m);
   });
 }
@@ -2132,13 +2149,13 @@ int goal_asm_jacobian_noalloc(goal_mech m, goal_solinfo s, int adjoint, int save
     // element matrices (FP64; FP32 ones take half), element residuals, then
     // (J2) the point states
     const int kind = adjoint ? goal::ASM_ADJOINT : goal::ASM_JACOBIAN;
-    const bool pts = goal::uses_point_pass(m->model, kind);
+    const bool pts = m->model == goal::MODEL_J2;
     auto need_of = [&](int64_t n) {
-      return n * (nd * nd + nd) + (pts ? goal::point_state_doubles(n * m->st->nq, goal::point_stride(kind)) : 0);
+      return n * (nd * nd + nd) + (pts ? goal::point_state_doubles(n * m->st->nq, goal::kPointTangent) : 0);
     };
     const int64_t need = need_of(ne);
     if (need > kNoallocScratchDoubles) {
-      int64_t most = kNoallocScratchDoubles / (nd * nd + nd + (pts ? m->st->nq * goal::point_stride(kind) : 0));
+      int64_t most = kNoallocScratchDoubles / (nd * nd + nd + (pts ? m->st->nq * goal::kPointTangent : 0));
       while (most > 0 && need_of(most) > kNoallocScratchDoubles) --most;
       return set_error(GOAL_ERR_INVALID,
                        "goal_asm_jacobian_noalloc: %lld elements need %lld doubles of scratch, more than its "
@@ -2151,7 +2168,7 @@ int goal_asm_jacobian_noalloc(goal_mech m, goal_solinfo s, int adjoint, int save
     // every value the gather reads is written by this call's element pass, and
     // every point state the element pass reads by its point pass, so nothing
     // left from an earlier call needs clearing
-    run_assembly(m, s, kind, a, true, base + ne * nd * nd, base, base + ne * (nd * nd + nd));
+    run_assembly(m, s, kind, a, base + ne * nd * nd, base, base + ne * (nd * nd + nd));
     return finish_assembly(m);
   });
 }
@@ -2195,7 +2212,7 @@ int goal_batch_tune(goal_batch b, int reps, int* blocks_out, float* ms_out) {
         goal::AsmArgs a = asm_args(m);
         a.save_state = 1;
         HIPCHK(hipEventRecord(e0, stream()));
-        run_assembly(m, s, goal::ASM_JACOBIAN, a, true);
+        run_assembly(m, s, goal::ASM_JACOBIAN, a);
         HIPCHK(hipEventRecord(e1, stream()));
         HIPCHK(hipEventSynchronize(e1));
         float ms = 0.f;
@@ -2256,7 +2273,7 @@ int goal_batch_capture(goal_batch b) {
       b->infos[i]->zero_R = b->infos[i]->zero_dMdu = b->infos[i]->zero_vals = true;
       goal::AsmArgs a = asm_args(m);
       a.save_state = 1;
-      run_assembly(m, b->infos[i], goal::ASM_JACOBIAN, a, true);
+      run_assembly(m, b->infos[i], goal::ASM_JACOBIAN, a);
     }
     sync();
     if (b->exec) (void)hipGraphExecDestroy(b->exec);
@@ -2271,7 +2288,7 @@ int goal_batch_capture(goal_batch b) {
         b->infos[i]->zero_R = b->infos[i]->zero_dMdu = b->infos[i]->zero_vals = true;
         goal::AsmArgs a = asm_args(b->mechs[i]);
         a.save_state = 1;
-        run_assembly(b->mechs[i], b->infos[i], goal::ASM_JACOBIAN, a, true);
+        run_assembly(b->mechs[i], b->infos[i], goal::ASM_JACOBIAN, a);
       }
     } catch (...) {
       hipGraph_t g = nullptr;
@@ -2303,7 +2320,7 @@ int goal_asm_localize(goal_mech m, goal_solinfo s, const double* z_diff, const d
     a.save_state = 0;
     a.z_diff = z_diff;
     a.z_coarse = z_coarse;
-    run_assembly(m, s, goal::ASM_LOCALIZE, a, false);
+    run_residual(m, s, goal::ASM_LOCALIZE, a);
     return finish_assembly(m);
   });
 }

@@ -59,11 +59,10 @@ struct AsmArgs {
   // neo-Hookean only: this launch takes element groups [group_lo, group_hi)
   // (group_hi == 0: all of them), so an assembly can be split into chunks
   int64_t group_lo, group_hi;
-  // J2 (all kinds but ASM_LOCALIZE): the point states, written by a
-  // thread-per-point pass before the element pass reads them.  Per point
-  // p = e * nq + q, PS values, all times w dv: the generalized stress
-  // [P, r1, s3] (13) and, for the Jacobian kinds, the nonzero entries of the
-  // point tangent D (13 x 13; rows P, r1, s3; columns F, p, grad p):
+  // J2, Jacobian kinds: the point states, written by a thread-per-point pass
+  // before the element pass reads them.  Per point p = e * nq + q,
+  // kPointTangent values, all times w dv: the generalized stress [P, r1, s3]
+  // (13) and the nonzero entries of the point tangent D (13 x 13; rows P, r1, s3; columns F, p, grad p):
   //   13 + 13 c + r   D[r][c], c < 9 (the F directions, every row)
   //   130 + r         D[r][9], r < 10 (the p column; its s3 rows are zero)
   //   140 + 3 I + j   D[10 + j][10 + I] (grad p acts on s3 only)
@@ -77,16 +76,14 @@ struct AsmArgs {
 // different LDS banks (a 32-byte stride puts every eighth row on the same one).
 constexpr int kShapeRow = 5;
 
-// Doubles per point in AsmArgs::pt: residual kinds, Jacobian kinds.
+// Doubles per point: the generalized stress, and with the tangent's entries (AsmArgs::pt).
 constexpr int kPointStress = 13;
-constexpr int kPointTangent = 13 + 117 + 10 + 9;
+constexpr int kPointTangent = kPointStress + 117 + 10 + 9;
 __host__ __device__ inline int64_t point_state_index(int64_t p, int k, int ps) {
   return ((p >> 6) * ps + k) * 64 + (p & 63);
 }
 // Length of AsmArgs::pt for npts points: whole blocks of 64.
 inline int64_t point_state_doubles(int64_t npts, int ps) { return (npts + 63) / 64 * 64 * ps; }
-int point_stride(int kind);
-bool uses_point_pass(int model, int kind);
 
 // Node-owner gather of element residuals / matrices into R and the CSR values.
 struct GatherArgs {
@@ -125,7 +122,12 @@ struct QoiArgs {
   int* status;
 };
 
-// Launchers (goal_assembly.hip).  order: 1 or 2; quad_order: 1 or 2.
+// Residual kinds (goal_residual.hip): element residuals into a.emr, then their
+// sums by node, out[4 n + i] (+)= sum over node n's records.
+hipError_t launch_residual(int kind, int order, int quad_order, const AsmArgs& a, hipStream_t s);
+hipError_t launch_node_sum(int64_t nn, const int64_t* inc_ptr, const double* emr, int overwrite, double* out,
+                           hipStream_t s);
+// Launchers (goal_assembly.hip), Jacobian kinds.  order: 1 or 2; quad_order: 1 or 2.
 hipError_t launch_element(int kind, int order, int quad_order, const AsmArgs& a, int blocks, hipStream_t s);
 hipError_t launch_gather(int order, const GatherArgs& g, int blocks, hipStream_t s);
 // Nodes per run the gather kernel accepts (plan_gather_ranges must respect it).
