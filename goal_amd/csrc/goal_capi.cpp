@@ -222,12 +222,14 @@ struct AmgHierarchy {
   int coarse_n = 0;
 };
 
-// Node clusters of a quadratic disc (goal_cluster.hpp), made when the first
-// neo-Hookean four-point mechanics on it is; no runs where a node has more
-// neighbours than a run takes blocks, or no element.
+// Node clusters of a disc (goal_cluster.hpp), made when the first mechanics
+// that uses them is; no runs where a node has more neighbours than a run takes
+// blocks, or no element.
 struct ClusterPlan {
   int64_t num_runs = 0;
   DevBuf<int4> runs, chunks;
+  DevBuf<int2> spans;            // linear elements only
+  DevBuf<int32_t> linear_elems;  // linear elements only
   DevBuf<uint32_t> elems;
   DevBuf<goal::ClusterLane> lanes;
   DevBuf<int32_t> nodes, conn;
@@ -510,6 +512,57 @@ void cluster_build(goal_disc d) {
   d->cluster = std::move(p);
 }
 
+// The same for linear elements.
+void linear_cluster_build(goal_disc d) {
+  auto p = std::make_unique<ClusterPlan>();
+  const int64_t nn = d->mesh.num_nodes, ne = d->mesh.num_elems;
+  const int64_t groups = (nn + goal::kLinearNodes - 1) / goal::kLinearNodes;
+  // lanes are counted in 32 bits: at most one per visit (ten an element) and a wavefront's padding per run
+  if (d->max_degree <= goal::kClusterSlots && ne > 0 && 10 * ne + 64 * nn < (int64_t(1) << 31)) {
+    size_t tb = 0;
+    HIPCHK(goal::cluster_temp_bytes(nn, &tb));
+    DevBuf<uint8_t> temp, box;
+    DevBuf<uint32_t> code;
+    DevBuf<int32_t> place, parts, sizes, bad;
+    temp.alloc((int64_t)tb);
+    box.alloc(48);
+    code.alloc(2 * nn);
+    place.alloc(nn);
+    parts.alloc(groups + 1);
+    bad.alloc(1);
+    p->nodes.alloc(nn);
+    HIPCHK(goal::linear_order(d->coords.p, nn, temp.p, tb, reinterpret_cast<unsigned long long*>(box.p), code.p,
+                              code.p + nn, place.p, p->nodes.p, stream()));
+    const goal::ClusterMesh m{p->nodes.p, d->inc_ptr.p, d->inc.p,  d->row_ptr.p,
+                              d->posi.p,  d->pos.p,     d->cols.p, place.p};
+    HIPCHK(hipMemsetAsync(bad.p, 0, sizeof(int32_t), stream()));
+    HIPCHK(goal::linear_split(m, nn, temp.p, tb, parts.p, bad.p, stream()));
+    int32_t runs = 0, unfit = 0;
+    HIPCHK(hipMemcpyAsync(&runs, parts.p + groups, sizeof(int32_t), hipMemcpyDeviceToHost, stream()));
+    HIPCHK(hipMemcpyAsync(&unfit, bad.p, sizeof(int32_t), hipMemcpyDeviceToHost, stream()));
+    sync();
+    if (!unfit) {
+      sizes.alloc(2 * ((int64_t)runs + 1));
+      int32_t *nlanes = sizes.p, *nelems = sizes.p + runs + 1;
+      HIPCHK(goal::linear_tables(m, nn, runs, parts.p, temp.p, tb, nlanes, nelems, nullptr, nullptr, nullptr, nullptr,
+                                 stream()));
+      int32_t lanes = 0, elems = 0;
+      HIPCHK(hipMemcpyAsync(&lanes, nlanes + runs, sizeof(int32_t), hipMemcpyDeviceToHost, stream()));
+      HIPCHK(hipMemcpyAsync(&elems, nelems + runs, sizeof(int32_t), hipMemcpyDeviceToHost, stream()));
+      sync();
+      p->runs.alloc(runs);
+      p->spans.alloc(runs);
+      p->linear_elems.alloc(elems);
+      p->lanes.alloc(lanes);
+      HIPCHK(goal::linear_tables(m, nn, runs, parts.p, temp.p, tb, nlanes, nelems, p->runs.p, p->spans.p,
+                                 p->linear_elems.p, p->lanes.p, stream()));
+      p->num_runs = runs;
+    }
+    sync();  // the work buffers are released on return
+  }
+  d->cluster = std::move(p);
+}
+
 // The node adjacency's column lists on the host (the multigrid aggregation
 // runs there); copied from the device on first use.
 const std::vector<int32_t>& host_node_adj(goal_disc d) {
@@ -695,10 +748,54 @@ int64_t point_states(goal_mech m) {
 }
 
 // Whether the element matrices of an assembly are summed where they are formed
-// (one kernel over node clusters) instead of going through memory.
+// (over node clusters) instead of going through memory.
+bool uses_clusters(const goal_mech_s* m) {
+  return m->d->mesh.order == 2 ? m->quad_order == 2 && m->model == goal::MODEL_NEOHOOKEAN
+                               : m->quad_order == 1 && m->model != goal::MODEL_ELASTIC;
+}
 bool clustered(goal_mech m) {
-  return m->tangent == 64 && m->model == goal::MODEL_NEOHOOKEAN && m->quad_order == 2 && m->d->cluster &&
-         m->d->cluster->num_runs > 0;
+  return m->tangent == 64 && uses_clusters(m) && m->d->cluster && m->d->cluster->num_runs > 0;
+}
+
+// Linear elements: the point states in pt (kLinearPoint doubles an element), then the blocks.
+void run_linear_clustered(goal_mech m, goal_solinfo s, int kind, goal::AsmArgs a, double* pt) {
+  goal_disc d = m->d;
+  const ClusterPlan& p = *d->cluster;
+  if (!pt) {
+    const int64_t n = goal::kLinearPoint * d->mesh.num_elems;
+    if (m->pt.n < n) m->pt.alloc(n);
+    pt = m->pt.p;
+  }
+  a.pt = pt;
+  goal::LinearArgs c{};
+  c.num_runs = p.num_runs;
+  c.num_elems = a.num_elems;
+  c.runs = p.runs.p;
+  c.spans = p.spans.p;
+  c.elems = p.linear_elems.p;
+  c.lanes = p.lanes.p;
+  c.nodes = p.nodes.p;
+  c.row_ptr = d->row_ptr.p;
+  c.pt = pt;
+  c.R = s->R.p;
+  c.vals = s->vals.p;
+  c.overwrite_R = s->zero_R ? 1 : 0;
+  c.overwrite_vals = s->zero_vals ? 1 : 0;
+  c.xcd_remap = a.xcd_remap;
+  if (m->timing) HIPCHK(hipEventRecord(m->ev[0], stream()));
+  HIPCHK(goal::launch_linear_points(a, stream()));
+  if (m->timing) HIPCHK(hipEventRecord(m->ev[1], stream()));
+  if (s->zero_dMdu) {
+    HIPCHK(goal::launch_fill(s->dMdu.p, s->dMdu.n, 0.0, stream()));
+    s->zero_dMdu = false;
+  }
+  HIPCHK(goal::launch_linear_cluster(kind == goal::ASM_ADJOINT, m->model == goal::MODEL_J2, c, asm_blocks(m),
+                                     stream()));
+  if (m->timing) {
+    HIPCHK(hipEventRecord(m->ev[2], stream()));
+    m->timed = true;
+  }
+  s->zero_R = s->zero_vals = false;
 }
 
 void run_clustered(goal_mech m, goal_solinfo s, int kind, const goal::AsmArgs& a) {
@@ -777,7 +874,8 @@ void run_residual(goal_mech m, goal_solinfo s, int kind, goal::AsmArgs a) {
 void run_assembly(goal_mech m, goal_solinfo s, int kind, goal::AsmArgs a, double* emr_buf = nullptr,
                   double* em_buf = nullptr, double* pt_buf = nullptr) {
   if (clustered(m)) {
-    run_clustered(m, s, kind, a);
+    if (m->d->mesh.order == 2) run_clustered(m, s, kind, a);
+    else run_linear_clustered(m, s, kind, a, em_buf);  // a matrix buffer takes the smaller states
     return;
   }
   const bool own_buffers = emr_buf == nullptr;
@@ -2048,7 +2146,10 @@ int goal_mech_create(goal_disc d, goal_states st, int num_sets, const goal_mater
     m->status.alloc(1);
     HIPCHK(hipMemsetAsync(m->status.p, 0, sizeof(int), stream()));
     m->elem_value.alloc(d->mesh.num_elems);
-    if (m->model == GOAL_MODEL_NEOHOOKEAN && d->mesh.order == 2 && quad_order == 2 && !d->cluster) cluster_build(d);
+    if (uses_clusters(m.get()) && !d->cluster) {
+      if (d->mesh.order == 2) cluster_build(d);
+      else linear_cluster_build(d);
+    }
     sync();
     *out = m.release();
     return GOAL_OK;

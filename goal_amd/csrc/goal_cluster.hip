@@ -247,7 +247,7 @@ __global__ __launch_bounds__(kBlock) void cluster_lanes_kernel(ClusterMesh m, co
 #pragma unroll
           for (int k = 0; k < 4; ++k) {
             const int ru = (four >> (8 * k)) & 255;
-            if (ru < mine || (ru == mine && u + k < s)) lane += ru < 4 ? 16 >> ru : 1;
+            if (ru < mine || (ru == mine && u + k < s)) lane += ru < 9 ? cluster_lanes_of_rank(ru) : 0;
           }
         }
         int node = 0;
@@ -476,6 +476,10 @@ struct PairSum {
 #pragma unroll
     for (int k = 0; k < 4; ++k) f(r[k]);
   }
+  template <typename F>
+  __device__ __forceinline__ void all(F f) {
+    each(f);
+  }
 };
 
 // Adds one visit: element table P, local nodes la and lb; shape[4 a + q] = N_a
@@ -544,14 +548,18 @@ __device__ __forceinline__ void visit(const double* P, const double* shape, int 
 // lane ^ 4 and ^ 8 by then).
 template <int STEP>
 __device__ inline double partner(double v) {
-  constexpr int ctrl = STEP == 0 ? 0xB1 : STEP == 1 ? 0x4E : STEP == 2 ? 0x141 : 0x140;
-  const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), ctrl, 0xF, 0xF, true);
-  const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), ctrl, 0xF, 0xF, true);
-  return __hiloint2double(hi, lo);
+  if constexpr (STEP >= 4) {  // lane ^ 16, lane ^ 32: pairs with more than 48 visits
+    return __shfl_xor(v, 1 << STEP, 64);
+  } else {
+    constexpr int ctrl = STEP == 0 ? 0xB1 : STEP == 1 ? 0x4E : STEP == 2 ? 0x141 : 0x140;
+    const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), ctrl, 0xF, 0xF, true);
+    const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), ctrl, 0xF, 0xF, true);
+    return __hiloint2double(hi, lo);
+  }
 }
-template <int STEP>
-__device__ __forceinline__ void join(int lg, PairSum& s) {
-  s.each([&](double& v) {
+template <int STEP, typename Sum>
+__device__ __forceinline__ void join(int lg, Sum& s) {
+  s.all([&](double& v) {
     const double o = partner<STEP>(v);
     if (lg > STEP) v += o;
   });
@@ -709,6 +717,479 @@ __global__ __launch_bounds__(kClusterThreads, 3) void cluster_kernel(ClusterArgs
   }
 }
 
+// ----------------------------------------------------------- linear tets
+// One workgroup per run of nodes [lo, hi): its incidences in LDS, the distinct
+// elements among them numbered by first appearance.
+struct LinearRun {
+  int nodes[kLinearNodes], first[kLinearNodes + 1], rec0[kLinearNodes + 1];
+  int elem[kLinearRecs], info[kLinearRecs];  // element; first incidence of it << 2 | local node
+  uint16_t slot[kLinearRecs], pos[4 * kLinearRecs];
+  int ne;
+};
+// false: too many incidences or blocks (nothing else is set then)
+__device__ bool linear_load(const ClusterMesh& m, int64_t lo, int64_t hi, LinearRun& r) {
+  const int tid = threadIdx.x, nn = (int)(hi - lo);
+  __syncthreads();
+  if (tid == 0) {
+    r.first[0] = r.rec0[0] = 0;
+    for (int i = 0; i < nn; ++i) {
+      const int64_t n = m.nodes[lo + i];
+      r.nodes[i] = (int)n;
+      const int64_t deg = (m.row_ptr[4 * n + 1] - m.row_ptr[4 * n]) / 4, inc = m.inc_ptr[n + 1] - m.inc_ptr[n];
+      // no overflow: a node has at most 65535 neighbours, and once over a limit the sums only stay there
+      r.first[i + 1] = (int)min((int64_t)r.first[i] + deg, (int64_t)1 << 20);
+      r.rec0[i + 1] = (int)min((int64_t)r.rec0[i] + (inc > 0 ? inc : (int64_t)1 << 20), (int64_t)1 << 20);
+    }
+  }
+  __syncthreads();
+  const int n = r.rec0[nn];
+  if (n > kLinearRecs || r.first[nn] > kClusterSlots) return false;  // a node without elements ends here too
+  for (int t = tid; t < n; t += kBlock) {
+    int node = 0;
+    while (r.rec0[node + 1] <= t) ++node;
+    const int64_t k = m.inc_ptr[r.nodes[node]] + (t - r.rec0[node]);
+    const int32_t s = m.inc[k];
+    r.elem[t] = s / 4;
+    r.info[t] = s % 4;
+    for (int b = 0; b < 4; ++b) r.pos[4 * t + b] = m.posi[4 * k + b];
+  }
+  __syncthreads();
+  for (int t = tid; t < n; t += kBlock) {
+    const int e = r.elem[t];
+    int u = 0;
+    while (r.elem[u] != e) ++u;
+    r.info[t] |= u << 2;
+  }
+  __syncthreads();
+  if (tid < 64) {
+    int base = 0;
+    for (int t0 = 0; t0 < n; t0 += 64) {
+      const int t = t0 + tid;
+      const bool is = t < n && (r.info[t] >> 2) == t;
+      const unsigned long long b = __ballot(is);
+      if (is) r.slot[t] = (uint16_t)(base + __popcll(b & ((1ull << tid) - 1)));
+      base += __popcll(b);
+    }
+    if (tid == 0) r.ne = base;
+  }
+  __syncthreads();
+  return true;
+}
+
+// parts[g]: the runs (1, 2, 4 or 8) that group g's nodes need to fit.
+__global__ __launch_bounds__(kBlock) void linear_split_kernel(ClusterMesh m, int64_t nn, int32_t* parts,
+                                                              int32_t* bad) {
+  __shared__ LinearRun r;
+  const int64_t lo = (int64_t)blockIdx.x * kLinearNodes, hi = min(lo + kLinearNodes, nn);
+  int p = 1;
+  for (; p <= kLinearNodes; p *= 2) {
+    const int64_t step = kLinearNodes / p;
+    bool fits = true;
+    for (int64_t a = lo; a < hi && fits; a += step) fits = linear_load(m, a, min(a + step, hi), r) && r.ne <= kLinearElems;
+    if (fits) break;
+  }
+  if (threadIdx.x) return;
+  if (p > kLinearNodes) {
+    atomicMax(bad, 1);
+    p = kLinearNodes;
+  }
+  const int64_t step = kLinearNodes / p;
+  parts[blockIdx.x] = (int)((hi - lo + step - 1) / step);
+}
+
+__global__ __launch_bounds__(kBlock) void linear_tables_kernel(ClusterMesh m, int64_t nn, const int32_t* parts,
+                                                               int32_t* nlanes, int32_t* nelems, int4* runs,
+                                                               int2* spans, int32_t* elems, ClusterLane* lanes) {
+  __shared__ LinearRun r;
+  __shared__ int cnt[kClusterSlots], total;
+  __shared__ __align__(4) uint8_t rank[kClusterSlots + 4];
+  const int tid = threadIdx.x;
+  const int64_t lo = (int64_t)blockIdx.x * kLinearNodes, hi = min(lo + kLinearNodes, nn);
+  const int run0 = parts[blockIdx.x], np = parts[blockIdx.x + 1] - run0;
+  int64_t step = kLinearNodes;  // np runs came from 1, 2, 4 or 8 equal parts of the group, the last ones empty at the end of the nodes
+  while ((hi - lo + step - 1) / step < np) step /= 2;
+  for (int p = 0; p < np; ++p) {
+    const int64_t a0 = lo + p * step, a1 = min(a0 + step, hi);
+    const int run = run0 + p;
+    linear_load(m, a0, a1, r);  // fits: linear_split saw to it
+    const int rn = (int)(a1 - a0), n = r.rec0[rn], nb = r.first[rn], nb4 = (nb + 3) / 4 * 4;
+    if (tid == 0) total = 0;
+    for (int s = tid; s < nb; s += kBlock) cnt[s] = 0;
+    __syncthreads();
+    for (int t = tid; t < n; t += kBlock) {
+      int node = 0;
+      while (r.rec0[node + 1] <= t) ++node;
+      for (int b = 0; b < 4; ++b) atomicAdd(&cnt[r.first[node] + r.pos[4 * t + b]], 1);
+    }
+    __syncthreads();
+    for (int s = tid; s < nb4; s += kBlock) {
+      int c = s < nb ? cnt[s] : 0;
+      if (c) {
+        int node = 0;
+        while (r.first[node + 1] <= s) ++node;
+        const int64_t ga = r.nodes[node], gb = m.cols[m.row_ptr[4 * ga] + 4 * (s - r.first[node])] / 4;
+        if (m.place[gb] < m.place[ga]) c = cnt[s] = 0;  // the pair is b's run's
+        else atomicAdd(&total, 1 << cluster_log_lanes(c));
+      }
+      rank[s] = (uint8_t)cluster_rank(c);
+    }
+    __syncthreads();
+    if (!lanes) {
+      if (tid == 0) {
+        nlanes[run] = (total + 63) / 64 * 64;
+        nelems[run] = r.ne;
+      }
+      continue;
+    }
+    const int base = nlanes[run], end = nlanes[run + 1], e0 = nelems[run];
+    if (tid == 0) {
+      runs[run] = int4{(int)a0, (int)a1, e0, r.ne};
+      spans[run] = int2{base, end};
+    }
+    for (int t = tid; t < n; t += kBlock)
+      if ((r.info[t] >> 2) == t) elems[e0 + r.slot[t]] = r.elem[t];
+    for (int t = base + total + tid; t < end; t += kBlock) lanes[t] = ClusterLane{0, 0};  // idle lanes: no visits
+    for (int s = tid; s < nb; s += kBlock) {
+      const int c = cnt[s];
+      if (!c) continue;
+      const int mine = rank[s], lg = cluster_log_lanes(c);
+      int lane = 0;  // lanes of the pairs before this one
+      for (int u = 0; u < nb; u += 4) {
+        const uint32_t four = *reinterpret_cast<const uint32_t*>(rank + u);
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+          const int ru = (four >> (8 * k)) & 255;
+          if (ru < mine || (ru == mine && u + k < s)) lane += ru < 9 ? cluster_lanes_of_rank(ru) : 0;
+        }
+      }
+      int node = 0;
+      while (r.first[node + 1] <= s) ++node;
+      const int pos = s - r.first[node];
+      const int64_t ga = r.nodes[node], gb = m.cols[m.row_ptr[4 * ga] + 4 * pos] / 4;
+      const int64_t rb = m.row_ptr[4 * gb];
+      uint64_t pos_t = 0;
+      // lane j's visits, in incidence order: the pair's visits v = j, j + 2^lg, ..
+      for (int j = 0; j < (1 << lg); ++j) {
+        uint64_t w = 0;
+        int v = 0, k = 0;
+        for (int t = r.rec0[node]; t < r.rec0[node + 1]; ++t)
+          for (int b = 0; b < 4; ++b)
+            if (r.pos[4 * t + b] == pos) {
+              if ((v & ((1 << lg) - 1)) == j) {
+                const int a = r.info[t] & 3;
+                w |= (uint64_t)(r.slot[r.info[t] >> 2] | (a << 9) | (b << 11)) << (13 * k++);
+                pos_t = m.pos[((int64_t)r.elem[t] * 4 + b) * 4 + a];
+              }
+              ++v;
+            }
+        ClusterLane o;
+        o.x = w | ((uint64_t)k << kLaneCount) | ((uint64_t)pos << kLanePos) | ((uint64_t)node << kLaneNode) |
+              ((uint64_t)lg << kLaneLog) | kLaneFirst | (ga == gb ? kLaneDiag : 0);
+        o.y = (uint64_t)(rb / 16) | ((uint64_t)((m.row_ptr[4 * gb + 1] - rb) / 4) << kLaneDegT) | (pos_t << kLanePosT);
+        lanes[base + lane + j] = o;
+      }
+    }
+  }
+}
+
+// An element's point state: f_a = F^{-T} grad N_a of its nodes, then with
+// dev = dev(b) (neo-Hookean: b = F F^T; J2: the trial elastic b) and the scalars
+// the same tangent as the quadratic elements' (top of this file), with C times
+// theta for J2 and, where it yields, one more term.  J2's stress is s = theta
+// mu dev, theta = 1 - 2 mubar dgam / |s_tr|; along L = e_k (x) f_b, with ed = dev
+// f, ee = dev ed, t3 = tr b / 3, nu = mu / |s_tr| and the last Newton iterate's
+// derivative alpha d|s_tr| + beta d mubar,
+//   ds = theta ds_tr + N kappa_k,  N f_a = nu ed_a,
+//   kappa_k = A (2 mu nu (ee_b + t3 ed_b) - 2/3 |s_tr| f_b)_k + B (2 mu / 3) ed_bk,
+//   A = 2 mubar (dgam / |s_tr| - alpha),  B = -2 (dgam + mubar beta),
+// so K(ai, bk) += ed_ai (q1 ee_b + q2 ed_b + q3 f_b)_k.  All times w dv.
+enum : int { lF = 0, lDev = 12, lC = 18, lCT, lPJ, lJ, lBeta, lT, lPi, lKap = lPi + 3, lR1, lQ1, lQ2, lQ3, lPt };
+static_assert(lPt == kLinearPoint, "32 doubles an element");
+
+// Bound by its memory traffic (256 bytes written an element; 1.0 ms on the 5.3 M-tet J2 bar).
+template <int MODEL>
+__global__ __launch_bounds__(256) void linear_points_kernel(AsmArgs a) {
+  const int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x, ne = a.num_elems;
+  if (e >= ne) return;
+  const int4 ec4 = reinterpret_cast<const int4*>(a.conn)[e];
+  const int32_t ec[4] = {ec4.x, ec4.y, ec4.z, ec4.w};
+  const MatParams mp = a.mats[a.elem_set ? a.elem_set[e] : 0];
+  double D[3][4], p = 0.0;
+  {
+    double U[4][4];
+#pragma unroll
+    for (int v = 0; v < 4; ++v)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) U[v][i] = a.x[4 * (int64_t)ec[v] + i];
+    p = 0.25 * ((U[0][3] + U[1][3]) + (U[2][3] + U[3][3]));
+#pragma unroll
+    for (int v = 1; v < 4; ++v)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) D[v - 1][i] = U[v][i] - U[0][i];
+  }
+  double gl[4][3], W, tau;
+  {
+    double X[4][3];
+#pragma unroll
+    for (int v = 0; v < 4; ++v)
+#pragma unroll
+      for (int c = 0; c < 3; ++c) X[v][c] = a.coords[3 * (int64_t)ec[v] + c];
+    W = dev::tet_gradlambda(X, gl) / 6.0;
+    tau = a.stabilization ? dev::stab_tau(X, mp) : 0.0;
+  }
+  dev::QP qp;
+#pragma unroll
+  for (int j = 0; j < 3; ++j) {
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {
+      qp.H[3 * i + j] = D[0][i] * gl[1][j] + D[1][i] * gl[2][j] + D[2][i] * gl[3][j];
+      qp.F[3 * i + j] = qp.H[3 * i + j] + (i == j ? 1.0 : 0.0);
+    }
+    qp.g[j] = D[0][3] * gl[1][j] + D[1][3] * gl[2][j] + D[2][3] * gl[3][j];
+  }
+  qp.p = p;
+  qp.J = dev::det3(qp.F);
+  dev::inv3(qp.F, qp.J, qp.Fi);
+  const double J = qp.J, iJ = 1.0 / J;
+  double o[kLinearPoint];
+  if constexpr (MODEL == MODEL_NEOHOOKEAN) {
+    double b[6];
+#pragma unroll
+    for (int i = 0; i < 3; ++i)
+#pragma unroll
+      for (int j = i; j < 3; ++j)
+        b[sym(i, j)] = qp.F[3 * i] * qp.F[3 * j] + qp.F[3 * i + 1] * qp.F[3 * j + 1] + qp.F[3 * i + 2] * qp.F[3 * j + 2];
+    const double third = (b[0] + b[3] + b[5]) / 3.0;
+    b[0] -= third;
+    b[3] -= third;
+    b[5] -= third;
+    const double Jm13 = 1.0 / cbrt(J), Jm23 = Jm13 * Jm13;
+    if (a.save_state) {
+      const double m = mp.mu * (Jm23 * Jm23 * Jm13);
+#pragma unroll
+      for (int k = 0; k < 9; ++k) a.sigma[k * ne + e] = m * b[sym(k / 3, k % 3)] + (k % 4 == 0 ? p : 0.0);
+    }
+#pragma unroll
+    for (int k = 0; k < 6; ++k) o[lDev + k] = b[k];
+    o[lC] = W * (mp.mu * Jm23);
+    o[lCT] = o[lC] * third;
+    o[lQ1] = o[lQ2] = o[lQ3] = 0.0;
+  } else {
+    double Fpo[9];
+    for (int k = 0; k < 9; ++k) Fpo[k] = a.Fp_old[k * ne + e];
+    dev::J2Model m;
+    m.init(qp, mp, Fpo, a.eqps_old[e]);
+    if (m.failed()) atomicOr(a.status, 1);
+    if (a.save_state) {
+      a.eqps[e] = m.alpha;
+      if (m.plastic) {
+        double Fpn[9];
+        m.new_Fp(Fpo, Fpn);
+        for (int k = 0; k < 9; ++k) a.Fp[k * ne + e] = Fpn[k];
+      }
+      for (int k = 0; k < 9; ++k) a.sigma[k * ne + e] = m.sig[k];
+    }
+    const double mu = mp.mu, t3 = m.mubar / mu;
+#pragma unroll
+    for (int i = 0; i < 3; ++i)
+#pragma unroll
+      for (int j = i; j < 3; ++j) o[lDev + sym(i, j)] = m.str[3 * i + j] / mu;
+    double theta = 1.0, q1 = 0.0, q2 = 0.0, q3 = 0.0;
+    if (m.plastic) {
+      double X, al, bt;
+      (void)m.newton(1.0, 0.0, X, al);
+      (void)m.newton(0.0, 1.0, X, bt);
+      theta = 1.0 - 2.0 * m.mubar * m.dgam / m.smag;
+      const double A = 2.0 * m.mubar * (m.dgam / m.smag - al), B = -2.0 * (m.dgam + m.mubar * bt);
+      const double nu = mu / m.smag;
+      q1 = W * nu * (2.0 * mu * A * nu);
+      q2 = W * nu * (2.0 * mu * A * nu * t3 + (2.0 * mu / 3.0) * B);
+      q3 = (-2.0 / 3.0) * W * A * mu;
+    }
+    o[lC] = W * (theta * mu);
+    o[lCT] = o[lC] * t3;
+    o[lQ1] = q1;
+    o[lQ2] = q2;
+    o[lQ3] = q3;
+  }
+#pragma unroll
+  for (int v = 0; v < 4; ++v)
+#pragma unroll
+    for (int k = 0; k < 3; ++k)
+      o[lF + 3 * v + k] = qp.Fi[k] * gl[v][0] + qp.Fi[3 + k] * gl[v][1] + qp.Fi[6 + k] * gl[v][2];
+#pragma unroll
+  for (int k = 0; k < 3; ++k) o[lPi + k] = qp.Fi[k] * qp.g[0] + qp.Fi[3 + k] * qp.g[1] + qp.Fi[6 + k] * qp.g[2];
+  o[lPJ] = W * (p * J);
+  o[lJ] = W * J;
+  o[lBeta] = W * (-0.5 * (J + iJ));
+  o[lT] = W * J * tau;
+  o[lKap] = W / mp.kappa;
+  o[lR1] = W * (p / mp.kappa - 0.5 * (J - iJ));
+  double2* out = reinterpret_cast<double2*>(a.pt + kLinearPoint * e);
+#pragma unroll
+  for (int k = 0; k < kLinearPoint / 2; ++k) out[k] = double2{o[2 * k], o[2 * k + 1]};
+}
+
+// A pair's sums for linear tets: with plastic points K(ai, bk) and K(bk, ai) differ (vu[3 i + k] = K(bk, ai)).
+template <bool PLASTIC>
+struct LinearSum : PairSum {
+  double vu[PLASTIC ? 9 : 1];
+  template <typename F>
+  __device__ __forceinline__ void all(F f) {
+    each(f);
+    if constexpr (PLASTIC)
+#pragma unroll
+      for (int k = 0; k < 9; ++k) f(vu[k]);
+  }
+};
+
+template <bool PLASTIC>
+__device__ __forceinline__ void linear_visit(const double* p, int la, int lb, bool diag, LinearSum<PLASTIC>& s) {
+  double fa[3], fb[3], ha[3], hb[3], dv[6];
+#pragma unroll
+  for (int k = 0; k < 3; ++k) {
+    fa[k] = p[lF + 3 * la + k];
+    fb[k] = p[lF + 3 * lb + k];
+  }
+#pragma unroll
+  for (int k = 0; k < 6; ++k) dv[k] = p[lDev + k];
+#pragma unroll
+  for (int j = 0; j < 3; ++j) {
+    ha[j] = dv[sym(j, 0)] * fa[0] + dv[sym(j, 1)] * fa[1] + dv[sym(j, 2)] * fa[2];
+    hb[j] = dv[sym(j, 0)] * fb[0] + dv[sym(j, 1)] * fb[1] + dv[sym(j, 2)] * fb[2];
+  }
+  const double d = fa[0] * fb[0] + fa[1] * fb[1] + fa[2] * fb[2];
+  {
+    const double C = p[lC], CT = p[lCT], PJ = p[lPJ];
+    const double hd = ha[0] * fb[0] + ha[1] * fb[1] + ha[2] * fb[2];
+    const double m = (-2.0 / 3.0) * C, A = PJ - (2.0 / 3.0) * CT, S = CT - PJ, gg = C * hd + CT * d;
+    if (diag) {
+#pragma unroll
+      for (int i = 0; i < 3; ++i) s.r[i] += C * ha[i] + PJ * fa[i];
+    }
+    double xa[3], xb[3];  // q1 ee + q2 ed + q3 f
+    if constexpr (PLASTIC) {
+      const double q1 = p[lQ1], q2 = p[lQ2], q3 = p[lQ3];
+#pragma unroll
+      for (int j = 0; j < 3; ++j) {
+        xa[j] = q1 * (dv[sym(j, 0)] * ha[0] + dv[sym(j, 1)] * ha[1] + dv[sym(j, 2)] * ha[2]) + q2 * ha[j] + q3 * fa[j];
+        xb[j] = q1 * (dv[sym(j, 0)] * hb[0] + dv[sym(j, 1)] * hb[1] + dv[sym(j, 2)] * hb[2]) + q2 * hb[j] + q3 * fb[j];
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {
+      const double u = m * ha[i] + A * fa[i], v = m * fa[i], w = S * fb[i];
+#pragma unroll
+      for (int k = 0; k < 3; ++k) {
+        double t = u * fb[k] + v * hb[k] + w * fa[k];
+        if (i == k) t += gg;
+        if constexpr (PLASTIC) {
+          s.uu[3 * i + k] += t + ha[i] * xb[k];
+          s.vu[3 * i + k] += t + hb[k] * xa[i];
+        } else {
+          s.uu[3 * i + k] += t;
+        }
+      }
+    }
+  }
+  pin(s.uu);
+  stage_end();
+  constexpr double N = 0.25;
+  const double J = p[lJ], be = p[lBeta], t = p[lT];
+  const double pi[3] = {p[lPi], p[lPi + 1], p[lPi + 2]};
+  const double pa = pi[0] * fa[0] + pi[1] * fa[1] + pi[2] * fa[2];
+  const double pb = pi[0] * fb[0] + pi[1] * fb[1] + pi[2] * fb[2];
+  const double td = t * d, ta = t * pa, tb = t * pb, jn = J * N, al = be * N + ta, bl = be * N + tb;
+#pragma unroll
+  for (int i = 0; i < 3; ++i) {
+    s.ab_c[i] += jn * fa[i];
+    s.ba_c[i] += jn * fb[i];
+    const double tp = td * pi[i];
+    s.ab_r[i] += al * fb[i] - tb * fa[i] - tp;
+    s.ba_r[i] += bl * fa[i] - ta * fb[i] - tp;
+  }
+  s.pp += td + p[lKap] * (N * N);
+  if (diag) s.r[3] += p[lR1] * N + ta;
+}
+
+// Bound by memory and its latency: blocks stored once, states read about three
+// times (each element is in three runs; mostly from the L2 of the run's XCD),
+// 16 bytes of work list per lane.  On the 5.3 M-tet J2 bar 2.6 ms; with the
+// point pass 3.6 ms where the element matrices (2 KB a tet) through memory and
+// their gather took 9.6, and on 162 tets 34 against 41 us, so no size keeps the two passes.
+// Eight vertices a run: their states fill a quarter of a CU's LDS; sixteen
+// would read the states 2.5 instead of 2.9 times but leave two workgroups a CU.
+// Without plastic points 112 registers and four waves a SIMD, with them 168 and
+// three.
+constexpr int kLinearStride = kLinearPoint + 1;  // odd: the elements spread over the LDS banks
+
+template <bool PLASTIC, bool TR>
+__global__ __launch_bounds__(256, PLASTIC ? 3 : 4) void linear_cluster_kernel(LinearArgs a) {
+  __shared__ double pe[kLinearElems * kLinearStride];
+  __shared__ int64_t nbase[kLinearNodes];
+  __shared__ int32_t nid[kLinearNodes], nlen[kLinearNodes];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  for (int64_t it = 0;; ++it) {
+    const int64_t run = run_of(it, a.num_runs, a.xcd_remap);
+    if (run < 0) break;
+    const int4 r = a.runs[run];
+    const int2 sp = a.spans[run];
+    if (it > 0) lds_barrier();  // the last run's states are free
+    if (tid < r.y - r.x) {  // the run's nodes: CSR base and row length
+      const int32_t n = a.nodes[r.x + tid];
+      const int64_t b = a.row_ptr[4 * (int64_t)n];
+      nid[tid] = n;
+      nbase[tid] = b;
+      nlen[tid] = (int)(a.row_ptr[4 * (int64_t)n + 1] - b);
+    }
+    // 16 threads copy an element's state, 16 bytes each
+    for (int i = tid / 16; i < r.w; i += 256 / 16) {
+      const int k = tid & 15;
+      const double2 v = reinterpret_cast<const double2*>(a.pt + (int64_t)kLinearPoint * a.elems[r.z + i])[k];
+      pe[kLinearStride * i + 2 * k] = v.x;
+      pe[kLinearStride * i + 2 * k + 1] = v.y;
+    }
+    lds_barrier();
+    for (int g = sp.x + 64 * wave; g < sp.y; g += 256) {
+      const ClusterLane e = a.lanes[g + lane];
+      const int n = (int)(e.x >> kLaneCount) & 3, lg = (int)(e.x >> kLaneLog) & 7;
+      const bool diag = e.x & kLaneDiag;
+      LinearSum<PLASTIC> s;
+      s.all([](double& v) { v = 0.0; });
+      uint64_t code = e.x;
+#pragma unroll 1
+      for (int v = 0; v < n; ++v, code >>= 13)
+        linear_visit<PLASTIC>(pe + kLinearStride * (int)(code & 511), (int)(code >> 9) & 3, (int)(code >> 11) & 3, diag,
+                              s);
+      const int most = __builtin_amdgcn_readfirstlane(lg);  // the first lane's pair has the most lanes
+      if (most > 0) join<0>(lg, s);
+      if (most > 1) join<1>(lg, s);
+      if (most > 2) join<2>(lg, s);
+      if (most > 3) join<3>(lg, s);
+      if (most > 4) join<4>(lg, s);
+      if (most > 5) join<5>(lg, s);
+      const bool mine = n > 0 && !(lane & ((1 << lg) - 1));
+      const int nl = (int)(e.x >> kLaneNode) & 31;
+      BlockPlace ab = {0, nlen[nl], a.overwrite_vals}, ba = ab;
+      if (mine) ab.at = reinterpret_cast<uint64_t>(a.vals + nbase[nl] + 4 * ((int)(e.x >> kLanePos) & 511));
+      if (mine && !diag) {
+        ba.at = reinterpret_cast<uint64_t>(a.vals + 16 * (int64_t)(e.y & ((uint64_t(1) << kLaneDegT) - 1)) +
+                                           4 * (int64_t)(e.y >> kLanePosT));
+        ba.len = 4 * ((int)(e.y >> kLaneDegT) & 4095);
+      }
+      const double* vu = PLASTIC ? s.vu : s.uu;
+      put_block(ab, lane & 1, TR ? vu : s.uu, false, TR ? s.ba_r : s.ab_c, TR ? s.ba_c : s.ab_r, s.pp);
+      put_block(ba, lane & 1, TR ? s.uu : vu, true, TR ? s.ab_r : s.ba_c, TR ? s.ab_c : s.ba_r, s.pp);
+      if (mine && diag) {
+        double* o = a.R + 4 * (int64_t)nid[nl];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) o[i] = (a.overwrite_R ? 0.0 : o[i]) + s.r[i];
+      }
+    }
+  }
+}
+
 }  // namespace
 
 // scratch of the sort over n nodes and of scans over up to n + 1 entries
@@ -722,28 +1203,38 @@ hipError_t cluster_temp_bytes(int64_t nn, size_t* bytes) {
   return err;
 }
 
-hipError_t cluster_order(const int32_t* conn, const double* coords, int64_t ne, int64_t nn, void* temp,
-                         size_t temp_bytes, unsigned long long* box, int32_t* keys, int32_t* keys_sorted,
-                         int32_t* rank, int32_t* place, int32_t* nodes, int64_t* seg, hipStream_t s) {
+namespace {
+// nodes: the nodes along the Morton curve; place: its inverse.
+hipError_t morton_order(const double* coords, int64_t nn, void* temp, size_t temp_bytes, unsigned long long* box,
+                        uint32_t* code, uint32_t* code_sorted, int32_t* place, int32_t* iota, int32_t* nodes,
+                        hipStream_t s) {
   hipError_t err = hipMemsetAsync(box, 0xff, 3 * sizeof(*box), s);
   if (err == hipSuccess) err = hipMemsetAsync(box + 3, 0, 3 * sizeof(*box), s);
   if (err != hipSuccess) return err;
   hipLaunchKernelGGL(cluster_box_kernel, dim3(std::min(grid_for(nn), 1024u)), dim3(kBlock), 0, s, coords, nn, box);
-  uint32_t* code = reinterpret_cast<uint32_t*>(keys);
-  hipLaunchKernelGGL(cluster_morton_kernel, dim3(grid_for(nn)), dim3(kBlock), 0, s, coords, nn, box, code, place);
+  hipLaunchKernelGGL(cluster_morton_kernel, dim3(grid_for(nn)), dim3(kBlock), 0, s, coords, nn, box, code, iota);
   err = hipGetLastError();
   if (err != hipSuccess) return err;
   size_t tb = temp_bytes;
-  err = hipcub::DeviceRadixSort::SortPairs(temp, tb, code, reinterpret_cast<uint32_t*>(keys_sorted), place, nodes,
-                                           (int)nn, 0, 30, s);
+  err = hipcub::DeviceRadixSort::SortPairs(temp, tb, code, code_sorted, iota, nodes, (int)nn, 0, 30, s);
   if (err != hipSuccess) return err;
-  hipLaunchKernelGGL(cluster_place_kernel, dim3(grid_for(nn)), dim3(kBlock), 0, s, nodes, nn, rank);
+  hipLaunchKernelGGL(cluster_place_kernel, dim3(grid_for(nn)), dim3(kBlock), 0, s, nodes, nn, place);
+  return hipGetLastError();
+}
+}  // namespace
+
+hipError_t cluster_order(const int32_t* conn, const double* coords, int64_t ne, int64_t nn, void* temp,
+                         size_t temp_bytes, unsigned long long* box, int32_t* keys, int32_t* keys_sorted,
+                         int32_t* rank, int32_t* place, int32_t* nodes, int64_t* seg, hipStream_t s) {
+  hipError_t err = morton_order(coords, nn, temp, temp_bytes, box, reinterpret_cast<uint32_t*>(keys),
+                                reinterpret_cast<uint32_t*>(keys_sorted), rank, place, nodes, s);
+  if (err != hipSuccess) return err;
   for (int pass = 0; pass < 3; ++pass)
     hipLaunchKernelGGL(cluster_keys_kernel, dim3(grid_for(pass == 0 ? nn : 6 * ne)), dim3(kBlock), 0, s, conn, ne, nn,
                        pass, rank, keys, place);
   err = hipGetLastError();
   if (err != hipSuccess) return err;
-  tb = temp_bytes;
+  size_t tb = temp_bytes;
   err = hipcub::DeviceRadixSort::SortPairs(temp, tb, keys, keys_sorted, place, nodes, (int)nn, 0, 31, s);
   if (err != hipSuccess) return err;
   hipLaunchKernelGGL(cluster_segments_kernel, dim3(grid_for(nn + 1)), dim3(kBlock), 0, s, keys_sorted, nn, seg);
@@ -787,6 +1278,55 @@ hipError_t cluster_conn(int64_t num_chunks, const int4* chunk_tab, const uint32_
                         int32_t* chunk_conn, hipStream_t s) {
   hipLaunchKernelGGL(cluster_conn_kernel, dim3(grid_for(num_chunks * kClusterElems * 10)), dim3(kBlock), 0, s,
                      num_chunks, chunk_tab, elem_tab, conn, chunk_conn);
+  return hipGetLastError();
+}
+
+hipError_t linear_order(const double* coords, int64_t nn, void* temp, size_t temp_bytes, unsigned long long* box,
+                        uint32_t* code, uint32_t* code_sorted, int32_t* place, int32_t* nodes, hipStream_t s) {
+  // place holds the unsorted ids until the last kernel of the order writes it
+  return morton_order(coords, nn, temp, temp_bytes, box, code, code_sorted, place, place, nodes, s);
+}
+
+hipError_t linear_split(const ClusterMesh& m, int64_t nn, void* temp, size_t temp_bytes, int32_t* parts, int32_t* bad,
+                        hipStream_t s) {
+  const int64_t groups = (nn + kLinearNodes - 1) / kLinearNodes;
+  hipLaunchKernelGGL(linear_split_kernel, dim3((unsigned)groups), dim3(kBlock), 0, s, m, nn, parts, bad);
+  hipError_t err = hipGetLastError();
+  if (err != hipSuccess) return err;
+  return hipcub::DeviceScan::ExclusiveSum(temp, temp_bytes, parts, parts, (int)(groups + 1), s);
+}
+
+hipError_t linear_tables(const ClusterMesh& m, int64_t nn, int64_t num_runs, const int32_t* parts, void* temp,
+                         size_t temp_bytes, int32_t* nlanes, int32_t* nelems, int4* runs, int2* spans, int32_t* elems,
+                         ClusterLane* lanes, hipStream_t s) {
+  const int64_t groups = (nn + kLinearNodes - 1) / kLinearNodes;
+  hipLaunchKernelGGL(linear_tables_kernel, dim3((unsigned)groups), dim3(kBlock), 0, s, m, nn, parts, nlanes, nelems,
+                     runs, spans, elems, lanes);
+  hipError_t err = hipGetLastError();
+  if (err != hipSuccess || lanes) return err;
+  size_t tb = temp_bytes;
+  err = hipcub::DeviceScan::ExclusiveSum(temp, tb, nlanes, nlanes, (int)(num_runs + 1), s);
+  if (err != hipSuccess) return err;
+  tb = temp_bytes;
+  return hipcub::DeviceScan::ExclusiveSum(temp, tb, nelems, nelems, (int)(num_runs + 1), s);
+}
+
+hipError_t launch_linear_points(const AsmArgs& a, hipStream_t s) {
+  if (a.num_elems == 0) return hipSuccess;
+  const dim3 grid((unsigned)((a.num_elems + 255) / 256));
+  if (a.model == MODEL_J2) hipLaunchKernelGGL(linear_points_kernel<MODEL_J2>, grid, dim3(256), 0, s, a);
+  else hipLaunchKernelGGL(linear_points_kernel<MODEL_NEOHOOKEAN>, grid, dim3(256), 0, s, a);
+  return hipGetLastError();
+}
+
+hipError_t launch_linear_cluster(bool transpose, bool plastic, const LinearArgs& a, int blocks, hipStream_t s) {
+  if (a.num_runs == 0) return hipSuccess;
+  if (blocks <= 0) blocks = (int)std::min<int64_t>((a.num_runs + 7) / 8 * 8, int64_t(1) << 30);  // as launch_cluster
+  const dim3 grid(blocks), block(256);
+  if (plastic && transpose) hipLaunchKernelGGL((linear_cluster_kernel<true, true>), grid, block, 0, s, a);
+  else if (plastic) hipLaunchKernelGGL((linear_cluster_kernel<true, false>), grid, block, 0, s, a);
+  else if (transpose) hipLaunchKernelGGL((linear_cluster_kernel<false, true>), grid, block, 0, s, a);
+  else hipLaunchKernelGGL((linear_cluster_kernel<false, false>), grid, block, 0, s, a);
   return hipGetLastError();
 }
 

@@ -14,7 +14,7 @@
 // every element that holds b beside a is among a's: the run of the node that
 // comes first in the order forms both.  Within a chunk the unit of work is a
 // visit: what one element adds to one such pair.  A pair's visits go to 1, 2,
-// 4, 8 or 16 lanes, the fewest with at most three visits each; each lane sums
+// 4, .. 64 lanes, the fewest with at most three visits each; each lane sums
 // its visits in registers and the pair's lanes then add theirs.  Pairs are
 // ordered by lanes, then visits, so a wavefront's lanes have equal work.
 #pragma once
@@ -151,9 +151,12 @@ struct ClusterFill {
 };
 
 // Lanes (as a power of two) of a pair with n visits.
-__host__ __device__ inline int cluster_log_lanes(int n) { return n <= 3 ? 0 : n <= 6 ? 1 : n <= 12 ? 2 : n <= 24 ? 3 : 4; }
+__host__ __device__ inline int cluster_log_lanes(int n) {
+  return n <= 3 ? 0 : n <= 6 ? 1 : n <= 12 ? 2 : n <= 24 ? 3 : n <= 48 ? 4 : n <= 96 ? 5 : 6;
+}
 // Order of the pairs of a chunk: lower first.
-__host__ __device__ inline int cluster_rank(int n) { return n == 0 ? 9 : n > 3 ? 4 - cluster_log_lanes(n) : 7 - n; }
+__host__ __device__ inline int cluster_rank(int n) { return n == 0 ? 9 : n > 3 ? 6 - cluster_log_lanes(n) : 9 - n; }
+__host__ __device__ inline int cluster_lanes_of_rank(int rank) { return rank < 6 ? 64 >> rank : 1; }
 
 // A lane's work.  x: three visits of 13 bits each (element slot 5, local node
 // of a 4, of b 4), their number (2 bits), b's position in a's adjacency (9
@@ -172,9 +175,36 @@ struct alignas(16) ClusterLane {
   uint64_t x, y;
 };
 
+// Linear tets with one point (neo-Hookean, J2) go the same way, in two kernels:
+// the point states are formed once, 32 doubles an element, and copied to LDS by
+// the runs that need them.  Their runs are up to eight vertices that follow
+// each other on the Morton curve (in a regular mesh of six tets per cell a
+// 2 x 2 x 2 brick: 192 incidences of 120 elements; where the curve and the mesh do
+// not line up, up to 156).  A visit's 13 bits are
+// element slot 9, local a 2, local b 2.
+constexpr int kLinearElems = 160;   // elements per run
+constexpr int kLinearNodes = 8;     // vertices per run
+constexpr int kLinearRecs = 1024;   // incidences per run
+constexpr int kLinearPoint = 32;    // doubles per element
+static_assert(kLinearElems <= 3 * 64 && kLinearElems < 512 && kLinearNodes <= kClusterNodes, "the fields of a lane's work");
+struct LinearArgs {
+  int64_t num_runs, num_elems;
+  const int4* runs;         // node_lo, node_hi, first element of the list, elements
+  const int2* spans;        // first and last lane
+  const int32_t* elems;
+  const ClusterLane* lanes;
+  const int32_t* nodes;
+  const int64_t* row_ptr;
+  const double* pt;         // [elements][kLinearPoint]
+  double* R;
+  double* vals;
+  int overwrite_R, overwrite_vals, xcd_remap;
+};
+
 // One neo-Hookean assembly of a quadratic mesh with four points (ASM_JACOBIAN
 // or, transposed, ASM_ADJOINT), FP64.
 struct MatParams;
+struct AsmArgs;
 struct ClusterArgs {
   int64_t num_runs, num_elems;
   const int4* runs;
@@ -215,6 +245,21 @@ hipError_t cluster_lanes(const ClusterMesh& m, int64_t num_runs, int64_t num_chu
                          int32_t* nlanes, void* temp, size_t temp_bytes, ClusterLane* lanes, hipStream_t s);
 hipError_t cluster_conn(int64_t num_chunks, const int4* chunk_tab, const uint32_t* elem_tab, const int32_t* conn,
                         int32_t* chunk_conn, hipStream_t s);
+// linear_split: runs per group of kLinearNodes ordered nodes into parts
+// [groups + 1] (then scanned), or a number above kLinearNodes into *bad when a
+// node's incidences do not fit a run.  linear_tables: with lanes null the
+// lanes (whole wavefronts) and elements of every run into nlanes, nelems
+// [runs + 1] (then scanned); else the tables.
+hipError_t linear_order(const double* coords, int64_t nn, void* temp, size_t temp_bytes, unsigned long long* box,
+                        uint32_t* code, uint32_t* code_sorted, int32_t* place, int32_t* nodes, hipStream_t s);
+hipError_t linear_split(const ClusterMesh& m, int64_t nn, void* temp, size_t temp_bytes, int32_t* parts, int32_t* bad,
+                        hipStream_t s);
+hipError_t linear_tables(const ClusterMesh& m, int64_t nn, int64_t num_runs, const int32_t* parts, void* temp,
+                         size_t temp_bytes, int32_t* nlanes, int32_t* nelems, int4* runs, int2* spans, int32_t* elems,
+                         ClusterLane* lanes, hipStream_t s);
+// Point states of every element (model neo-Hookean or J2; states saved as asked) into a.pt.
+hipError_t launch_linear_points(const AsmArgs& a, hipStream_t s);
+hipError_t launch_linear_cluster(bool transpose, bool plastic, const LinearArgs& a, int blocks, hipStream_t s);
 hipError_t launch_cluster(bool transpose, const ClusterArgs& a, int blocks, hipStream_t s);
 
 }  // namespace goal
