@@ -903,131 +903,156 @@ __global__ __launch_bounds__(kBlock) void linear_tables_kernel(ClusterMesh m, in
 //   kappa_k = A (2 mu nu (ee_b + t3 ed_b) - 2/3 |s_tr| f_b)_k + B (2 mu / 3) ed_bk,
 //   A = 2 mubar (dgam / |s_tr| - alpha),  B = -2 (dgam + mubar beta),
 // so K(ai, bk) += ed_ai (q1 ee_b + q2 ed_b + q3 f_b)_k.  All times w dv.
-enum : int { lF = 0, lDev = 12, lC = 18, lCT, lPJ, lJ, lBeta, lT, lPi, lKap = lPi + 3, lR1, lQ1, lQ2, lQ3, lPt };
-static_assert(lPt == kLinearPoint, "32 doubles an element");
+// dev is traceless: its last entry is not kept.
+enum : int { lF = 0, lDev = 12, lC = 17, lCT, lPJ, lJ, lBeta, lT, lPi, lKap = lPi + 3, lR1, lQ1, lQ2, lQ3, lPt };
+static_assert(lPt == kLinearPoint - 1, "31 of 32 doubles an element");
 
-// Bound by its memory traffic (256 bytes written an element; 1.0 ms on the 5.3 M-tet J2 bar).
+// Bound by its memory traffic (J2: some 520 bytes an element, 256 of them the
+// state; 0.85 ms = 3.2 TB/s on the 5.3 M-tet bar, two waves a SIMD of 204
+// registers; held to 168 for three waves it took 0.91).
 template <int MODEL>
 __global__ __launch_bounds__(256) void linear_points_kernel(AsmArgs a) {
+  __shared__ double stage[4][64 * 17];
   const int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x, ne = a.num_elems;
-  if (e >= ne) return;
-  const int4 ec4 = reinterpret_cast<const int4*>(a.conn)[e];
-  const int32_t ec[4] = {ec4.x, ec4.y, ec4.z, ec4.w};
-  const MatParams mp = a.mats[a.elem_set ? a.elem_set[e] : 0];
-  double D[3][4], p = 0.0;
-  {
-    double U[4][4];
-#pragma unroll
-    for (int v = 0; v < 4; ++v)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) U[v][i] = a.x[4 * (int64_t)ec[v] + i];
-    p = 0.25 * ((U[0][3] + U[1][3]) + (U[2][3] + U[3][3]));
-#pragma unroll
-    for (int v = 1; v < 4; ++v)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) D[v - 1][i] = U[v][i] - U[0][i];
-  }
-  double gl[4][3], W, tau;
-  {
-    double X[4][3];
-#pragma unroll
-    for (int v = 0; v < 4; ++v)
-#pragma unroll
-      for (int c = 0; c < 3; ++c) X[v][c] = a.coords[3 * (int64_t)ec[v] + c];
-    W = dev::tet_gradlambda(X, gl) / 6.0;
-    tau = a.stabilization ? dev::stab_tau(X, mp) : 0.0;
-  }
-  dev::QP qp;
-#pragma unroll
-  for (int j = 0; j < 3; ++j) {
-#pragma unroll
-    for (int i = 0; i < 3; ++i) {
-      qp.H[3 * i + j] = D[0][i] * gl[1][j] + D[1][i] * gl[2][j] + D[2][i] * gl[3][j];
-      qp.F[3 * i + j] = qp.H[3 * i + j] + (i == j ? 1.0 : 0.0);
-    }
-    qp.g[j] = D[0][3] * gl[1][j] + D[1][3] * gl[2][j] + D[2][3] * gl[3][j];
-  }
-  qp.p = p;
-  qp.J = dev::det3(qp.F);
-  dev::inv3(qp.F, qp.J, qp.Fi);
-  const double J = qp.J, iJ = 1.0 / J;
   double o[kLinearPoint];
-  if constexpr (MODEL == MODEL_NEOHOOKEAN) {
-    double b[6];
+  o[kLinearPoint - 1] = 0.0;
+  if (e < ne) {
+    const int4 ec4 = reinterpret_cast<const int4*>(a.conn)[e];
+    const int32_t ec[4] = {ec4.x, ec4.y, ec4.z, ec4.w};
+    const MatParams mp = a.mats[a.elem_set ? a.elem_set[e] : 0];
+    double D[3][4], p = 0.0;
+    {
+      double U[4][4];
 #pragma unroll
-    for (int i = 0; i < 3; ++i)
+      for (int v = 0; v < 4; ++v)
 #pragma unroll
-      for (int j = i; j < 3; ++j)
-        b[sym(i, j)] = qp.F[3 * i] * qp.F[3 * j] + qp.F[3 * i + 1] * qp.F[3 * j + 1] + qp.F[3 * i + 2] * qp.F[3 * j + 2];
-    const double third = (b[0] + b[3] + b[5]) / 3.0;
-    b[0] -= third;
-    b[3] -= third;
-    b[5] -= third;
-    const double Jm13 = 1.0 / cbrt(J), Jm23 = Jm13 * Jm13;
-    if (a.save_state) {
-      const double m = mp.mu * (Jm23 * Jm23 * Jm13);
+        for (int i = 0; i < 4; ++i) U[v][i] = a.x[4 * (int64_t)ec[v] + i];
+      p = 0.25 * ((U[0][3] + U[1][3]) + (U[2][3] + U[3][3]));
 #pragma unroll
-      for (int k = 0; k < 9; ++k) a.sigma[k * ne + e] = m * b[sym(k / 3, k % 3)] + (k % 4 == 0 ? p : 0.0);
+      for (int v = 1; v < 4; ++v)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) D[v - 1][i] = U[v][i] - U[0][i];
     }
+    double gl[4][3], W, tau;
+    {
+      double X[4][3];
 #pragma unroll
-    for (int k = 0; k < 6; ++k) o[lDev + k] = b[k];
-    o[lC] = W * (mp.mu * Jm23);
-    o[lCT] = o[lC] * third;
-    o[lQ1] = o[lQ2] = o[lQ3] = 0.0;
-  } else {
-    double Fpo[9];
-    for (int k = 0; k < 9; ++k) Fpo[k] = a.Fp_old[k * ne + e];
-    dev::J2Model m;
-    m.init(qp, mp, Fpo, a.eqps_old[e]);
-    if (m.failed()) atomicOr(a.status, 1);
-    if (a.save_state) {
-      a.eqps[e] = m.alpha;
-      if (m.plastic) {
-        double Fpn[9];
-        m.new_Fp(Fpo, Fpn);
-        for (int k = 0; k < 9; ++k) a.Fp[k * ne + e] = Fpn[k];
+      for (int v = 0; v < 4; ++v)
+#pragma unroll
+        for (int c = 0; c < 3; ++c) X[v][c] = a.coords[3 * (int64_t)ec[v] + c];
+      W = dev::tet_gradlambda(X, gl) / 6.0;
+      tau = a.stabilization ? dev::stab_tau(X, mp) : 0.0;
+    }
+    dev::QP qp;
+#pragma unroll
+    for (int j = 0; j < 3; ++j) {
+#pragma unroll
+      for (int i = 0; i < 3; ++i) {
+        qp.H[3 * i + j] = D[0][i] * gl[1][j] + D[1][i] * gl[2][j] + D[2][i] * gl[3][j];
+        qp.F[3 * i + j] = qp.H[3 * i + j] + (i == j ? 1.0 : 0.0);
       }
-      for (int k = 0; k < 9; ++k) a.sigma[k * ne + e] = m.sig[k];
+      qp.g[j] = D[0][3] * gl[1][j] + D[1][3] * gl[2][j] + D[2][3] * gl[3][j];
     }
-    const double mu = mp.mu, t3 = m.mubar / mu;
+    qp.p = p;
+    qp.J = dev::det3(qp.F);
+    dev::inv3(qp.F, qp.J, qp.Fi);
+    const double J = qp.J, iJ = 1.0 / J;
+    if constexpr (MODEL == MODEL_NEOHOOKEAN) {
+      double b[6];
 #pragma unroll
-    for (int i = 0; i < 3; ++i)
+      for (int i = 0; i < 3; ++i)
 #pragma unroll
-      for (int j = i; j < 3; ++j) o[lDev + sym(i, j)] = m.str[3 * i + j] / mu;
-    double theta = 1.0, q1 = 0.0, q2 = 0.0, q3 = 0.0;
-    if (m.plastic) {
-      double X, al, bt;
-      (void)m.newton(1.0, 0.0, X, al);
-      (void)m.newton(0.0, 1.0, X, bt);
-      theta = 1.0 - 2.0 * m.mubar * m.dgam / m.smag;
-      const double A = 2.0 * m.mubar * (m.dgam / m.smag - al), B = -2.0 * (m.dgam + m.mubar * bt);
-      const double nu = mu / m.smag;
-      q1 = W * nu * (2.0 * mu * A * nu);
-      q2 = W * nu * (2.0 * mu * A * nu * t3 + (2.0 * mu / 3.0) * B);
-      q3 = (-2.0 / 3.0) * W * A * mu;
+        for (int j = i; j < 3; ++j)
+          b[sym(i, j)] = qp.F[3 * i] * qp.F[3 * j] + qp.F[3 * i + 1] * qp.F[3 * j + 1] + qp.F[3 * i + 2] * qp.F[3 * j + 2];
+      const double third = (b[0] + b[3] + b[5]) / 3.0;
+      b[0] -= third;
+      b[3] -= third;
+      b[5] -= third;
+      const double Jm13 = 1.0 / cbrt(J), Jm23 = Jm13 * Jm13;
+      if (a.save_state) {
+        const double m = mp.mu * (Jm23 * Jm23 * Jm13);
+#pragma unroll
+        for (int k = 0; k < 9; ++k) a.sigma[k * ne + e] = m * b[sym(k / 3, k % 3)] + (k % 4 == 0 ? p : 0.0);
+      }
+#pragma unroll
+      for (int k = 0; k < 5; ++k) o[lDev + k] = b[k];
+      o[lC] = W * (mp.mu * Jm23);
+      o[lCT] = o[lC] * third;
+      o[lQ1] = o[lQ2] = o[lQ3] = 0.0;
+    } else {
+      double Fpo[9];
+      for (int k = 0; k < 9; ++k) Fpo[k] = a.Fp_old[k * ne + e];
+      dev::J2Model m;
+      m.init(qp, mp, Fpo, a.eqps_old[e]);
+      if (m.failed()) atomicOr(a.status, 1);
+      if (a.save_state) {
+        a.eqps[e] = m.alpha;
+        if (m.plastic) {
+          double Fpn[9];
+          m.new_Fp(Fpo, Fpn);
+          for (int k = 0; k < 9; ++k) a.Fp[k * ne + e] = Fpn[k];
+        }
+        for (int k = 0; k < 9; ++k) a.sigma[k * ne + e] = m.sig[k];
+      }
+      const double mu = mp.mu, t3 = m.mubar / mu;
+#pragma unroll
+      for (int i = 0; i < 3; ++i)
+#pragma unroll
+        for (int j = i; j < 3; ++j)
+          if (i < 2) o[lDev + sym(i, j)] = m.str[3 * i + j] / mu;
+      double theta = 1.0, q1 = 0.0, q2 = 0.0, q3 = 0.0;
+      if (m.plastic) {
+        double X, al, bt;
+        (void)m.newton(1.0, 0.0, X, al);
+        (void)m.newton(0.0, 1.0, X, bt);
+        theta = 1.0 - 2.0 * m.mubar * m.dgam / m.smag;
+        const double A = 2.0 * m.mubar * (m.dgam / m.smag - al), B = -2.0 * (m.dgam + m.mubar * bt);
+        const double nu = mu / m.smag;
+        q1 = W * nu * (2.0 * mu * A * nu);
+        q2 = W * nu * (2.0 * mu * A * nu * t3 + (2.0 * mu / 3.0) * B);
+        q3 = (-2.0 / 3.0) * W * A * mu;
+      }
+      o[lC] = W * (theta * mu);
+      o[lCT] = o[lC] * t3;
+      o[lQ1] = q1;
+      o[lQ2] = q2;
+      o[lQ3] = q3;
     }
-    o[lC] = W * (theta * mu);
-    o[lCT] = o[lC] * t3;
-    o[lQ1] = q1;
-    o[lQ2] = q2;
-    o[lQ3] = q3;
+#pragma unroll
+    for (int v = 0; v < 4; ++v)
+#pragma unroll
+      for (int k = 0; k < 3; ++k)
+        o[lF + 3 * v + k] = qp.Fi[k] * gl[v][0] + qp.Fi[3 + k] * gl[v][1] + qp.Fi[6 + k] * gl[v][2];
+#pragma unroll
+    for (int k = 0; k < 3; ++k) o[lPi + k] = qp.Fi[k] * qp.g[0] + qp.Fi[3 + k] * qp.g[1] + qp.Fi[6 + k] * qp.g[2];
+    o[lPJ] = W * (p * J);
+    o[lJ] = W * J;
+    o[lBeta] = W * (-0.5 * (J + iJ));
+    o[lT] = W * J * tau;
+    o[lKap] = W / mp.kappa;
+    o[lR1] = W * (p / mp.kappa - 0.5 * (J - iJ));
   }
+  // Out through LDS, 16 values a round: eight lanes then store an element's
+  // 128 bytes together, where a lane's own 16-byte stores lie 256 bytes apart
+  // (5.3 M-tet J2 bar: 0.98 -> 0.85 ms).
+  const int lane = threadIdx.x & 63;
+  double* w = stage[threadIdx.x >> 6];
+  const int64_t e0 = e - lane;
 #pragma unroll
-  for (int v = 0; v < 4; ++v)
+  for (int h = 0; h < 2; ++h) {
+    __builtin_amdgcn_wave_barrier();
 #pragma unroll
-    for (int k = 0; k < 3; ++k)
-      o[lF + 3 * v + k] = qp.Fi[k] * gl[v][0] + qp.Fi[3 + k] * gl[v][1] + qp.Fi[6 + k] * gl[v][2];
+    for (int k = 0; k < 16; ++k) w[17 * lane + k] = o[16 * h + k];
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 #pragma unroll
-  for (int k = 0; k < 3; ++k) o[lPi + k] = qp.Fi[k] * qp.g[0] + qp.Fi[3 + k] * qp.g[1] + qp.Fi[6 + k] * qp.g[2];
-  o[lPJ] = W * (p * J);
-  o[lJ] = W * J;
-  o[lBeta] = W * (-0.5 * (J + iJ));
-  o[lT] = W * J * tau;
-  o[lKap] = W / mp.kappa;
-  o[lR1] = W * (p / mp.kappa - 0.5 * (J - iJ));
-  double2* out = reinterpret_cast<double2*>(a.pt + kLinearPoint * e);
-#pragma unroll
-  for (int k = 0; k < kLinearPoint / 2; ++k) out[k] = double2{o[2 * k], o[2 * k + 1]};
+    for (int j = 0; j < 8; ++j) {
+      const int i = 8 * j + (lane >> 3), k = 2 * (lane & 7);
+      if (e0 + i < ne)
+        *reinterpret_cast<double2*>(a.pt + kLinearPoint * (e0 + i) + 16 * h + k) = double2{w[17 * i + k], w[17 * i + k + 1]};
+    }
+  }
 }
 
 // A pair's sums for linear tets: with plastic points K(ai, bk) and K(bk, ai) differ (vu[3 i + k] = K(bk, ai)).
@@ -1052,7 +1077,8 @@ __device__ __forceinline__ void linear_visit(const double* p, int la, int lb, bo
     fb[k] = p[lF + 3 * lb + k];
   }
 #pragma unroll
-  for (int k = 0; k < 6; ++k) dv[k] = p[lDev + k];
+  for (int k = 0; k < 5; ++k) dv[k] = p[lDev + k];
+  dv[5] = -(dv[0] + dv[3]);
 #pragma unroll
   for (int j = 0; j < 3; ++j) {
     ha[j] = dv[sym(j, 0)] * fa[0] + dv[sym(j, 1)] * fa[1] + dv[sym(j, 2)] * fa[2];
@@ -1067,15 +1093,6 @@ __device__ __forceinline__ void linear_visit(const double* p, int la, int lb, bo
 #pragma unroll
       for (int i = 0; i < 3; ++i) s.r[i] += C * ha[i] + PJ * fa[i];
     }
-    double xa[3], xb[3];  // q1 ee + q2 ed + q3 f
-    if constexpr (PLASTIC) {
-      const double q1 = p[lQ1], q2 = p[lQ2], q3 = p[lQ3];
-#pragma unroll
-      for (int j = 0; j < 3; ++j) {
-        xa[j] = q1 * (dv[sym(j, 0)] * ha[0] + dv[sym(j, 1)] * ha[1] + dv[sym(j, 2)] * ha[2]) + q2 * ha[j] + q3 * fa[j];
-        xb[j] = q1 * (dv[sym(j, 0)] * hb[0] + dv[sym(j, 1)] * hb[1] + dv[sym(j, 2)] * hb[2]) + q2 * hb[j] + q3 * fb[j];
-      }
-    }
 #pragma unroll
     for (int i = 0; i < 3; ++i) {
       const double u = m * ha[i] + A * fa[i], v = m * fa[i], w = S * fb[i];
@@ -1083,17 +1100,31 @@ __device__ __forceinline__ void linear_visit(const double* p, int la, int lb, bo
       for (int k = 0; k < 3; ++k) {
         double t = u * fb[k] + v * hb[k] + w * fa[k];
         if (i == k) t += gg;
-        if constexpr (PLASTIC) {
-          s.uu[3 * i + k] += t + ha[i] * xb[k];
-          s.vu[3 * i + k] += t + hb[k] * xa[i];
-        } else {
-          s.uu[3 * i + k] += t;
-        }
+        s.uu[3 * i + k] += t;
+        if constexpr (PLASTIC) s.vu[3 * i + k] += t;
       }
     }
   }
   pin(s.uu);
   stage_end();
+  if constexpr (PLASTIC) {
+    const double q1 = p[lQ1], q2 = p[lQ2], q3 = p[lQ3];
+    auto extra = [&](const double* h, const double* f, int j) {  // q1 ee + q2 ed + q3 f
+      return q1 * (dv[sym(j, 0)] * h[0] + dv[sym(j, 1)] * h[1] + dv[sym(j, 2)] * h[2]) + q2 * h[j] + q3 * f[j];
+    };
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+      const double xa = extra(ha, fa, k), xb = extra(hb, fb, k);
+#pragma unroll
+      for (int i = 0; i < 3; ++i) {
+        s.uu[3 * i + k] += ha[i] * xb;
+        s.vu[3 * k + i] += hb[i] * xa;
+      }
+    }
+    pin(s.uu);
+    pin(s.vu);
+    stage_end();
+  }
   constexpr double N = 0.25;
   const double J = p[lJ], be = p[lBeta], t = p[lT];
   const double pi[3] = {p[lPi], p[lPi + 1], p[lPi + 2]};
@@ -1112,19 +1143,21 @@ __device__ __forceinline__ void linear_visit(const double* p, int la, int lb, bo
   if (diag) s.r[3] += p[lR1] * N + ta;
 }
 
-// Bound by memory and its latency: blocks stored once, states read about three
-// times (each element is in three runs; mostly from the L2 of the run's XCD),
-// 16 bytes of work list per lane.  On the 5.3 M-tet J2 bar 2.6 ms; with the
-// point pass 3.6 ms where the element matrices (2 KB a tet) through memory and
-// their gather took 9.6, and on 162 tets 34 against 41 us, so no size keeps the two passes.
-// Eight vertices a run: their states fill a quarter of a CU's LDS; sixteen
-// would read the states 2.5 instead of 2.9 times but leave two workgroups a CU.
-// Without plastic points 112 registers and four waves a SIMD, with them 168 and
-// three.
-constexpr int kLinearStride = kLinearPoint + 1;  // odd: the elements spread over the LDS banks
+// Bound by latency and the occupancy that hides it (blocks stored once, 1.75 GB
+// on the 5.3 M-tet J2 bar; states read about three times, each element being in
+// three runs; 16 bytes of work list per lane).  There it takes 1.57 ms, and with
+// the point pass 2.4 ms, where the element matrices (2 KB a tet) through memory
+// and their gather took 9.6; on 162 tets 34 against 41 us, so no size keeps the
+// two passes.  Eight vertices a run: about 176 lanes, three waves; sixteen would
+// read the states 2.5 instead of 2.9 times but leave two workgroups a CU.  The
+// states come in with seven loads in flight a thread (one: 2.6 ms; fourteen
+// spill: 3.7), and plastic visits in stages that keep to 168 registers (with
+// two waves a SIMD instead 2.2 ms; unstaged, spilling, 4.7).
+constexpr int kLinearStride = lPt;  // odd: the elements spread over the LDS banks
+constexpr int kLinearThreads = 192;
 
 template <bool PLASTIC, bool TR>
-__global__ __launch_bounds__(256, PLASTIC ? 3 : 4) void linear_cluster_kernel(LinearArgs a) {
+__global__ __launch_bounds__(kLinearThreads, PLASTIC ? 3 : 4) void linear_cluster_kernel(LinearArgs a) {
   __shared__ double pe[kLinearElems * kLinearStride];
   __shared__ int64_t nbase[kLinearNodes];
   __shared__ int32_t nid[kLinearNodes], nlen[kLinearNodes];
@@ -1143,16 +1176,35 @@ __global__ __launch_bounds__(256, PLASTIC ? 3 : 4) void linear_cluster_kernel(Li
       nbase[tid] = b;
       nlen[tid] = (int)(a.row_ptr[4 * (int64_t)n + 1] - b);
     }
-    // 16 threads copy an element's state, 16 bytes each
-    for (int i = tid / 16; i < r.w; i += 256 / 16) {
-      const int k = tid & 15;
-      const double2 v = reinterpret_cast<const double2*>(a.pt + (int64_t)kLinearPoint * a.elems[r.z + i])[k];
-      pe[kLinearStride * i + 2 * k] = v.x;
-      pe[kLinearStride * i + 2 * k + 1] = v.y;
+    int g = sp.x + 64 * wave;
+    ClusterLane e = {0, 0};  // a wave's first lane work is loaded with the states
+    if (g < sp.y) e = a.lanes[g + lane];
+    // 16 threads copy an element's state, 16 bytes each; seven loads in flight
+    constexpr int kStep = kLinearThreads / 16, kBatch = 7;
+    static_assert(kLinearElems <= 2 * kStep * kBatch, "two batches hold a run");
+    int q = tid;
+    asm volatile("" : "+v"(q));  // or fourteen addresses are kept over the runs, and spill
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const int i0 = q / 16 + h * kStep * kBatch, k = q & 15;
+      int32_t id[kBatch];
+      double2 v[kBatch];
+#pragma unroll
+      for (int j = 0; j < kBatch; ++j) id[j] = i0 + kStep * j < r.w ? a.elems[r.z + i0 + kStep * j] : -1;
+#pragma unroll
+      for (int j = 0; j < kBatch; ++j)
+        if (id[j] >= 0) v[j] = reinterpret_cast<const double2*>(a.pt + (int64_t)kLinearPoint * id[j])[k];
+#pragma unroll
+      for (int j = 0; j < kBatch; ++j)
+        if (id[j] >= 0) {
+          double* o = pe + kLinearStride * (i0 + kStep * j) + 2 * k;
+          o[0] = v[j].x;
+          if (k < 15) o[1] = v[j].y;
+        }
     }
     lds_barrier();
-    for (int g = sp.x + 64 * wave; g < sp.y; g += 256) {
-      const ClusterLane e = a.lanes[g + lane];
+    for (; g < sp.y; g += kLinearThreads) {
+      if (g >= sp.x + kLinearThreads) e = a.lanes[g + lane];
       const int n = (int)(e.x >> kLaneCount) & 3, lg = (int)(e.x >> kLaneLog) & 7;
       const bool diag = e.x & kLaneDiag;
       LinearSum<PLASTIC> s;
@@ -1322,7 +1374,7 @@ hipError_t launch_linear_points(const AsmArgs& a, hipStream_t s) {
 hipError_t launch_linear_cluster(bool transpose, bool plastic, const LinearArgs& a, int blocks, hipStream_t s) {
   if (a.num_runs == 0) return hipSuccess;
   if (blocks <= 0) blocks = (int)std::min<int64_t>((a.num_runs + 7) / 8 * 8, int64_t(1) << 30);  // as launch_cluster
-  const dim3 grid(blocks), block(256);
+  const dim3 grid(blocks), block(kLinearThreads);
   if (plastic && transpose) hipLaunchKernelGGL((linear_cluster_kernel<true, true>), grid, block, 0, s, a);
   else if (plastic) hipLaunchKernelGGL((linear_cluster_kernel<true, false>), grid, block, 0, s, a);
   else if (transpose) hipLaunchKernelGGL((linear_cluster_kernel<false, true>), grid, block, 0, s, a);
