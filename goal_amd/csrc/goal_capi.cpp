@@ -2446,10 +2446,14 @@ int goal_asm_qoi(goal_mech m, goal_solinfo s, int kind, int elem_set, double* va
     q.kind = kind;
     q.qoi_set = elem_set;
     q.elem_value = m->elem_value.p;
-    if (s) materialize(s);
-    q.dMdu = s ? s->dMdu.p : nullptr;
+    q.rec = d->rec.p;
+    q.emr = s ? element_residuals(m) : nullptr;
     q.status = m->status.p;
     HIPCHK(goal::launch_qoi(d->mesh.order, m->quad_order, q, stream()));
+    if (s) {
+      HIPCHK(goal::launch_node_sum(d->mesh.num_nodes, d->inc_ptr.p, q.emr, s->zero_dMdu ? 1 : 0, s->dMdu.p, stream()));
+      s->zero_dMdu = false;
+    }
     HIPCHK(goal::launch_reduce(0, m->elem_value.p, nullptr, d->mesh.num_elems, reduce_scratch(), result_slot(1), stream()));
     HIPCHK(hipMemcpyAsync(value, result_slot(1), sizeof(double), hipMemcpyDeviceToHost, stream()));
     sync();
@@ -2480,7 +2484,7 @@ int goal_learn_features(goal_mech m, double qoi_x, float* feat_dev) {
     q.kind = GOAL_QOI_AVG_VM;
     q.qoi_set = -1;
     q.elem_value = m->elem_value.p;
-    q.dMdu = nullptr;
+    q.emr = nullptr;
     q.status = m->status.p;
     HIPCHK(goal::launch_qoi(d->mesh.order, m->quad_order, q, stream()));
     require(d->mesh.num_elems > 0, "goal_learn_features: empty mesh");

@@ -118,7 +118,8 @@ struct QoiArgs {
   int kind;
   int qoi_set;              // element set integrated over (AvgVM), -1: all
   double* elem_value;       // [ne] per-element QoI contribution
-  double* dMdu;             // [num_dofs] or null: derivative scatter
+  const int32_t* rec;       // as AsmArgs
+  double* emr;              // [records][4] or null: the derivative, to be summed by node
   int* status;
 };
 
