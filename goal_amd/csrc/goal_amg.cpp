@@ -82,6 +82,9 @@ AmgCoarsening amg_coarsen(int64_t nf, const int64_t* fptr, const int32_t* fcol) 
 bool dense_inverse(int n, std::vector<double>& a) {
   std::vector<double> inv((size_t)n * n, 0.0);
   for (int i = 0; i < n; ++i) inv[(size_t)i * n + i] = 1.0;
+  // Row c is zero left of column c, and the rows of inv used so far right of
+  // column `used`, so the updates leave those columns out.
+  int used = 0;
   for (int c = 0; c < n; ++c) {
     int p = c;
     for (int r = c + 1; r < n; ++r)
@@ -96,19 +99,18 @@ bool dense_inverse(int n, std::vector<double>& a) {
         std::swap(a[(size_t)c * n + j], a[(size_t)p * n + j]);
         std::swap(inv[(size_t)c * n + j], inv[(size_t)p * n + j]);
       }
+    used = std::max(used, p + 1);
     const double d = 1.0 / a[(size_t)c * n + c];
-    for (int j = 0; j < n; ++j) {
-      a[(size_t)c * n + j] *= d;
-      inv[(size_t)c * n + j] *= d;
-    }
+    for (int j = c; j < n; ++j) a[(size_t)c * n + j] *= d;
+    for (int j = 0; j < used; ++j) inv[(size_t)c * n + j] *= d;
     for (int r = 0; r < n; ++r) {
       if (r == c) continue;
       const double f = a[(size_t)r * n + c];
       if (f == 0.0) continue;
-      for (int j = 0; j < n; ++j) {
-        a[(size_t)r * n + j] -= f * a[(size_t)c * n + j];
-        inv[(size_t)r * n + j] -= f * inv[(size_t)c * n + j];
-      }
+      double *ar = &a[(size_t)r * n], *ir = &inv[(size_t)r * n];
+      const double *ac = &a[(size_t)c * n], *ic = &inv[(size_t)c * n];
+      for (int j = c; j < n; ++j) ar[j] -= f * ac[j];
+      for (int j = 0; j < used; ++j) ir[j] -= f * ic[j];
     }
   }
   a.swap(inv);

@@ -272,13 +272,40 @@ struct goal_states_s {
 
 // zero_* only mark a buffer as pending zero; the next assembly then writes
 // it instead of adding to it, and any other access fills it first.
+// Pinned host memory that a kernel writes results to, and the event after it:
+// the host waits for those results alone, with later work already queued.
+struct ReadBack {
+  double* p = nullptr;
+  int64_t n = 0;
+  hipEvent_t done = nullptr;
+  ReadBack() = default;
+  ReadBack(const ReadBack&) = delete;
+  ReadBack& operator=(const ReadBack&) = delete;
+  ~ReadBack() {
+    if (p) (void)hipHostFree(p);
+    if (done) (void)hipEventDestroy(done);
+  }
+  void reserve(int64_t count) {  // nothing may be in flight
+    if (!done) HIPCHK(hipEventCreateWithFlags(&done, hipEventDisableTiming));
+    if (n >= count) return;
+    if (p) HIPCHK(hipHostFree(p));
+    p = nullptr;
+    n = 0;
+    HIPCHK(hipHostMalloc(reinterpret_cast<void**>(&p), sizeof(double) * count, hipHostMallocDefault));
+    n = count;
+  }
+  void record() { HIPCHK(hipEventRecord(done, stream())); }
+  void wait() { HIPCHK(hipEventSynchronize(done)); }
+};
+
 struct goal_solinfo_s {
   goal_disc d = nullptr;
   DevBuf<double> R, dMdu, vals;
   bool zero_R = false, zero_dMdu = false, zero_vals = false;
   // linear-solve workspace, kept between solves
-  DevBuf<double> V, t, z, binv, partial, h1, h2, y;
+  DevBuf<double> V, t, z, binv, partial, h1, h2, y, norms;
   DevBuf<int32_t> solve_status;
+  ReadBack back;
 };
 
 struct goal_mech_s {
@@ -1042,39 +1069,39 @@ void amg_setup(goal_solinfo s, int* status) {
     // Arnoldi on Binv A from a fixed start vector (classical Gram-Schmidt,
     // two passes); its Ritz values place the smoother's ellipse
     const int64_t nv = 4 * L.nn;
+    // (both passes always, so all of it is queued and the host waits once)
     double* Q = h.arn.p;
-    std::vector<double> v0(nv);
-    for (int64_t i = 0; i < nv; ++i)
-      v0[i] = (double)(goal::splitmix64(0xA3C5u + (uint64_t)i) >> 11) * (1.0 / 9007199254740992.0) - 0.5;
-    HIPCHK(hipMemcpyAsync(Q, v0.data(), sizeof(double) * nv, hipMemcpyHostToDevice, stream()));
-    auto norm2 = [&](const double* v) {  // waits
-      HIPCHK(goal::launch_reduce(1, v, nullptr, nv, reduce_scratch(), result_slot(3), stream()));
-      double r2 = 0.0;
-      HIPCHK(hipMemcpyAsync(&r2, result_slot(3), sizeof(double), hipMemcpyDeviceToHost, stream()));
-      sync();
-      return std::sqrt(r2);
-    };
-    const double q0 = norm2(Q);
-    HIPCHK(goal::launch_scale(nv, 1.0 / q0, Q, Q, stream()));
     constexpr int M = kAmgArnoldi;
-    std::vector<double> H((size_t)(M + 1) * M, 0.0), hc(M + 1);
-    int steps = 0;
+    constexpr int64_t kStep = 2 * M + 4;  // read-back per step
+    double* nrm = s->norms.p;
+    auto norm_to = [&](const double* v) {  // |v|^2 where launch_arnoldi_end takes it
+      HIPCHK(goal::launch_reduce(1, v, nullptr, nv, reduce_scratch(), nrm + 1, stream()));
+    };
+    HIPCHK(goal::launch_arnoldi_start(nv, Q, stream()));
+    norm_to(Q);
+    HIPCHK(goal::launch_arnoldi_end(nv, Q, nrm, nullptr, 0, nullptr, 0, nullptr, stream()));
     for (int j = 0; j < M; ++j) {
       double* w = Q + (int64_t)(j + 1) * nv;
       HIPCHK(goal::launch_product(amg_matrix(s, h, l), Q + (int64_t)j * nv, nullptr, L.r.p, stream()));
       HIPCHK(goal::launch_block_apply(L.nn, L.binv.p, L.r.p, w, stream()));
-      for (int pass = 0; pass < 2; ++pass) {
-        HIPCHK(goal::launch_multi_dot(nv, j + 1, Q, nv, w, s->partial.p, s->h1.p, stream()));
-        HIPCHK(goal::launch_multi_axpy(nv, j + 1, Q, nv, s->h1.p, -1.0, w, stream()));
-        HIPCHK(hipMemcpyAsync(hc.data(), s->h1.p, sizeof(double) * (j + 1), hipMemcpyDeviceToHost, stream()));
-        sync();
-        for (int i = 0; i <= j; ++i) H[(size_t)i * M + j] += hc[i];
+      for (double* hp : {s->h1.p, s->h2.p}) {
+        HIPCHK(goal::launch_multi_dot(nv, j + 1, Q, nv, w, s->partial.p, hp, stream()));
+        HIPCHK(goal::launch_multi_axpy(nv, j + 1, Q, nv, hp, -1.0, w, stream()));
       }
-      const double hn = norm2(w);
+      norm_to(w);
+      HIPCHK(goal::launch_arnoldi_end(nv, w, nrm, s->h1.p, j + 1, s->h2.p, j + 1, s->back.p + j * kStep, stream()));
+    }
+    s->back.record();
+    s->back.wait();
+    std::vector<double> H((size_t)(M + 1) * M, 0.0);
+    int steps = 0;
+    for (int j = 0; j < M; ++j) {
+      const double* r = s->back.p + j * kStep;
+      for (int i = 0; i <= j; ++i) H[(size_t)i * M + j] = r[2 + i] + r[2 + j + 1 + i];
+      const double hn = std::sqrt(r[1]);
       H[(size_t)(j + 1) * M + j] = hn;
       steps = j + 1;
       if (!(hn > 1e-12 * std::fabs(H[(size_t)j * M + j])) || !std::isfinite(hn)) break;  // invariant subspace
-      HIPCHK(goal::launch_scale(nv, 1.0 / hn, w, w, stream()));
     }
     std::vector<double> Hs((size_t)steps * steps);
     for (int i = 0; i < steps; ++i)
@@ -1139,18 +1166,20 @@ void amg_smooth(goal_solinfo s, AmgHierarchy& h, int l, const double* b, double*
   }
 }
 
-// x = V-cycle applied to b on level l.
-void amg_vcycle(goal_solinfo s, AmgHierarchy& h, int l, const double* b, double* x) {
+// x = V-cycle applied to b on level l: the level's pre-smoothing (on the
+// coarsest all of it), then the rest.
+void amg_begin(goal_solinfo s, AmgHierarchy& h, int l, const double* b, double* x) {
+  if (l + 1 == (int)h.lv.size()) HIPCHK(goal::launch_dense_matvec(h.coarse_n, h.coarse_inv.p, b, x, stream()));
+  else amg_smooth(s, h, l, b, x, true);
+}
+void amg_end(goal_solinfo s, AmgHierarchy& h, int l, const double* b, double* x) {
+  if (l + 1 == (int)h.lv.size()) return;
   AmgLevel& L = *h.lv[l];
-  if (l + 1 == (int)h.lv.size()) {
-    HIPCHK(goal::launch_dense_matvec(h.coarse_n, h.coarse_inv.p, b, x, stream()));
-    return;
-  }
   AmgLevel& C = *h.lv[l + 1];
-  amg_smooth(s, h, l, b, x, true);
   HIPCHK(goal::launch_product(amg_matrix(s, h, l), x, b, L.r.p, stream()));
   HIPCHK(goal::launch_restrict(L.nc, L.aptr.p, L.amem.p, L.r.p, C.b.p, stream()));
-  amg_vcycle(s, h, l + 1, C.b.p, C.x.p);
+  amg_begin(s, h, l + 1, C.b.p, C.x.p);
+  amg_end(s, h, l + 1, C.b.p, C.x.p);
   HIPCHK(goal::launch_prolong(L.nn, L.agg.p, C.x.p, x, stream()));
   amg_smooth(s, h, l, b, x, false);
 }
@@ -1981,7 +2010,9 @@ int goal_linear_solve_pc(goal_solinfo s, const double* b, double* x, double rtol
     const int mk = std::max(m, kAmgArnoldi);  // the multigrid set-up's Arnoldi shares these
     if (s->partial.n < (int64_t)(mk + 2) * nb) s->partial.alloc((int64_t)(mk + 2) * nb);
     if (s->h1.n < mk + 2) s->h1.alloc(mk + 2);
-    if (s->h2.n < m + 1) s->h2.alloc(m + 1);
+    if (s->h2.n < mk + 1) s->h2.alloc(mk + 1);
+    if (s->norms.n < 2) s->norms.alloc(2);
+    s->back.reserve(std::max<int64_t>(2 * (int64_t)m + 5, kAmgArnoldi * (2 * kAmgArnoldi + 4)));
     if (s->y.n < m + 1) s->y.alloc(m + 1);
     if (s->solve_status.n < 1) s->solve_status.alloc(1);
     HIPCHK(hipMemsetAsync(s->solve_status.p, 0, sizeof(int32_t), stream()));
@@ -1995,9 +2026,15 @@ int goal_linear_solve_pc(goal_solinfo s, const double* b, double* x, double rtol
     const bool amg = precond == GOAL_PRECOND_AMG;
     if (amg) amg_setup(s, s->solve_status.p);
     else HIPCHK(goal::launch_block_inverse(nn, rp, cols, A, s->binv.p, s->solve_status.p, stream()));
-    auto prec = [&](const double* in, double* out) {  // out = M^{-1} in
-      if (amg) amg_vcycle(s, *d->amg, 0, in, out);
+    // out = M^{-1} in, in two parts: the host waits for an Arnoldi step's
+    // coefficients between the next step's first part (the finest
+    // pre-smoothing) and the rest, so the GPU does not wait for the host
+    auto prec_begin = [&](const double* in, double* out) {
+      if (amg) amg_begin(s, *d->amg, 0, in, out);
       else HIPCHK(goal::launch_block_apply(nn, s->binv.p, in, out, stream()));
+    };
+    auto prec_end = [&](const double* in, double* out) {
+      if (amg) amg_end(s, *d->amg, 0, in, out);
     };
     auto norm2 = [&](const double* v) {  // waits
       HIPCHK(goal::launch_reduce(1, v, nullptr, n, reduce_scratch(), result_slot(2), stream()));
@@ -2006,7 +2043,7 @@ int goal_linear_solve_pc(goal_solinfo s, const double* b, double* x, double rtol
       sync();
       return std::sqrt(r);
     };
-    std::vector<double> H((size_t)(m + 1) * m), cs(m), sn(m), g(m + 1), hh1(m + 2), hh2(m + 1), yv(m + 1);
+    std::vector<double> H((size_t)(m + 1) * m), cs(m), sn(m), g(m + 1), yv(m + 1);
     auto Hm = [&](int i, int j) -> double& { return H[(size_t)j * (m + 1) + i]; };
     int total = 0;
     double beta0 = -1.0, relres = 0.0;
@@ -2022,30 +2059,35 @@ int goal_linear_solve_pc(goal_solinfo s, const double* b, double* x, double rtol
       std::fill(g.begin(), g.end(), 0.0);
       g[0] = beta;
       int j = 0;
-      bool done = false;
+      bool done = false, begun = false;
       while (j < m && total < max_iters) {
         double* w = V + (int64_t)(j + 1) * n;
-        prec(V + (int64_t)j * n, t);
+        if (!begun) prec_begin(V + (int64_t)j * n, t);
+        prec_end(V + (int64_t)j * n, t);
         HIPCHK(goal::launch_product(fine, t, nullptr, w, stream()));
         // classical Gram-Schmidt with the DGKS test (the reference's Belos
         // orthogonalization, src/goal_linear_solve.cpp:53-90): a second pass
         // only when the first removed more than 1 - 1/sqrt(2) of the norm
         // w is V_{j+1}, so one more dot in the same pass gives |w|^2
+        double* nrm = s->norms.p;
+        const goal::DgksTest test{nrm, s->h1.p + j + 1};
         HIPCHK(goal::launch_multi_dot(n, j + 2, V, n, w, s->partial.p, s->h1.p, stream()));
         HIPCHK(goal::launch_multi_axpy(n, j + 1, V, n, s->h1.p, -1.0, w, stream()));
-        HIPCHK(hipMemcpyAsync(hh1.data(), s->h1.p, sizeof(double) * (j + 2), hipMemcpyDeviceToHost, stream()));
-        double hn = norm2(w);  // waits, so hh1 has arrived
-        const double wn = std::sqrt(std::max(hh1[j + 1], 0.0));
-        std::fill(hh2.begin(), hh2.begin() + j + 1, 0.0);
-        if (hn < wn * 0.70710678118654752) {
-          HIPCHK(goal::launch_multi_dot(n, j + 1, V, n, w, s->partial.p, s->h2.p, stream()));
-          HIPCHK(goal::launch_multi_axpy(n, j + 1, V, n, s->h2.p, -1.0, w, stream()));
-          HIPCHK(hipMemcpyAsync(hh2.data(), s->h2.p, sizeof(double) * (j + 1), hipMemcpyDeviceToHost, stream()));
-          hn = norm2(w);
-        }
-        for (int i = 0; i <= j; ++i) Hm(i, j) = hh1[i] + hh2[i];
+        HIPCHK(goal::launch_reduce(1, w, nullptr, n, reduce_scratch(), nrm, stream()));
+        HIPCHK(goal::launch_multi_dot(n, j + 1, V, n, w, s->partial.p, s->h2.p, stream(), test));
+        HIPCHK(goal::launch_multi_axpy(n, j + 1, V, n, s->h2.p, -1.0, w, stream(), test));
+        HIPCHK(goal::launch_reduce(1, w, nullptr, n, reduce_scratch(), nrm + 1, stream()));
+        HIPCHK(goal::launch_arnoldi_end(n, w, nrm, s->h1.p, j + 2, s->h2.p, j + 1, s->back.p, stream()));
+        s->back.record();
+        begun = j + 1 < m && total + 1 < max_iters;
+        if (begun) prec_begin(w, t);  // for nothing if this step is the last
+        s->back.wait();
+        const double* r1 = s->back.p + 2;
+        const double* r2 = r1 + j + 2;
+        const bool again = goal::DgksTest::again(s->back.p[0], r1[j + 1]);
+        const double hn = std::sqrt(s->back.p[1]);
+        for (int i = 0; i <= j; ++i) Hm(i, j) = r1[i] + (again ? r2[i] : 0.0);
         Hm(j + 1, j) = hn;
-        if (hn > 0.0) HIPCHK(goal::launch_scale(n, 1.0 / hn, w, w, stream()));
         for (int i = 0; i < j; ++i) {
           const double a = Hm(i, j), c = Hm(i + 1, j);
           Hm(i, j) = cs[i] * a + sn[i] * c;
@@ -2076,7 +2118,8 @@ int goal_linear_solve_pc(goal_solinfo s, const double* b, double* x, double rtol
         HIPCHK(hipMemcpyAsync(s->y.p, yv.data(), sizeof(double) * j, hipMemcpyHostToDevice, stream()));
         HIPCHK(goal::launch_fill(z, n, 0.0, stream()));
         HIPCHK(goal::launch_multi_axpy(n, j, V, n, s->y.p, 1.0, z, stream()));
-        prec(z, t);
+        prec_begin(z, t);
+        prec_end(z, t);
         HIPCHK(goal::launch_axpy(x, t, 1.0, n, stream()));
         sync();  // yv is reused by the next cycle
       }

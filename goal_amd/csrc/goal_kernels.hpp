@@ -171,12 +171,28 @@ hipError_t launch_restrict(int64_t nc, const int64_t* aptr, const int32_t* amem,
                            hipStream_t s);
 hipError_t launch_prolong(int64_t nf, const int32_t* agg, const double* xc, double* x, hipStream_t s);
 hipError_t launch_dense_matvec(int n, const double* M, const double* x, double* y, hipStream_t s);
+// The DGKS test of a second Gram-Schmidt pass, on the device: |w| after the
+// first (norm2 = |w|^2) below 1/sqrt(2) of |w| before (from2 = its square).
+// Without it (null) the pass runs.
+struct DgksTest {
+  const double* norm2 = nullptr;
+  const double* from2 = nullptr;
+  __host__ __device__ static bool again(double norm2, double from2) {
+    return sqrt(norm2) < sqrt(from2 > 0.0 ? from2 : 0.0) * 0.70710678118654752;
+  }
+  __device__ bool again() const { return !norm2 || again(*norm2, *from2); }
+};
 // out[j] = V_j . w (j < k); partial holds k * multi_dot_blocks(n) doubles
 int multi_dot_blocks(int64_t n);
 hipError_t launch_multi_dot(int64_t n, int k, const double* V, int64_t ldv, const double* w, double* partial,
-                            double* out, hipStream_t s);
+                            double* out, hipStream_t s, DgksTest test = {});
 hipError_t launch_multi_axpy(int64_t n, int k, const double* V, int64_t ldv, const double* c, double sign, double* w,
-                             hipStream_t s);
+                             hipStream_t s, DgksTest test = {});
+// End of an Arnoldi step: w /= sqrt(norms[1]); host (pinned, or null) gets
+// norms[0..1], then h1[k1], h2[k2].
+hipError_t launch_arnoldi_end(int64_t n, double* w, const double* norms, const double* h1, int k1, const double* h2,
+                              int k2, double* host, hipStream_t s);
+hipError_t launch_arnoldi_start(int64_t n, double* q, hipStream_t s);
 hipError_t launch_scale(int64_t n, double a, const double* x, double* y, hipStream_t s);
 
 hipError_t launch_fill(double* p, int64_t n, double v, hipStream_t s);

@@ -301,7 +301,8 @@ constexpr int kDotGroup = 8;
 
 __global__ __launch_bounds__(kSolveThreads) void multi_dot_partial_kernel(int64_t n, int k, const double* V,
                                                                           int64_t ldv, const double* w,
-                                                                          double* partial) {
+                                                                          double* partial, DgksTest test) {
+  if (!test.again()) return;
   __shared__ double red[kSolveThreads / 64][kDotGroup];
   const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
   const int64_t stride = (int64_t)gridDim.x * kSolveThreads;
@@ -330,7 +331,9 @@ __global__ __launch_bounds__(kSolveThreads) void multi_dot_partial_kernel(int64_
 }
 
 // out[j] = sum_b partial[j][b], one block per j.
-__global__ __launch_bounds__(kSolveThreads) void multi_dot_final_kernel(int nb, const double* partial, double* out) {
+__global__ __launch_bounds__(kSolveThreads) void multi_dot_final_kernel(int nb, const double* partial, double* out,
+                                                                        DgksTest test) {
+  if (!test.again()) return;
   __shared__ double red[kSolveThreads / 64];
   const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, j = blockIdx.x;
   double s = 0.0;
@@ -347,12 +350,45 @@ __global__ __launch_bounds__(kSolveThreads) void multi_dot_final_kernel(int nb, 
 
 // w += sign * sum_j c_j V_j, j < k.
 __global__ __launch_bounds__(kSolveThreads) void multi_axpy_kernel(int64_t n, int k, const double* V, int64_t ldv,
-                                                                   const double* c, double sign, double* w) {
+                                                                   const double* c, double sign, double* w,
+                                                                   DgksTest test) {
   const int64_t i = (int64_t)blockIdx.x * kSolveThreads + threadIdx.x;
-  if (i >= n) return;
+  if (i >= n || !test.again()) return;
   double s = 0.0;
   for (int j = 0; j < k; ++j) s += c[j] * V[(int64_t)j * ldv + i];
   w[i] += sign * s;
+}
+
+// w /= |w| (as it is where |w| = 0), with |w|^2 already on the device, so the
+// next step can be queued before the host has seen the norm.  Block 0 hands
+// what the host needs (k1 + k2 coefficients, both squared norms) to its
+// pinned memory.
+__global__ __launch_bounds__(kSolveThreads) void arnoldi_end_kernel(int64_t n, double* w, const double* norms,
+                                                                    const double* h1, int k1, const double* h2, int k2,
+                                                                    double* host) {
+  const double hn = sqrt(norms[1]);
+  if (blockIdx.x == 0 && host) {
+    for (int j = threadIdx.x; j < k1; j += kSolveThreads) host[2 + j] = h1[j];
+    for (int j = threadIdx.x; j < k2; j += kSolveThreads) host[2 + k1 + j] = h2[j];
+    if (threadIdx.x < 2) host[threadIdx.x] = norms[threadIdx.x];
+    __threadfence_system();
+  }
+  const int64_t i = (int64_t)blockIdx.x * kSolveThreads + threadIdx.x;
+  if (i < n && hn > 0.0) w[i] = (1.0 / hn) * w[i];
+}
+
+// splitmix64 (goal_mesh.hpp), on the device
+__device__ inline uint64_t device_splitmix64(uint64_t x) {
+  x += 0x9E3779B97F4A7C15ull;
+  x = (x ^ (x >> 30)) * 0xBF58476D1CE4E5B9ull;
+  x = (x ^ (x >> 27)) * 0x94D049BB133111EBull;
+  return x ^ (x >> 31);
+}
+
+// The start vector of the smoother's Arnoldi steps: fixed noise in [-1/2, 1/2).
+__global__ __launch_bounds__(kSolveThreads) void arnoldi_start_kernel(int64_t n, double* q) {
+  const int64_t i = (int64_t)blockIdx.x * kSolveThreads + threadIdx.x;
+  if (i < n) q[i] = (double)(device_splitmix64(0xA3C5u + (uint64_t)i) >> 11) * (1.0 / 9007199254740992.0) - 0.5;
 }
 
 // y = a * x  (y may alias x)
@@ -466,18 +502,31 @@ hipError_t launch_block_apply(int64_t nn, const double* binv, const double* x, d
 }
 
 hipError_t launch_multi_dot(int64_t n, int k, const double* V, int64_t ldv, const double* w, double* partial,
-                            double* out, hipStream_t s) {
+                            double* out, hipStream_t s, DgksTest test) {
   if (k == 0) return hipSuccess;
   const int nb = multi_dot_blocks(n);
-  hipLaunchKernelGGL(multi_dot_partial_kernel, dim3(nb, (k + kDotGroup - 1) / kDotGroup), dim3(kSolveThreads), 0, s, n, k, V, ldv, w, partial);
-  hipLaunchKernelGGL(multi_dot_final_kernel, dim3(k), dim3(kSolveThreads), 0, s, nb, partial, out);
+  hipLaunchKernelGGL(multi_dot_partial_kernel, dim3(nb, (k + kDotGroup - 1) / kDotGroup), dim3(kSolveThreads), 0, s, n, k, V, ldv, w, partial, test);
+  hipLaunchKernelGGL(multi_dot_final_kernel, dim3(k), dim3(kSolveThreads), 0, s, nb, partial, out, test);
   return hipGetLastError();
 }
 
 hipError_t launch_multi_axpy(int64_t n, int k, const double* V, int64_t ldv, const double* c, double sign, double* w,
-                             hipStream_t s) {
+                             hipStream_t s, DgksTest test) {
   if (n == 0 || k == 0) return hipSuccess;
-  hipLaunchKernelGGL(multi_axpy_kernel, grid_for(n), dim3(kSolveThreads), 0, s, n, k, V, ldv, c, sign, w);
+  hipLaunchKernelGGL(multi_axpy_kernel, grid_for(n), dim3(kSolveThreads), 0, s, n, k, V, ldv, c, sign, w, test);
+  return hipGetLastError();
+}
+
+hipError_t launch_arnoldi_end(int64_t n, double* w, const double* norms, const double* h1, int k1, const double* h2,
+                              int k2, double* host, hipStream_t s) {
+  if (n == 0) return hipSuccess;
+  hipLaunchKernelGGL(arnoldi_end_kernel, grid_for(n), dim3(kSolveThreads), 0, s, n, w, norms, h1, k1, h2, k2, host);
+  return hipGetLastError();
+}
+
+hipError_t launch_arnoldi_start(int64_t n, double* q, hipStream_t s) {
+  if (n == 0) return hipSuccess;
+  hipLaunchKernelGGL(arnoldi_start_kernel, grid_for(n), dim3(kSolveThreads), 0, s, n, q);
   return hipGetLastError();
 }
 
