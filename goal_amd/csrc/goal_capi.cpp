@@ -242,6 +242,7 @@ struct goal_disc_s {
   DevBuf<int32_t> node_adj_dev;           // the nodes' neighbours on the device
   std::unique_ptr<AmgHierarchy> amg;
   std::unique_ptr<ClusterPlan> cluster;
+  std::mutex cluster_mutex;
   int max_degree = 0;
   int64_t num_dofs = 0, nnz = 0;
   // gather plan: runs of consecutive nodes whose CSR values fit `gather_cap`
@@ -2189,9 +2190,12 @@ int goal_mech_create(goal_disc d, goal_states st, int num_sets, const goal_mater
     m->status.alloc(1);
     HIPCHK(hipMemsetAsync(m->status.p, 0, sizeof(int), stream()));
     m->elem_value.alloc(d->mesh.num_elems);
-    if (uses_clusters(m.get()) && !d->cluster) {
-      if (d->mesh.order == 2) cluster_build(d);
-      else linear_cluster_build(d);
+    if (uses_clusters(m.get())) {
+      std::lock_guard<std::mutex> one(d->cluster_mutex);  // mechanics of one disc may be made by several threads
+      if (!d->cluster) {
+        if (d->mesh.order == 2) cluster_build(d);
+        else linear_cluster_build(d);
+      }
     }
     sync();
     *out = m.release();
