@@ -2535,7 +2535,7 @@ int goal_learn_features(goal_mech m, double qoi_x, float* feat_dev) {
     q.status = m->status.p;
     HIPCHK(goal::launch_qoi(d->mesh.order, m->quad_order, q, stream()));
     require(d->mesh.num_elems > 0, "goal_learn_features: empty mesh");
-    if (m->feat_vol.n < 10 * ne) m->feat_vol.alloc(10 * ne);
+    if (m->feat_vol.n < goal::kFeatElem * ne) m->feat_vol.alloc(goal::kFeatElem * ne);
     if (m->feat_vm.n < 10 * nn) m->feat_vm.alloc(10 * nn);
     goal::FeatureArgs f{};
     f.num_elems = ne;

@@ -276,6 +276,7 @@ struct MlpArgs {
   float* adam_v;       // [kMlpParams]
 };
 
+constexpr int kFeatElem = 12;  // doubles per element in the features' scratch
 struct FeatureArgs {
   int64_t num_elems, num_nodes;
   int npe;
@@ -290,7 +291,7 @@ struct FeatureArgs {
   const int64_t* inc_ptr;   // node -> incidence records
   const int32_t* inc;       // record -> e * npe + local node
   double qoi_x;             // QoI subdomain {x < qoi_x}
-  double* elem_scratch;     // [ne][10] volume, grad u
+  double* elem_scratch;     // [ne][kFeatElem] von Mises integral, grad u, volume
   double* node_scratch;     // [num_nodes][10] recovered vm, grad u
   float* feat;              // [ne][kMlpIn]
 };

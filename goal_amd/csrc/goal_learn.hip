@@ -71,49 +71,75 @@ __device__ inline void load_vertices(const FeatureArgs& a, int64_t e, double X[4
     }
 }
 
-// Per element: volume and grad u, into elem_scratch[e][0..9].
+// Per element, into its row of elem_scratch: the von Mises integral, grad u and
+// the volume, all that the recovery reads of it.  A wave's rows go out through
+// LDS as one run: 53 us for 1.97 M tets, where each lane's own stores, 80 bytes
+// apart, took 70.
+constexpr int kRow = kFeatElem, kRowH = 1, kRowVol = 10;
+static_assert(kRowVol < kRow && kRow <= 16 && kRow % 2 == 0, "one lane of sixteen per value, stored in pairs");
 __global__ __launch_bounds__(kFeatThreads) void elem_geometry_kernel(FeatureArgs a) {
+  __shared__ double stage[kFeatThreads / 64][64 * (kRow + 1)];
   const int64_t e = (int64_t)blockIdx.x * kFeatThreads + threadIdx.x;
-  if (e >= a.num_elems) return;
-  double X[4][3], U[4][3], H[9];
-  load_vertices(a, e, X, U);
-  linear_grad(X, U, H);
-  double* o = a.elem_scratch + 10 * e;
-  o[0] = tet_volume(a.coords, a.conn + e * a.npe);
-  for (int k = 0; k < 9; ++k) o[1 + k] = H[k];
+  const int lane = threadIdx.x & 63;
+  double* w = stage[threadIdx.x >> 6];
+  if (e < a.num_elems) {
+    double X[4][3], U[4][3], H[9];
+    load_vertices(a, e, X, U);
+    linear_grad(X, U, H);
+    double* o = w + (kRow + 1) * lane;  // odd: the rows spread over the banks
+    o[0] = a.elem_vm[e];
+    for (int k = 0; k < 9; ++k) o[kRowH + k] = H[k];
+    o[kRowVol] = tet_volume(a.coords, a.conn + e * a.npe);
+    for (int k = kRowVol + 1; k < kRow; ++k) o[k] = 0.0;
+  }
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  const int64_t e0 = e - lane;
+#pragma unroll
+  for (int j = 0; j < kRow / 2; ++j) {
+    const int i = (64 * j + lane) / (kRow / 2), k = 2 * ((64 * j + lane) % (kRow / 2));
+    if (e0 + i < a.num_elems)
+      reinterpret_cast<double2*>(a.elem_scratch + kRow * e0)[64 * j + lane] =
+          double2{w[(kRow + 1) * i + k], w[(kRow + 1) * i + k + 1]};
+  }
 }
 
 // Volume-weighted nodal means of the element von Mises stress and of grad u:
 // node_scratch[n] = (sum int_e vm, sum |e| H_e) / sum |e| over the incident
 // elements in ascending order.
-// Sixteen lanes per node, one per value (lane 0 vm, 1-9 |e| H, 10 |e|), so an
-// element's ten values come as one run of 80 bytes and a node's elements four
-// at a time; each sum keeps its order.  Bound by the chain incidence -> element
-// row.  1.97 M tets (343 K nodes): 184 us; with one thread per node, whose
-// loads lie a node's elements apart, 345.
+// Sixteen lanes per node, one per value of an element's row, so a row comes as
+// one run of one or two lines, and a node's elements four at a time; each sum
+// keeps its order.  Bound by the lines the L2 delivers (about 36 a node).  1.97 M
+// tets (343 K nodes): 106 us; with the von Mises integrals apart and 80-byte rows
+// (2.6 lines an element) 184; with one thread per node 345.
 __global__ __launch_bounds__(kFeatThreads) void recover_kernel(FeatureArgs a) {
   constexpr int kAhead = 4;
   const int c = threadIdx.x & 15;
   const int64_t n = (int64_t)blockIdx.x * (kFeatThreads / 16) + threadIdx.x / 16;
   if (n >= a.num_nodes) return;  // uniform per group of 16 lanes
-  const int64_t k1 = a.inc_ptr[n + 1];
+  const int64_t k0 = a.inc_ptr[n], k1 = a.inc_ptr[n + 1];
   double s = 0.0;
-  for (int64_t k = a.inc_ptr[n]; k < k1; k += kAhead) {
-    double x[kAhead], y[kAhead];
+  for (int64_t kb = k0; kb < k1; kb += 16) {  // sixteen incidences, one a lane
+    const int32_t r = a.inc[kb + c < k1 ? kb + c : k0];
+    const int32_t mine = a.npe == 4 ? r / 4 : r / 10;
+    const int m = (int)(k1 - kb < 16 ? k1 - kb : 16);
+    for (int j0 = 0; j0 < m; j0 += kAhead) {
+      double x[kAhead];
 #pragma unroll
-    for (int j = 0; j < kAhead; ++j) {
-      const int32_t r = a.inc[k + j < k1 ? k + j : k];
-      const int64_t e = a.npe == 4 ? r / 4 : r / 10;
-      const double* g = a.elem_scratch + 10 * e;
-      x[j] = c == 0 ? a.elem_vm[e] : g[c < 10 ? c : 0];
-      y[j] = g[0];
+      for (int j = 0; j < kAhead; ++j) {  // past the end: an element of this node again, not added
+        const int64_t e = __shfl(mine, j0 + j, 16);  // by all sixteen: the source lane may be one without a value
+        x[j] = c <= kRowVol ? a.elem_scratch[kRow * e + c] : 0.0;
+      }
+#pragma unroll
+      for (int j = 0; j < kAhead; ++j) {
+        const double vol = __shfl(x[j], kRowVol, 16);
+        if (j0 + j < m) s += (c >= kRowH && c < kRowVol ? vol : 1.0) * x[j];
+      }
     }
-#pragma unroll
-    for (int j = 0; j < kAhead; ++j)
-      if (k + j < k1) s += (c > 0 && c < 10 ? y[j] : 1.0) * x[j];
   }
-  const double w = __shfl(s, 10, 16);
-  if (c < 10) a.node_scratch[10 * n + c] = w > 0.0 ? s / w : 0.0;
+  const double w = __shfl(s, kRowVol, 16);
+  if (c < kRowVol) a.node_scratch[10 * n + c] = w > 0.0 ? s / w : 0.0;
 }
 
 __device__ inline float flog10(double v) { return (float)log10(v); }
@@ -135,7 +161,7 @@ __global__ __launch_bounds__(kFeatThreads) void features_kernel(FeatureArgs a) {
   double X[4][3];
   for (int i = 0; i < 4; ++i)
     for (int c = 0; c < 3; ++c) X[i][c] = a.coords[3 * (int64_t)v[i] + c];
-  const double* ge = a.elem_scratch + 10 * e;
+  const double* ge = a.elem_scratch + kRow * e;
   double star[10] = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
   for (int i = 0; i < 4; ++i) {
     const double* nv = a.node_scratch + 10 * (int64_t)v[i];
@@ -143,8 +169,8 @@ __global__ __launch_bounds__(kFeatThreads) void features_kernel(FeatureArgs a) {
   }
   double h2 = 0.0, d2 = 0.0;
   for (int k = 0; k < 9; ++k) {
-    h2 += ge[1 + k] * ge[1 + k];
-    d2 += (ge[1 + k] - star[1 + k]) * (ge[1 + k] - star[1 + k]);
+    h2 += ge[kRowH + k] * ge[kRowH + k];
+    d2 += (ge[kRowH + k] - star[1 + k]) * (ge[kRowH + k] - star[1 + k]);
   }
   double l2 = 0.0;
   for (int k = 0; k < 6; ++k) {
@@ -158,7 +184,7 @@ __global__ __launch_bounds__(kFeatThreads) void features_kernel(FeatureArgs a) {
   const MatParams m = a.mats[a.elem_set[e]];
   const double E = 9.0 * m.kappa * m.mu / (3.0 * m.kappa + m.mu);
   const double nu = (3.0 * m.kappa - 2.0 * m.mu) / (2.0 * (3.0 * m.kappa + m.mu));
-  const double vm = a.elem_vm[e] / ge[0];
+  const double vm = ge[0] / ge[kRowVol];
   double eq = 0.0;
   if (a.eqps) {
     for (int q = 0; q < a.nq; ++q) eq += a.eqps[e * a.nq + q];
