@@ -1,12 +1,14 @@
-// Element assembly for goal's mixed u-p Total Lagrangian tets, in two passes.
+// Element assembly for goal's mixed u-p Total Lagrangian tets, in two passes:
+// the Jacobian kinds that are not summed over node clusters (goal_cluster.hip)
+// - FP32 tangent, elastic, quadratic J2, linear tets with four points,
+// quadratic ones with one, and meshes that the clusters do not take.
 //
 // Pass 1 (element_kernel) runs, per element, the evaluator chain that
 // goal::assemble() runs hook by hook (src/goal_assembly.cpp:65-88, chain order
 // src/goal_mechanics.cpp:97-146): gather of u and p, interpolation at the
 // quadrature points, kinematics F = I + grad u and J, the constitutive model,
 // Mixed, MResidual, PResidual and Stabilization.  It writes the element
-// residual r_e and, for the Jacobian, the element matrix k_e to element-major
-// buffers with coalesced stores.
+// residual r_e and the element matrix k_e by incidence record.
 //
 // Pass 2 (gather_kernel) is the scatter (Displacement/Pressure::scatter,
 // src/goal_displacement.cpp:77-86,177-214, src/goal_pressure.cpp:76-83,170-203)

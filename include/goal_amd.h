@@ -256,14 +256,14 @@ int goal_mech_destroy(goal_mech m);
  * "overlap" (neo-Hookean only: 2..1024 runs the element pass in this many
  * chunks and gathers each finished chunk's node ranges on a second stream,
  * bitwise equal to one pass; 0 off; -1, the default, is one pass; not used
- * under stream capture, nor by the FP64 Jacobians of ten-node four-point tets,
- * which one kernel forms without a gather: goal_mech_timing counts all of it
- * as the element pass),
+ * under stream capture, nor by the FP64 Jacobians that sum their blocks over
+ * node clusters: ten-node four-point and four-node one-point tets),
  * "overlap_blocks" (element workgroups per chunk, 0 = 5/6 of the resident
  * grid). */
 int goal_mech_set_option(goal_mech m, const char* key, int64_t value);
 /* Device time of the last assembly's element pass and node gather, in ms
- * (waits for it).  Needs the "timing" option.  No counterpart in the
+ * (waits for it); over node clusters all of it (ten-node tets), or the point
+ * states and the block sums (four-node tets).  Needs the "timing" option.  No counterpart in the
  * reference (goal::time() brackets whole phases on the host,
  * src/goal_primal.cpp:76-108); it is for profiling callers. */
 int goal_mech_timing(goal_mech m, float* element_ms, float* gather_ms);
