@@ -807,23 +807,20 @@ void run_linear_clustered(goal_mech m, goal_solinfo s, int kind, goal::AsmArgs a
   c.pt = pt;
   c.R = s->R.p;
   c.vals = s->vals.p;
+  c.zero = s->zero_dMdu ? s->dMdu.p : nullptr;
   c.overwrite_R = s->zero_R ? 1 : 0;
   c.overwrite_vals = s->zero_vals ? 1 : 0;
   c.xcd_remap = a.xcd_remap;
   if (m->timing) HIPCHK(hipEventRecord(m->ev[0], stream()));
   HIPCHK(goal::launch_linear_points(a, stream()));
   if (m->timing) HIPCHK(hipEventRecord(m->ev[1], stream()));
-  if (s->zero_dMdu) {
-    HIPCHK(goal::launch_fill(s->dMdu.p, s->dMdu.n, 0.0, stream()));
-    s->zero_dMdu = false;
-  }
   HIPCHK(goal::launch_linear_cluster(kind == goal::ASM_ADJOINT, m->model == goal::MODEL_J2, c, asm_blocks(m),
                                      stream()));
   if (m->timing) {
     HIPCHK(hipEventRecord(m->ev[2], stream()));
     m->timed = true;
   }
-  s->zero_R = s->zero_vals = false;
+  s->zero_R = s->zero_vals = s->zero_dMdu = false;
 }
 
 void run_clustered(goal_mech m, goal_solinfo s, int kind, const goal::AsmArgs& a) {
@@ -846,23 +843,20 @@ void run_clustered(goal_mech m, goal_solinfo s, int kind, const goal::AsmArgs& a
   c.sigma = a.sigma;
   c.R = s->R.p;
   c.vals = s->vals.p;
+  c.zero = s->zero_dMdu ? s->dMdu.p : nullptr;
   c.overwrite_R = s->zero_R ? 1 : 0;
   c.overwrite_vals = s->zero_vals ? 1 : 0;
   c.stabilization = a.stabilization;
   c.save_state = a.save_state;
   c.xcd_remap = a.xcd_remap;
   if (m->timing) HIPCHK(hipEventRecord(m->ev[0], stream()));
-  if (s->zero_dMdu) {
-    HIPCHK(goal::launch_fill(s->dMdu.p, s->dMdu.n, 0.0, stream()));
-    s->zero_dMdu = false;
-  }
   HIPCHK(goal::launch_cluster(kind == goal::ASM_ADJOINT, c, asm_blocks(m), stream()));
   if (m->timing) {  // all of it counts as the element pass: there is no gather
     HIPCHK(hipEventRecord(m->ev[1], stream()));
     HIPCHK(hipEventRecord(m->ev[2], stream()));
     m->timed = true;
   }
-  s->zero_R = s->zero_vals = false;
+  s->zero_R = s->zero_vals = s->zero_dMdu = false;
 }
 
 // Element residuals between the passes: the mechanics' own, allocated on first use.

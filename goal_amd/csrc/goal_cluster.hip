@@ -621,6 +621,14 @@ __device__ __forceinline__ void lds_barrier() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
 
+// A pending clear of the functional's derivative goes along with the runs, each
+// node being in one: a launch less (162 tets 34.4 -> 32.6 us, 3,072 quadratic
+// ones 51.1 -> 46.6).
+__device__ __forceinline__ void clear_node(double* zero, int32_t n) {
+  double2* z = reinterpret_cast<double2*>(zero + 4 * (int64_t)n);
+  z[0] = z[1] = double2{0.0, 0.0};
+}
+
 // The chunks of a workgroup's runs, one after the other: chunk r is run r's
 // first, its further ones are r.z .. r.w.
 struct ClusterCursor {
@@ -665,6 +673,7 @@ __global__ __launch_bounds__(kClusterThreads, 3) void cluster_kernel(ClusterArgs
       const int32_t n = a.nodes[cur.r.x + lane];
       const int64_t b = a.row_ptr[4 * (int64_t)n];
       nid[lane] = n;
+      if (a.zero) clear_node(a.zero, n);
       nbase[lane] = b;
       nlen[lane] = (int)(a.row_ptr[4 * (int64_t)n + 1] - b);
     }
@@ -1237,6 +1246,7 @@ __global__ __launch_bounds__(kLinearThreads, PLASTIC ? 3 : 4) void linear_cluste
         double* o = a.R + 4 * (int64_t)nid[nl];
 #pragma unroll
         for (int i = 0; i < 4; ++i) o[i] = (a.overwrite_R ? 0.0 : o[i]) + s.r[i];
+        if (a.zero) clear_node(a.zero, nid[nl]);  // at the node table it cost the plastic kernel 2%
       }
     }
   }

@@ -198,6 +198,7 @@ struct LinearArgs {
   const double* pt;         // [elements][kLinearPoint]
   double* R;
   double* vals;
+  double* zero;             // [4 nodes] cleared along the way, or null
   int overwrite_R, overwrite_vals, xcd_remap;
 };
 
@@ -221,6 +222,7 @@ struct ClusterArgs {
   double* sigma;
   double* R;
   double* vals;
+  double* zero;             // [4 nodes] cleared along the way, or null
   int overwrite_R, overwrite_vals;
   int stabilization, save_state, xcd_remap;
 };

@@ -56,6 +56,13 @@ def test_one_kernel_assembly_matches_oracle(kind, adjoint):
     assert rel(st.get("sigma"), ost.sigma) < RTOL
     mech.jacobian(si, adjoint=adjoint)  # added to what is there
     assert rel(si.R(), 2 * Ro) < RTOL and rel(si.vals(), 2 * Vo) < RTOL
+    mech.qoi(g.QOI_AVG_DISP, si)
+    dm = si.dMdu()
+    mech.jacobian(si, adjoint=adjoint)
+    assert dm.any() and np.array_equal(si.dMdu(), dm)  # no clear is pending
+    si.zero_all()
+    mech.jacobian(si, adjoint=adjoint)
+    assert not si.dMdu().any()
     for blocks in (1, 8, 40):  # grids smaller than the runs, with and without the XCD slabs
         mech.set_option("blocks", blocks)
         si.zero_all()
