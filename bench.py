@@ -397,7 +397,7 @@ def summarize_batch(kt_dir, fetch_dir, write_dir, commands, replays):
     the kernel trace (each one dispatch per kernel node of the graph), with
     HBM traffic from the FETCH_SIZE / WRITE_SIZE runs over the same dispatches."""
     specs = batch_meshes()
-    nodes = sum(2 if sp_["order"] == 2 else 3 for sp_ in specs)  # fill; P2: one kernel, P1: points and block sums
+    nodes = sum(1 if sp_["order"] == 2 else 2 for sp_ in specs)  # P2: one kernel, P1: points and block sums
     trace = sorted(_read_csv(_find(kt_dir, "kernel_trace.csv")), key=lambda r: int(r["Start_Timestamp"]))
     timed = trace[-replays * nodes:]
     spans = []
@@ -444,7 +444,7 @@ def summarize_batch(kt_dir, fetch_dir, write_dir, commands, replays):
              f"The batched workload: {len(specs)} seeded box meshes, {sum(ne):,} tets in all "
              f"({min(ne):,} to {max(ne):,} per mesh). Even meshes are P2 neo-Hookean with 4 points, odd ones P1 J2 "
              f"with 1 point and per-point history.",
-             f"One captured HIP graph holds every mesh's residual + Jacobian assembly: per mesh one fill, then one "
+             f"One captured HIP graph holds every mesh's residual + Jacobian assembly: per mesh one "
              f"kernel over node clusters (P2) or the point states and the block sums (P1): {nodes} dispatches per "
              f"replay.", "", "Commands (repository root on the GPU host):", ""]
     lines += [f"    {c}" for c in commands]
