@@ -325,6 +325,8 @@ struct goal_mech_s {
   DevBuf<double> elem_value;
   DevBuf<double> emr, em;  // element residuals / matrices between the two passes
   DevBuf<double> pt;       // J2 point states between the point pass and the element pass
+  DevBuf<double> linear_pt;  // linear elements' point states over node clusters; apart from pt, whose size
+                             // differs: a captured graph holds this one's address
   DevBuf<double> feat_vol, feat_vm;  // learned-indicator feature scratch
   bool timing = false, timed = false;
   hipEvent_t ev[3] = {nullptr, nullptr, nullptr};
@@ -791,8 +793,8 @@ void run_linear_clustered(goal_mech m, goal_solinfo s, int kind, goal::AsmArgs a
   const ClusterPlan& p = *d->cluster;
   if (!pt) {
     const int64_t n = goal::kLinearPoint * d->mesh.num_elems;
-    if (m->pt.n < n) m->pt.alloc(n);
-    pt = m->pt.p;
+    if (m->linear_pt.n < n) m->linear_pt.alloc(n);
+    pt = m->linear_pt.p;
   }
   a.pt = pt;
   goal::LinearArgs c{};
