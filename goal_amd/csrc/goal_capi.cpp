@@ -222,17 +222,36 @@ struct AmgHierarchy {
   int coarse_n = 0;
 };
 
-// Node clusters of a disc (goal_cluster.hpp), made when the first mechanics
-// that uses them is; no runs where a node has more neighbours than a run takes
-// blocks, or no element.
+// Parts of one allocation.
+struct Carve {
+  size_t size = 0;
+  template <typename T>
+  size_t take(int64_t n) {
+    const size_t at = size;
+    size += (sizeof(T) * (size_t)n + 255) / 256 * 256;
+    return at;
+  }
+};
+struct Arena : DevBuf<uint8_t> {
+  void alloc(const Carve& c) { DevBuf<uint8_t>::alloc((int64_t)c.size); }
+  template <typename T>
+  T* at(size_t offset) const {
+    return reinterpret_cast<T*>(p + offset);
+  }
+};
+
+// Node clusters of a disc (goal_cluster.hpp), made by the first Jacobian that
+// takes them (clusters_of); no runs where a node has more neighbours than a run
+// takes blocks, or no element.
 struct ClusterPlan {
   int64_t num_runs = 0;
-  DevBuf<int4> runs, chunks;
-  DevBuf<int2> spans;            // linear elements only
-  DevBuf<int32_t> linear_elems;  // linear elements only
-  DevBuf<uint32_t> elems;
-  DevBuf<goal::ClusterLane> lanes;
-  DevBuf<int32_t> nodes, conn;
+  Arena mem, lane_mem;
+  int4 *runs = nullptr, *chunks = nullptr;
+  int2* spans = nullptr;            // linear elements only
+  int32_t* linear_elems = nullptr;  // linear elements only
+  uint32_t* elems = nullptr;
+  goal::ClusterLane* lanes = nullptr;
+  int32_t *nodes = nullptr, *conn = nullptr;
 };
 
 struct goal_disc_s {
@@ -475,122 +494,117 @@ void disc_build(goal_disc d) {
   sync();  // the graph buffers are released on return
 }
 
-// The disc's node clusters: ordered by key, sized, then filled, on the device.
-void cluster_build(goal_disc d) {
+// The node clusters of a quadratic disc: ordered by key, sized, then filled, on
+// the device.
+std::unique_ptr<ClusterPlan> cluster_build(goal_disc d) {
   auto p = std::make_unique<ClusterPlan>();
   const int64_t nn = d->mesh.num_nodes, ne = d->mesh.num_elems;
-  if (d->max_degree <= goal::kClusterSlots && ne > 0) {
-    size_t tb = 0;
-    HIPCHK(goal::cluster_temp_bytes(std::max(nn, 10 * ne), &tb));
-    // one work buffer: sort and scan scratch, then the arrays over nodes and incidences
-    DevBuf<uint8_t> work;
-    size_t at = 0;
-    auto reserve = [&](int64_t bytes) {
-      const size_t o = at;
-      at += ((size_t)bytes + 255) / 256 * 256;
-      return o;
-    };
-    const size_t o_temp = reserve((int64_t)tb), o_box = reserve(48), o_most = reserve(4), o_seg = reserve(8 * (nn + 1));
-    size_t o_n[7];
-    for (size_t& o : o_n) o = reserve(4 * (nn + 1));
-    const size_t o_recs = reserve(8 * 10 * ne);
-    work.alloc((int64_t)at);
-    auto ints = [&](size_t o) { return reinterpret_cast<int32_t*>(work.p + o); };
-    void* temp = work.p + o_temp;
-    int64_t* seg = reinterpret_cast<int64_t*>(work.p + o_seg);
-    int32_t *keys = ints(o_n[0]), *sorted = ints(o_n[1]), *rank = ints(o_n[2]), *place = ints(o_n[3]),
-            *nr = ints(o_n[4]), *nx = ints(o_n[5]), *nk = ints(o_n[6]), *most = ints(o_most);
-    int2* recs = reinterpret_cast<int2*>(work.p + o_recs);
-    p->nodes.alloc(nn);
-    HIPCHK(goal::cluster_order(d->conn.p, d->coords.p, ne, nn, temp, tb,
-                               reinterpret_cast<unsigned long long*>(work.p + o_box), keys, sorted, rank, place,
-                               p->nodes.p, seg, stream()));
-    const goal::ClusterMesh m{p->nodes.p, d->inc_ptr.p, d->inc.p, d->row_ptr.p, d->posi.p, d->pos.p, d->cols.p, place};
-    HIPCHK(hipMemsetAsync(most, 0, sizeof(int32_t), stream()));
-    HIPCHK(goal::cluster_count(m, seg, nn, temp, tb, nr, nx, nk, most, stream()));
-    int32_t runs = 0, more = 0, nb = 0, lanes = 0;
-    HIPCHK(hipMemcpyAsync(&runs, nr + nn, sizeof(int32_t), hipMemcpyDeviceToHost, stream()));
-    HIPCHK(hipMemcpyAsync(&more, nx + nn, sizeof(int32_t), hipMemcpyDeviceToHost, stream()));
-    HIPCHK(hipMemcpyAsync(&nb, most, sizeof(int32_t), hipMemcpyDeviceToHost, stream()));
-    sync();
-    if (nb <= goal::kClusterSlots && runs > 0) {
-      const int64_t chunks = (int64_t)runs + more;
-      p->runs.alloc(runs);
-      p->chunks.alloc(chunks);
-      p->elems.alloc(chunks * goal::kClusterElems);
-      p->conn.alloc(chunks * goal::kClusterElems * 10);
-      DevBuf<int32_t> sizes;  // lanes of every chunk, then its incidences
-      sizes.alloc(3 * chunks + 2);
-      int32_t* nlanes = sizes.p;
-      int2* spans = reinterpret_cast<int2*>(sizes.p + (chunks + 2) / 2 * 2);
-      HIPCHK(goal::cluster_fill(m, seg, nn, nr, nx, nk, runs, p->runs.p, p->chunks.p, spans, p->elems.p, recs,
-                                stream()));
-      HIPCHK(hipMemsetAsync(nlanes + chunks, 0, sizeof(int32_t), stream()));
-      HIPCHK(goal::cluster_lanes(m, runs, chunks, p->runs.p, p->chunks.p, spans, p->elems.p, recs, nlanes, temp, tb,
-                                 nullptr, stream()));
-      HIPCHK(hipMemcpyAsync(&lanes, nlanes + chunks, sizeof(int32_t), hipMemcpyDeviceToHost, stream()));
-      sync();
-      p->lanes.alloc(lanes);
-      HIPCHK(goal::cluster_lanes(m, runs, chunks, p->runs.p, p->chunks.p, spans, p->elems.p, recs, nlanes, temp, tb,
-                                 p->lanes.p, stream()));
-      HIPCHK(goal::cluster_conn(chunks, p->chunks.p, p->elems.p, d->conn.p, p->conn.p, stream()));
-      p->num_runs = runs;
-      sync();  // the work buffers are released here and on return
-    }
-    sync();  // the work buffers are released on return
-  }
-  d->cluster = std::move(p);
+  if (d->max_degree > goal::kClusterSlots || ne == 0) return p;
+  size_t tb = 0;
+  HIPCHK(goal::cluster_temp_bytes(std::max(nn, 10 * ne), &tb));
+  Carve c;
+  const size_t o_temp = c.take<uint8_t>((int64_t)tb), o_box = c.take<uint64_t>(6), o_most = c.take<int32_t>(1),
+               o_totals = c.take<int4>(1), o_seg = c.take<int64_t>(nn + 1), o_recs = c.take<int2>(10 * ne);
+  size_t o_n[8];
+  for (size_t& o : o_n) o = c.take<int32_t>(nn + 1);
+  Arena work;
+  work.alloc(c);
+  void* temp = work.at<void>(o_temp);
+  int64_t* seg = work.at<int64_t>(o_seg);
+  int2* recs = work.at<int2>(o_recs);
+  int4* totals = work.at<int4>(o_totals);
+  int32_t* ni[8];
+  for (int i = 0; i < 8; ++i) ni[i] = work.at<int32_t>(o_n[i]);
+  int32_t *place = ni[0], *nodes = ni[1], *nr = ni[2], *nx = ni[3], *nk = ni[4], *most = work.at<int32_t>(o_most);
+  HIPCHK(goal::cluster_order(d->conn.p, d->coords.p, ne, nn, temp, tb, work.at<unsigned long long>(o_box), ni[5],
+                             ni[6], ni[7], place, nodes, seg, stream()));
+  goal::ClusterMesh m{nodes, d->inc_ptr.p, d->inc.p, d->row_ptr.p, d->posi.p, d->pos.p, d->cols.p, place};
+  HIPCHK(hipMemsetAsync(most, 0, sizeof(int32_t), stream()));
+  HIPCHK(goal::cluster_count(m, seg, nn, temp, tb, nr, nx, nk, most, stream()));
+  HIPCHK(goal::cluster_totals(nr + nn, nx + nn, most, most, totals, stream()));
+  int4 t{};
+  HIPCHK(hipMemcpyAsync(&t, totals, sizeof(t), hipMemcpyDeviceToHost, stream()));
+  sync();
+  const int64_t runs = t.x, chunks = (int64_t)t.x + t.y;
+  // lanes are counted in 32 bits: at most one per visit and a wavefront's padding per chunk
+  if (t.z > goal::kClusterSlots || runs == 0 || 55 * ne + 64 * chunks >= (int64_t(1) << 32)) return p;
+  Carve k;
+  const size_t o_runs = k.take<int4>(runs), o_chunks = k.take<int4>(chunks), o_spans = k.take<int2>(chunks),
+               o_elems = k.take<uint32_t>(chunks * goal::kClusterElems),
+               o_conn = k.take<int32_t>(chunks * goal::kClusterElems * 10), o_nodes = k.take<int32_t>(nn),
+               o_nlanes = k.take<int32_t>(chunks + 1);
+  p->mem.alloc(k);
+  p->runs = p->mem.at<int4>(o_runs);
+  p->chunks = p->mem.at<int4>(o_chunks);
+  p->elems = p->mem.at<uint32_t>(o_elems);
+  p->conn = p->mem.at<int32_t>(o_conn);
+  p->nodes = p->mem.at<int32_t>(o_nodes);
+  int2* spans = p->mem.at<int2>(o_spans);
+  int32_t* nlanes = p->mem.at<int32_t>(o_nlanes);
+  HIPCHK(hipMemcpyAsync(p->nodes, nodes, sizeof(int32_t) * nn, hipMemcpyDeviceToDevice, stream()));
+  HIPCHK(goal::cluster_fill(m, seg, nn, nr, nx, nk, runs, p->runs, p->chunks, spans, p->elems, recs, stream()));
+  HIPCHK(hipMemsetAsync(nlanes + chunks, 0, sizeof(int32_t), stream()));
+  HIPCHK(goal::cluster_lanes(m, runs, chunks, p->runs, p->chunks, spans, p->elems, recs, nlanes, temp, tb, nullptr,
+                             stream()));
+  int32_t lanes = 0;
+  HIPCHK(hipMemcpyAsync(&lanes, nlanes + chunks, sizeof(int32_t), hipMemcpyDeviceToHost, stream()));
+  sync();
+  if (lanes < 0) return std::make_unique<ClusterPlan>();  // 2^31 lanes and more
+  Carve l;
+  l.take<goal::ClusterLane>(lanes);
+  p->lane_mem.alloc(l);
+  p->lanes = p->lane_mem.at<goal::ClusterLane>(0);
+  HIPCHK(goal::cluster_lanes(m, runs, chunks, p->runs, p->chunks, spans, p->elems, recs, nlanes, temp, tb, p->lanes,
+                             stream()));
+  HIPCHK(goal::cluster_conn(chunks, p->chunks, p->elems, d->conn.p, p->conn, stream()));
+  sync();  // the work buffer is released on return
+  p->num_runs = runs;
+  return p;
 }
 
 // The same for linear elements.
-void linear_cluster_build(goal_disc d) {
+std::unique_ptr<ClusterPlan> linear_cluster_build(goal_disc d) {
   auto p = std::make_unique<ClusterPlan>();
   const int64_t nn = d->mesh.num_nodes, ne = d->mesh.num_elems;
-  const int64_t groups = (nn + goal::kLinearNodes - 1) / goal::kLinearNodes;
+  const int64_t groups = (nn + goal::kLinearNodes - 1) / goal::kLinearNodes, most = goal::kLinearNodes * groups;
   // lanes are counted in 32 bits: at most one per visit (ten an element) and a wavefront's padding per run
-  if (d->max_degree <= goal::kClusterSlots && ne > 0 && 10 * ne + 64 * nn < (int64_t(1) << 31)) {
-    size_t tb = 0;
-    HIPCHK(goal::cluster_temp_bytes(nn, &tb));
-    DevBuf<uint8_t> temp, box;
-    DevBuf<uint32_t> code;
-    DevBuf<int32_t> place, parts, sizes, bad;
-    temp.alloc((int64_t)tb);
-    box.alloc(48);
-    code.alloc(2 * nn);
-    place.alloc(nn);
-    parts.alloc(groups + 1);
-    bad.alloc(1);
-    p->nodes.alloc(nn);
-    HIPCHK(goal::linear_order(d->coords.p, nn, temp.p, tb, reinterpret_cast<unsigned long long*>(box.p), code.p,
-                              code.p + nn, place.p, p->nodes.p, stream()));
-    const goal::ClusterMesh m{p->nodes.p, d->inc_ptr.p, d->inc.p,  d->row_ptr.p,
-                              d->posi.p,  d->pos.p,     d->cols.p, place.p};
-    HIPCHK(hipMemsetAsync(bad.p, 0, sizeof(int32_t), stream()));
-    HIPCHK(goal::linear_split(m, nn, temp.p, tb, parts.p, bad.p, stream()));
-    int32_t runs = 0, unfit = 0;
-    HIPCHK(hipMemcpyAsync(&runs, parts.p + groups, sizeof(int32_t), hipMemcpyDeviceToHost, stream()));
-    HIPCHK(hipMemcpyAsync(&unfit, bad.p, sizeof(int32_t), hipMemcpyDeviceToHost, stream()));
-    sync();
-    if (!unfit) {
-      sizes.alloc(2 * ((int64_t)runs + 1));
-      int32_t *nlanes = sizes.p, *nelems = sizes.p + runs + 1;
-      HIPCHK(goal::linear_tables(m, nn, runs, parts.p, temp.p, tb, nlanes, nelems, nullptr, nullptr, nullptr, nullptr,
-                                 stream()));
-      int32_t lanes = 0, elems = 0;
-      HIPCHK(hipMemcpyAsync(&lanes, nlanes + runs, sizeof(int32_t), hipMemcpyDeviceToHost, stream()));
-      HIPCHK(hipMemcpyAsync(&elems, nelems + runs, sizeof(int32_t), hipMemcpyDeviceToHost, stream()));
-      sync();
-      p->runs.alloc(runs);
-      p->spans.alloc(runs);
-      p->linear_elems.alloc(elems);
-      p->lanes.alloc(lanes);
-      HIPCHK(goal::linear_tables(m, nn, runs, parts.p, temp.p, tb, nlanes, nelems, p->runs.p, p->spans.p,
-                                 p->linear_elems.p, p->lanes.p, stream()));
-      p->num_runs = runs;
-    }
-    sync();  // the work buffers are released on return
-  }
-  d->cluster = std::move(p);
+  if (d->max_degree > goal::kClusterSlots || ne == 0 || 10 * ne + 64 * nn >= (int64_t(1) << 31)) return p;
+  size_t tb = 0;
+  HIPCHK(goal::cluster_temp_bytes(most, &tb));
+  Carve c;
+  const size_t o_temp = c.take<uint8_t>((int64_t)tb), o_box = c.take<uint64_t>(6), o_bad = c.take<int32_t>(1),
+               o_totals = c.take<int4>(1), o_code = c.take<uint32_t>(2 * nn), o_place = c.take<int32_t>(nn),
+               o_nodes = c.take<int32_t>(nn), o_parts = c.take<int32_t>(groups + 1),
+               o_nlanes = c.take<int32_t>(most + 1), o_nelems = c.take<int32_t>(most + 1);
+  Arena work;
+  work.alloc(c);
+  void* temp = work.at<void>(o_temp);
+  uint32_t* code = work.at<uint32_t>(o_code);
+  int32_t *place = work.at<int32_t>(o_place), *nodes = work.at<int32_t>(o_nodes), *parts = work.at<int32_t>(o_parts),
+          *nlanes = work.at<int32_t>(o_nlanes), *nelems = work.at<int32_t>(o_nelems), *bad = work.at<int32_t>(o_bad);
+  HIPCHK(goal::linear_order(d->coords.p, nn, temp, tb, work.at<unsigned long long>(o_box), code, code + nn, place,
+                            nodes, stream()));
+  const goal::ClusterMesh m{nodes, d->inc_ptr.p, d->inc.p, d->row_ptr.p, d->posi.p, d->pos.p, d->cols.p, place};
+  HIPCHK(hipMemsetAsync(bad, 0, sizeof(int32_t), stream()));
+  HIPCHK(goal::linear_split(m, nn, temp, tb, parts, nlanes, nelems, bad, work.at<int4>(o_totals), stream()));
+  int4 t{};  // runs, lanes, elements of the runs, whether a node does not fit
+  HIPCHK(hipMemcpyAsync(&t, work.at<int4>(o_totals), sizeof(t), hipMemcpyDeviceToHost, stream()));
+  sync();
+  if (t.w) return p;
+  Carve k;
+  const size_t o_runs = k.take<int4>(t.x), o_spans = k.take<int2>(t.x), o_elems = k.take<int32_t>(t.z),
+               o_kept = k.take<int32_t>(nn), o_lanes = k.take<goal::ClusterLane>(t.y);
+  p->mem.alloc(k);
+  p->runs = p->mem.at<int4>(o_runs);
+  p->spans = p->mem.at<int2>(o_spans);
+  p->linear_elems = p->mem.at<int32_t>(o_elems);
+  p->nodes = p->mem.at<int32_t>(o_kept);
+  p->lanes = p->mem.at<goal::ClusterLane>(o_lanes);
+  HIPCHK(hipMemcpyAsync(p->nodes, nodes, sizeof(int32_t) * nn, hipMemcpyDeviceToDevice, stream()));
+  HIPCHK(goal::linear_tables(m, nn, parts, nlanes, nelems, p->runs, p->spans, p->linear_elems, p->lanes, stream()));
+  sync();  // the work buffer is released on return
+  p->num_runs = t.x;
+  return p;
 }
 
 // The node adjacency's column lists on the host (the multigrid aggregation
@@ -777,20 +791,32 @@ int64_t point_states(goal_mech m) {
   return goal::point_state_doubles(m->d->mesh.num_elems * m->st->nq, goal::kPointTangent);
 }
 
-// Whether the element matrices of an assembly are summed where they are formed
-// (over node clusters) instead of going through memory.
+// Whether the element matrices of an assembly can be summed where they are
+// formed (over node clusters) instead of going through memory.
 bool uses_clusters(const goal_mech_s* m) {
-  return m->d->mesh.order == 2 ? m->quad_order == 2 && m->model == goal::MODEL_NEOHOOKEAN
-                               : m->quad_order == 1 && m->model != goal::MODEL_ELASTIC;
+  return m->tangent == 64 &&
+         (m->d->mesh.order == 2 ? m->quad_order == 2 && m->model == goal::MODEL_NEOHOOKEAN
+                                : m->quad_order == 1 && m->model != goal::MODEL_ELASTIC);
 }
-bool clustered(goal_mech m) {
-  return m->tangent == 64 && uses_clusters(m) && m->d->cluster && m->d->cluster->num_runs > 0;
+// The node clusters an assembly takes, or null: then it takes the element pass
+// and the gather.  Made by the disc's first Jacobian that can take them, so
+// that meshes which only assemble residuals, functionals or features never pay
+// for them.  A first Jacobian that must not allocate settles the disc on the two
+// passes: all Jacobians of a disc have the same bits.
+const ClusterPlan* clusters_of(goal_mech m, bool may_alloc) {
+  if (!uses_clusters(m)) return nullptr;
+  goal_disc d = m->d;
+  std::lock_guard<std::mutex> one(d->cluster_mutex);  // several threads may assemble mechanics of one disc
+  if (!d->cluster) {
+    if (!may_alloc) d->cluster = std::make_unique<ClusterPlan>();
+    else d->cluster = d->mesh.order == 2 ? cluster_build(d) : linear_cluster_build(d);
+  }
+  return d->cluster->num_runs > 0 ? d->cluster.get() : nullptr;
 }
 
 // Linear elements: the point states in pt (kLinearPoint doubles an element), then the blocks.
-void run_linear_clustered(goal_mech m, goal_solinfo s, int kind, goal::AsmArgs a, double* pt) {
+void run_linear_clustered(goal_mech m, goal_solinfo s, int kind, const ClusterPlan& p, goal::AsmArgs a, double* pt) {
   goal_disc d = m->d;
-  const ClusterPlan& p = *d->cluster;
   if (!pt) {
     const int64_t n = goal::kLinearPoint * d->mesh.num_elems;
     if (m->linear_pt.n < n) m->linear_pt.alloc(n);
@@ -800,11 +826,11 @@ void run_linear_clustered(goal_mech m, goal_solinfo s, int kind, goal::AsmArgs a
   goal::LinearArgs c{};
   c.num_runs = p.num_runs;
   c.num_elems = a.num_elems;
-  c.runs = p.runs.p;
-  c.spans = p.spans.p;
-  c.elems = p.linear_elems.p;
-  c.lanes = p.lanes.p;
-  c.nodes = p.nodes.p;
+  c.runs = p.runs;
+  c.spans = p.spans;
+  c.elems = p.linear_elems;
+  c.lanes = p.lanes;
+  c.nodes = p.nodes;
   c.row_ptr = d->row_ptr.p;
   c.pt = pt;
   c.R = s->R.p;
@@ -825,18 +851,17 @@ void run_linear_clustered(goal_mech m, goal_solinfo s, int kind, goal::AsmArgs a
   s->zero_R = s->zero_vals = s->zero_dMdu = false;
 }
 
-void run_clustered(goal_mech m, goal_solinfo s, int kind, const goal::AsmArgs& a) {
+void run_clustered(goal_mech m, goal_solinfo s, int kind, const ClusterPlan& p, const goal::AsmArgs& a) {
   goal_disc d = m->d;
-  const ClusterPlan& p = *d->cluster;
   goal::ClusterArgs c{};
   c.num_runs = p.num_runs;
   c.num_elems = a.num_elems;
-  c.runs = p.runs.p;
-  c.chunks = p.chunks.p;
-  c.chunk_elems = p.elems.p;
-  c.chunk_conn = p.conn.p;
-  c.lanes = p.lanes.p;
-  c.nodes = p.nodes.p;
+  c.runs = p.runs;
+  c.chunks = p.chunks;
+  c.chunk_elems = p.elems;
+  c.chunk_conn = p.conn;
+  c.lanes = p.lanes;
+  c.nodes = p.nodes;
   c.row_ptr = d->row_ptr.p;
   c.coords = a.coords;
   c.x = a.x;
@@ -897,12 +922,12 @@ void run_residual(goal_mech m, goal_solinfo s, int kind, goal::AsmArgs a) {
 // first use); the two give the same bits.
 void run_assembly(goal_mech m, goal_solinfo s, int kind, goal::AsmArgs a, double* emr_buf = nullptr,
                   double* em_buf = nullptr, double* pt_buf = nullptr) {
-  if (clustered(m)) {
-    if (m->d->mesh.order == 2) run_clustered(m, s, kind, a);
-    else run_linear_clustered(m, s, kind, a, em_buf);  // a matrix buffer takes the smaller states
+  const bool own_buffers = emr_buf == nullptr;
+  if (const ClusterPlan* p = clusters_of(m, own_buffers)) {
+    if (m->d->mesh.order == 2) run_clustered(m, s, kind, *p, a);
+    else run_linear_clustered(m, s, kind, *p, a, em_buf);  // a matrix buffer takes the smaller states
     return;
   }
-  const bool own_buffers = emr_buf == nullptr;
   goal_disc d = m->d;
   const int64_t nd = 4 * (int64_t)d->mesh.nodes_per_elem;
   if (!emr_buf) {
@@ -2186,13 +2211,6 @@ int goal_mech_create(goal_disc d, goal_states st, int num_sets, const goal_mater
     m->status.alloc(1);
     HIPCHK(hipMemsetAsync(m->status.p, 0, sizeof(int), stream()));
     m->elem_value.alloc(d->mesh.num_elems);
-    if (uses_clusters(m.get())) {
-      std::lock_guard<std::mutex> one(d->cluster_mutex);  // mechanics of one disc may be made by several threads
-      if (!d->cluster) {
-        if (d->mesh.order == 2) cluster_build(d);
-        else linear_cluster_build(d);
-      }
-    }
     sync();
     *out = m.release();
     return GOAL_OK;

@@ -59,8 +59,11 @@ __device__ inline double from_ordered(unsigned long long u) {
   return __longlong_as_double((long long)((u >> 63) ? (u & 0x7fffffffffffffffull) : ~u));
 }
 
-// box[0..2], [3..5]: smallest and largest coordinates (ordered_bits), zero and ~0 before
+// box[0..2], [3..5]: smallest and largest coordinates (ordered_bits), ~0 and zero
+// before.  One atomic per workgroup and bound: with one per wave their turns on
+// six addresses took 280 us for 275 K nodes.
 __global__ __launch_bounds__(kBlock) void cluster_box_kernel(const double* X, int64_t nn, unsigned long long* box) {
+  __shared__ unsigned long long part[kBlock / 64][6];
   unsigned long long lo[3] = {~0ull, ~0ull, ~0ull}, hi[3] = {0, 0, 0};
   for (int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x; i < nn; i += (int64_t)gridDim.x * kBlock)
     for (int c = 0; c < 3; ++c) {
@@ -74,9 +77,17 @@ __global__ __launch_bounds__(kBlock) void cluster_box_kernel(const double* X, in
       hi[c] = max(hi[c], (unsigned long long)__shfl_xor((long long)hi[c], off, 64));
     }
     if ((threadIdx.x & 63) == 0) {
-      atomicMin(&box[c], lo[c]);
-      atomicMax(&box[3 + c], hi[c]);
+      part[threadIdx.x >> 6][c] = lo[c];
+      part[threadIdx.x >> 6][3 + c] = hi[c];
     }
+  }
+  __syncthreads();
+  if (threadIdx.x < 6) {
+    unsigned long long v = part[0][threadIdx.x];
+    for (int w = 1; w < kBlock / 64; ++w)
+      v = threadIdx.x < 3 ? min(v, part[w][threadIdx.x]) : max(v, part[w][threadIdx.x]);
+    if (threadIdx.x < 3) atomicMin(&box[threadIdx.x], v);
+    else atomicMax(&box[threadIdx.x], v);
   }
 }
 
@@ -140,12 +151,18 @@ __global__ __launch_bounds__(kBlock) void cluster_place_kernel(const int32_t* no
     place[nodes[i]] = (int32_t)i;
 }
 
+// One wavefront walks a key's part of the nodes.  Bound by the latency of a
+// node's loads.  P2 8^3: 25 us each, 64^3: 1.0 and 1.2 ms; one thread a key, which
+// looked an element up in its list entry by entry, took 270 us and 2.0 ms.
 __global__ __launch_bounds__(kBlock) void cluster_count_kernel(ClusterMesh m, const int64_t* seg, int64_t nn,
                                                                int32_t* runs, int32_t* more, int32_t* recs,
                                                                int32_t* most) {
-  for (int64_t a = (int64_t)blockIdx.x * kBlock + threadIdx.x; a <= nn; a += (int64_t)gridDim.x * kBlock) {
+  const int64_t waves = (int64_t)gridDim.x * (kBlock / 64);
+  for (int64_t a = (int64_t)blockIdx.x * (kBlock / 64) + (threadIdx.x >> 6); a <= nn; a += waves) {
     ClusterCount c;
-    if (a < nn && seg[a] < seg[a + 1]) walk_cluster(m, seg[a], seg[a + 1], c);
+    const int64_t lo = a < nn ? seg[a] : 0, hi = a < nn ? seg[a + 1] : 0;
+    if (lo < hi) walk_cluster(m, lo, hi, c);
+    if (threadIdx.x & 63) continue;
     runs[a] = c.runs;
     more[a] = c.chunks > c.runs ? c.chunks - c.runs : 0;
     recs[a] = c.recs;
@@ -158,8 +175,10 @@ __global__ __launch_bounds__(kBlock) void cluster_fill_kernel(ClusterMesh m, con
                                                               const int32_t* recs, int64_t num_runs, int4* run_tab,
                                                               int4* chunk_tab, int2* span_tab, uint32_t* elem_tab,
                                                               int2* rec_tab) {
-  for (int64_t a = (int64_t)blockIdx.x * kBlock + threadIdx.x; a < nn; a += (int64_t)gridDim.x * kBlock) {
-    if (seg[a] == seg[a + 1]) continue;
+  const int64_t waves = (int64_t)gridDim.x * (kBlock / 64);
+  for (int64_t a = (int64_t)blockIdx.x * (kBlock / 64) + (threadIdx.x >> 6); a < nn; a += waves) {
+    const int64_t lo = seg[a], hi = seg[a + 1];
+    if (lo == hi) continue;
     ClusterFill f;
     f.runs = run_tab;
     f.chunks = chunk_tab;
@@ -169,23 +188,78 @@ __global__ __launch_bounds__(kBlock) void cluster_fill_kernel(ClusterMesh m, con
     f.r = runs[a];
     f.x = (int)num_runs + more[a];
     f.k = recs[a];
-    walk_cluster(m, seg[a], seg[a + 1], f);
+    f.writes = (threadIdx.x & 63) == 0;
+    walk_cluster(m, lo, hi, f);
   }
 }
 
-// One workgroup per run: the pairs of each of its chunks, one thread per
-// (row node, position), the visits of a pair in incidence order.
+// out: four totals, for one read-back.
+__global__ void cluster_totals_kernel(const int32_t* a, const int32_t* b, const int32_t* c, const int32_t* d,
+                                      int4* out) {
+  *out = int4{*a, *b, *c, *d};
+}
+
+// First lane of every pair (block s < nb with cnt[s] > 0 visits): the pairs in
+// order of cluster_rank, then of s.  By groups of 64 blocks: a group's pairs of a
+// rank are counted by ballot, and the lanes before them are a prefix over ranks
+// and groups.  With one thread a pair that counted the pairs before it and then
+// looked through its node's incidences once a lane, the tables of 1.57 M linear
+// tets took 2 x 2.2 ms (sizes, then tables) and those of 83 K quadratic ones 2 x
+// 0.55; now 0.3 (linear_split counts the lanes too) and 1.1, and 2 x 0.26.
+constexpr int kRanks = 9, kGroups = kClusterSlots / 64;
+static_assert(kRanks * kGroups <= 128 && kGroups <= 64, "two entries a lane");
+__device__ void order_pairs(const int* cnt, int nb, int* before, uint16_t* at) {  // before: [kRanks * kGroups]
+  const int tid = threadIdx.x, lane = tid & 63;
+  for (int g = tid >> 6; g < kGroups; g += kBlock / 64) {
+    const int s = 64 * g + lane, rank = s < nb ? cluster_rank(cnt[s]) : kRanks;
+    for (int k = 0; k < kRanks; ++k) {
+      const unsigned long long b = __ballot(rank == k);
+      if (rank == k) at[s] = (uint16_t)(cluster_lanes_of_rank(k) * __popcll(b & ((1ull << lane) - 1)));
+      if (lane == 0) before[kGroups * k + g] = cluster_lanes_of_rank(k) * __popcll(b);
+    }
+  }
+  __syncthreads();
+  if (tid < 64) {
+    int carry = 0;
+    for (int i0 = 0; i0 < kRanks * kGroups; i0 += 64) {
+      const int i = i0 + lane, v = i < kRanks * kGroups ? before[i] : 0;
+      int sum = v;
+      for (int off = 1; off < 64; off <<= 1) {
+        const int o = __shfl_up(sum, off, 64);
+        if (lane >= off) sum += o;
+      }
+      if (i < kRanks * kGroups) before[i] = carry + sum - v;
+      carry += __shfl(sum, 63, 64);
+    }
+  }
+  __syncthreads();
+  for (int s = tid; s < nb; s += kBlock)
+    if (cnt[s]) at[s] = (uint16_t)(at[s] + before[kGroups * cluster_rank(cnt[s]) + s / 64]);
+  __syncthreads();
+}
+
+// The lanes that cnt's pairs take, added to *total (zero before).
+__device__ void count_lanes(int mine, int* total) {
+  for (int off = 32; off > 0; off >>= 1) mine += __shfl_xor(mine, off, 64);
+  if ((threadIdx.x & 63) == 0) atomicAdd(total, mine);
+  __syncthreads();
+}
+
+// One workgroup per run: the pairs of each of its chunks, one thread per visit
+// (row node's incidence, element node), the visits of a pair in incidence order.
 __global__ __launch_bounds__(kBlock) void cluster_lanes_kernel(ClusterMesh m, const int4* run_tab, int4* chunk_tab,
                                                                const int2* span_tab, const uint32_t* elem_tab,
                                                                const int2* recs, int32_t* nlanes,
                                                                ClusterLane* lanes) {
   constexpr int kRecs = 10 * kClusterElems;                // a chunk's incidences, at most
   __shared__ int first[kClusterNodes + 1];                 // first block of a node
-  __shared__ int rlo[kClusterNodes], rhi[kClusterNodes];   // a node's incidences in the chunk
+  __shared__ int rlo[kClusterNodes];                       // a node's first incidence in the chunk
   __shared__ uint16_t rpos[kRecs * 10];                    // their positions
   __shared__ int rinfo[kRecs];                             // element slot | local node << 8 | run-local node << 16
   __shared__ int cnt[kClusterSlots];                       // visits of a block's pair
-  __shared__ __align__(4) uint8_t rank[kClusterSlots + 4];
+  __shared__ int before[kRanks * kGroups];
+  __shared__ uint16_t at[kClusterSlots], src[kRecs * 10];  // first lane of a pair; a lane's first visit
+  __shared__ unsigned long long work[kRecs * 10];          // the visits of every lane
   __shared__ int total;
   const int tid = threadIdx.x;
   const int4 run = run_tab[blockIdx.x];
@@ -199,11 +273,11 @@ __global__ __launch_bounds__(kBlock) void cluster_lanes_kernel(ClusterMesh m, co
   if (tid == 0)
     for (int i = 0; i < nn; ++i) first[i + 1] += first[i];
   __syncthreads();
-  const int nb = first[nn], nb4 = (nb + 3) / 4 * 4;
+  const int nb = first[nn];
   for (int c = (int)blockIdx.x, nxt = run.z;; c = nxt++) {
     const int2 span = span_tab[c];
     const int nr = span.y - span.x;
-    if (tid < nn) rlo[tid] = rhi[tid] = 0;
+    if (tid < nn) rlo[tid] = 0;
     if (tid == 0) total = 0;
     for (int s = tid; s < nb; s += kBlock) cnt[s] = 0;
     for (int t = tid; t < nr; t += kBlock) rinfo[t] = recs[span.x + t].y;
@@ -212,72 +286,62 @@ __global__ __launch_bounds__(kBlock) void cluster_lanes_kernel(ClusterMesh m, co
     for (int t = tid; t < nr; t += kBlock) {
       const int node = rinfo[t] >> 16;
       if (t == 0 || (rinfo[t - 1] >> 16) != node) rlo[node] = t;
-      if (t + 1 == nr || (rinfo[t + 1] >> 16) != node) rhi[node] = t + 1;
     }
     for (int t = tid; t < 10 * nr; t += kBlock) atomicAdd(&cnt[first[rinfo[t / 10] >> 16] + rpos[t]], 1);
     __syncthreads();
-    for (int s = tid; s < nb4; s += kBlock) {
-      int n = s < nb ? cnt[s] : 0;
-      if (n) {
-        int node = 0;
-        while (first[node + 1] <= s) ++node;
-        const int64_t ga = m.nodes[run.x + node], gb = m.cols[m.row_ptr[4 * ga] + 4 * (s - first[node])] / 4;
-        if (m.place[gb] < m.place[ga]) n = cnt[s] = 0;  // the pair is b's run's
-        else atomicAdd(&total, 1 << cluster_log_lanes(n));
-      }
-      rank[s] = (uint8_t)cluster_rank(n);
+    int own = 0;
+    for (int s = tid; s < nb; s += kBlock) {
+      const int n = cnt[s];
+      if (!n) continue;
+      int node = 0;
+      while (first[node + 1] <= s) ++node;
+      const int64_t ga = m.nodes[run.x + node], gb = m.cols[m.row_ptr[4 * ga] + 4 * (s - first[node])] / 4;
+      if (m.place[gb] < m.place[ga]) cnt[s] = 0;  // the pair is b's run's
+      else own += 1 << cluster_log_lanes(n);
     }
-    __syncthreads();
+    count_lanes(own, &total);
     if (!lanes) {
       if (tid == 0) nlanes[c] = (total + 63) / 64 * 64;
     } else {
+      order_pairs(cnt, nb, before, at);
+      for (int l = tid; l < total; l += kBlock) work[l] = 0;
+      __syncthreads();
+      for (int i = tid; i < 10 * nr; i += kBlock) {
+        const int t = i / 10, b = i % 10, node = rinfo[t] >> 16, pos = rpos[i], n = cnt[first[node] + pos];
+        if (!n) continue;
+        int v = 0;  // visits of the pair before this one
+        for (int u = 10 * rlo[node]; u < i; ++u) v += rpos[u] == pos;
+        const int lg = cluster_log_lanes(n), lane = at[first[node] + pos] + (v & ((1 << lg) - 1));
+        const int code = (rinfo[t] & 31) | (((rinfo[t] >> 8) & 15) << 5) | (b << 9);
+        atomicOr(&work[lane], (unsigned long long)code << (13 * (v >> lg)));
+        if (!(v >> lg)) src[lane] = (uint16_t)i;
+      }
+      __syncthreads();
       const int base = nlanes[c], end = nlanes[c + 1];
       if (tid == 0) {
         chunk_tab[c].y = base;
         chunk_tab[c].z = end;
       }
-      for (int t = base + total + tid; t < end; t += kBlock) lanes[t] = ClusterLane{0, 0};  // idle lanes: no visits
-      for (int s = tid; s < nb; s += kBlock) {
-        const int n = cnt[s];
-        if (!n) continue;
-        const int mine = rank[s], lg = cluster_log_lanes(n);
-        int lane = 0;  // lanes of the pairs before this one
-        for (int u = 0; u < nb; u += 4) {
-          const uint32_t four = *reinterpret_cast<const uint32_t*>(rank + u);
-#pragma unroll
-          for (int k = 0; k < 4; ++k) {
-            const int ru = (four >> (8 * k)) & 255;
-            if (ru < mine || (ru == mine && u + k < s)) lane += ru < 9 ? cluster_lanes_of_rank(ru) : 0;
-          }
-        }
-        int node = 0;
-        while (first[node + 1] <= s) ++node;
-        const int pos = s - first[node];
-        const int64_t ga = m.nodes[run.x + node], gb = m.cols[m.row_ptr[4 * ga] + 4 * pos] / 4;
-        // an earlier chunk of the run that adds to this pair holds an earlier incidence of its node
-        bool earlier = false;
-        for (int64_t k = m.inc_ptr[ga]; k < recs[span.x + rlo[node]].x; ++k)
-          for (int b = 0; b < 10; ++b) earlier |= m.posi[10 * k + b] == pos;
-        uint16_t code[kClusterElems];
-        int at = 0;
-        for (int t = rlo[node]; t < rhi[node]; ++t)
-          for (int b = 0; b < 10; ++b)
-            if (rpos[10 * t + b] == pos && at < kClusterElems)
-              code[at++] = (uint16_t)((rinfo[t] & 31) | (((rinfo[t] >> 8) & 15) << 5) | (b << 9));
-        const int64_t e = elem_tab[(int64_t)c * kClusterElems + (code[0] & 31)] & ~kClusterOwned;
-        const int pos_t = m.pos[(10 * e + (code[0] >> 9)) * 10 + ((code[0] >> 5) & 15)];
-        const int64_t rb = m.row_ptr[4 * gb];
-        ClusterLane o;
-        o.y = (uint64_t)(rb / 16) | ((uint64_t)((m.row_ptr[4 * gb + 1] - rb) / 4) << kLaneDegT) |
-              ((uint64_t)pos_t << kLanePosT);
-        for (int j = 0; j < (1 << lg); ++j) {  // lane j's visits, in incidence order
-          uint64_t w = 0;
-          int k = 0;
-          for (int v = j; v < at; v += 1 << lg) w |= (uint64_t)code[v] << (13 * k++);
-          o.x = w | ((uint64_t)k << kLaneCount) | ((uint64_t)pos << kLanePos) | ((uint64_t)node << kLaneNode) |
+      for (int l = tid; l < end - base; l += kBlock) {
+        ClusterLane o = {0, 0};  // idle lanes: no visits
+        if (l < total) {
+          const int i = src[l], t = i / 10, b = i % 10, node = rinfo[t] >> 16, pos = rpos[i], s = first[node] + pos;
+          const int a = (rinfo[t] >> 8) & 15, lg = cluster_log_lanes(cnt[s]), j = l - at[s];
+          const int k = (cnt[s] - j + (1 << lg) - 1) >> lg;  // visits j, j + 2^lg, ..
+          const int64_t ga = m.nodes[run.x + node], gb = m.cols[m.row_ptr[4 * ga] + 4 * pos] / 4;
+          // an earlier chunk of the run that adds to this pair holds an earlier incidence of its node
+          bool earlier = false;
+          for (int64_t r = m.inc_ptr[ga]; r < recs[span.x + rlo[node]].x; ++r)
+            for (int q = 0; q < 10; ++q) earlier |= m.posi[10 * r + q] == pos;
+          const int64_t e = elem_tab[(int64_t)c * kClusterElems + (rinfo[t] & 31)] & ~kClusterOwned;
+          const int pos_t = m.pos[(10 * e + b) * 10 + a];
+          const int64_t rb = m.row_ptr[4 * gb];
+          o.x = work[l] | ((uint64_t)k << kLaneCount) | ((uint64_t)pos << kLanePos) | ((uint64_t)node << kLaneNode) |
                 ((uint64_t)lg << kLaneLog) | (earlier ? 0 : kLaneFirst) | (ga == gb ? kLaneDiag : 0);
-          lanes[base + lane + j] = o;
+          o.y = (uint64_t)(rb / 16) | ((uint64_t)((m.row_ptr[4 * gb + 1] - rb) / 4) << kLaneDegT) |
+                ((uint64_t)pos_t << kLanePosT);
         }
+        lanes[base + l] = o;
       }
     }
     __syncthreads();
@@ -731,28 +795,45 @@ __global__ __launch_bounds__(kClusterThreads, 3) void cluster_kernel(ClusterArgs
 // elements among them numbered by first appearance.
 struct LinearRun {
   int nodes[kLinearNodes], first[kLinearNodes + 1], rec0[kLinearNodes + 1];
-  int elem[kLinearRecs], info[kLinearRecs];  // element; first incidence of it << 2 | local node
-  uint16_t slot[kLinearRecs], pos[4 * kLinearRecs];
+  alignas(16) int elem[kLinearRecs];
+  int info[kLinearRecs];  // first incidence of the element << 2 | local node
+  alignas(8) uint16_t pos[4 * kLinearRecs];
+  uint16_t slot[kLinearRecs];
+  uint8_t node[kLinearRecs];
   int ne;
 };
 // false: too many incidences or blocks (nothing else is set then)
 __device__ bool linear_load(const ClusterMesh& m, int64_t lo, int64_t hi, LinearRun& r) {
+  static_assert(kLinearNodes == 8, "prefixes over eight lanes");
   const int tid = threadIdx.x, nn = (int)(hi - lo);
   __syncthreads();
-  if (tid == 0) {
-    r.first[0] = r.rec0[0] = 0;
-    for (int i = 0; i < nn; ++i) {
-      const int64_t n = m.nodes[lo + i];
-      r.nodes[i] = (int)n;
-      const int64_t deg = (m.row_ptr[4 * n + 1] - m.row_ptr[4 * n]) / 4, inc = m.inc_ptr[n + 1] - m.inc_ptr[n];
-      // no overflow: a node has at most 65535 neighbours, and once over a limit the sums only stay there
-      r.first[i + 1] = (int)min((int64_t)r.first[i] + deg, (int64_t)1 << 20);
-      r.rec0[i + 1] = (int)min((int64_t)r.rec0[i] + (inc > 0 ? inc : (int64_t)1 << 20), (int64_t)1 << 20);
+  if (tid < 64) {
+    // no overflow: eight terms of at most 2^20, which is over both limits; a node without elements ends here too
+    constexpr int64_t kMany = 1 << 20;
+    int deg = 0, inc = 0;
+    if (tid < nn) {
+      const int64_t n = m.nodes[lo + tid], d = (m.row_ptr[4 * n + 1] - m.row_ptr[4 * n]) / 4,
+                    k = m.inc_ptr[n + 1] - m.inc_ptr[n];
+      r.nodes[tid] = (int)n;
+      deg = (int)min(d, kMany);
+      inc = (int)(k > 0 ? min(k, kMany) : kMany);
     }
+    for (int off = 1; off < kLinearNodes; off <<= 1) {
+      const int d = __shfl_up(deg, off, 64), k = __shfl_up(inc, off, 64);
+      if (tid >= off) {
+        deg += d;
+        inc += k;
+      }
+    }
+    if (tid < nn) {
+      r.first[tid + 1] = deg;
+      r.rec0[tid + 1] = inc;
+    }
+    if (tid == 0) r.first[0] = r.rec0[0] = 0;
   }
   __syncthreads();
   const int n = r.rec0[nn];
-  if (n > kLinearRecs || r.first[nn] > kClusterSlots) return false;  // a node without elements ends here too
+  if (n > kLinearRecs || r.first[nn] > kClusterSlots) return false;
   for (int t = tid; t < n; t += kBlock) {
     int node = 0;
     while (r.rec0[node + 1] <= t) ++node;
@@ -760,13 +841,20 @@ __device__ bool linear_load(const ClusterMesh& m, int64_t lo, int64_t hi, Linear
     const int32_t s = m.inc[k];
     r.elem[t] = s / 4;
     r.info[t] = s % 4;
-    for (int b = 0; b < 4; ++b) r.pos[4 * t + b] = m.posi[4 * k + b];
+    r.node[t] = (uint8_t)node;
+    *reinterpret_cast<ushort4*>(r.pos + 4 * t) = reinterpret_cast<const ushort4*>(m.posi)[k];
   }
   __syncthreads();
   for (int t = tid; t < n; t += kBlock) {
     const int e = r.elem[t];
-    int u = 0;
-    while (r.elem[u] != e) ++u;
+    int u = 0;  // found at t at the latest
+    for (;; u += 4) {
+      const int4 v = *reinterpret_cast<const int4*>(r.elem + u);
+      if (v.x == e || v.y == e || v.z == e || v.w == e) {
+        u += v.x == e ? 0 : v.y == e ? 1 : v.z == e ? 2 : 3;
+        break;
+      }
+    }
     r.info[t] |= u << 2;
   }
   __syncthreads();
@@ -785,118 +873,123 @@ __device__ bool linear_load(const ClusterMesh& m, int64_t lo, int64_t hi, Linear
   return true;
 }
 
-// parts[g]: the runs (1, 2, 4 or 8) that group g's nodes need to fit.
+// cnt: the visits of every pair of a loaded run of rn nodes, 0 where the pair is
+// another run's.  The lanes they take.
+__device__ int linear_count(const ClusterMesh& m, const LinearRun& r, int rn, int* cnt, int* total) {
+  const int tid = threadIdx.x, n = r.rec0[rn], nb = r.first[rn];
+  if (tid == 0) *total = 0;
+  for (int s = tid; s < nb; s += kBlock) cnt[s] = 0;
+  __syncthreads();
+  for (int i = tid; i < 4 * n; i += kBlock) atomicAdd(&cnt[r.first[r.node[i >> 2]] + r.pos[i]], 1);
+  __syncthreads();
+  int own = 0;
+  for (int s = tid; s < nb; s += kBlock) {
+    const int c = cnt[s];
+    if (!c) continue;
+    int node = 0;
+    while (r.first[node + 1] <= s) ++node;
+    const int64_t ga = r.nodes[node], gb = m.cols[m.row_ptr[4 * ga] + 4 * (s - r.first[node])] / 4;
+    if (m.place[gb] < m.place[ga]) cnt[s] = 0;  // the pair is b's run's
+    else own += 1 << cluster_log_lanes(c);
+  }
+  count_lanes(own, total);
+  return *total;
+}
+
+// parts[g]: the runs (1, 2, 4 or 8) that group g's nodes need to fit; nlanes,
+// nelems [8 g + i]: the lanes (whole wavefronts) and elements of its run i, 0
+// where there is none.
 __global__ __launch_bounds__(kBlock) void linear_split_kernel(ClusterMesh m, int64_t nn, int32_t* parts,
-                                                              int32_t* bad) {
+                                                              int32_t* nlanes, int32_t* nelems, int32_t* bad) {
   __shared__ LinearRun r;
+  __shared__ int cnt[kClusterSlots], total;
+  __shared__ int2 size[kLinearNodes];
   const int64_t lo = (int64_t)blockIdx.x * kLinearNodes, hi = min(lo + kLinearNodes, nn);
   int p = 1;
   for (; p <= kLinearNodes; p *= 2) {
     const int64_t step = kLinearNodes / p;
     bool fits = true;
-    for (int64_t a = lo; a < hi && fits; a += step) fits = linear_load(m, a, min(a + step, hi), r) && r.ne <= kLinearElems;
+    int i = 0;
+    for (int64_t a = lo; a < hi && fits; a += step, ++i) {
+      const int64_t b = min(a + step, hi);
+      fits = linear_load(m, a, b, r) && r.ne <= kLinearElems;
+      if (!fits) break;
+      const int lanes = linear_count(m, r, (int)(b - a), cnt, &total);
+      if (threadIdx.x == 0) size[i] = int2{(lanes + 63) / 64 * 64, r.ne};
+    }
     if (fits) break;
   }
-  if (threadIdx.x) return;
-  if (p > kLinearNodes) {
-    atomicMax(bad, 1);
-    p = kLinearNodes;
+  __syncthreads();
+  const bool fit = p <= kLinearNodes;
+  const int64_t step = kLinearNodes / (fit ? p : kLinearNodes);
+  const int np = (int)((hi - lo + step - 1) / step), tid = threadIdx.x;
+  if (tid < kLinearNodes) {
+    nlanes[kLinearNodes * (int64_t)blockIdx.x + tid] = fit && tid < np ? size[tid].x : 0;
+    nelems[kLinearNodes * (int64_t)blockIdx.x + tid] = fit && tid < np ? size[tid].y : 0;
   }
-  const int64_t step = kLinearNodes / p;
-  parts[blockIdx.x] = (int)((hi - lo + step - 1) / step);
+  if (tid == 0) {
+    parts[blockIdx.x] = np;
+    if (!fit) atomicMax(bad, 1);
+  }
 }
 
 __global__ __launch_bounds__(kBlock) void linear_tables_kernel(ClusterMesh m, int64_t nn, const int32_t* parts,
-                                                               int32_t* nlanes, int32_t* nelems, int4* runs,
-                                                               int2* spans, int32_t* elems, ClusterLane* lanes) {
+                                                               const int32_t* nlanes, const int32_t* nelems,
+                                                               int4* runs, int2* spans, int32_t* elems,
+                                                               ClusterLane* lanes) {
   __shared__ LinearRun r;
-  __shared__ int cnt[kClusterSlots], total;
-  __shared__ __align__(4) uint8_t rank[kClusterSlots + 4];
+  __shared__ int cnt[kClusterSlots], before[kRanks * kGroups], total;
+  __shared__ uint16_t at[kClusterSlots], src[4 * kLinearRecs];  // first lane of a pair; a lane's first visit
+  __shared__ unsigned long long work[4 * kLinearRecs];          // the visits of every lane
   const int tid = threadIdx.x;
   const int64_t lo = (int64_t)blockIdx.x * kLinearNodes, hi = min(lo + kLinearNodes, nn);
   const int run0 = parts[blockIdx.x], np = parts[blockIdx.x + 1] - run0;
   int64_t step = kLinearNodes;  // np runs came from 1, 2, 4 or 8 equal parts of the group, the last ones empty at the end of the nodes
   while ((hi - lo + step - 1) / step < np) step /= 2;
   for (int p = 0; p < np; ++p) {
-    const int64_t a0 = lo + p * step, a1 = min(a0 + step, hi);
-    const int run = run0 + p;
+    const int64_t a0 = lo + p * step, a1 = min(a0 + step, hi), q = kLinearNodes * (int64_t)blockIdx.x + p;
+    const int run = run0 + p, rn = (int)(a1 - a0);
     linear_load(m, a0, a1, r);  // fits: linear_split saw to it
-    const int rn = (int)(a1 - a0), n = r.rec0[rn], nb = r.first[rn], nb4 = (nb + 3) / 4 * 4;
-    if (tid == 0) total = 0;
-    for (int s = tid; s < nb; s += kBlock) cnt[s] = 0;
+    linear_count(m, r, rn, cnt, &total);
+    order_pairs(cnt, r.first[rn], before, at);
+    for (int l = tid; l < total; l += kBlock) work[l] = 0;
     __syncthreads();
-    for (int t = tid; t < n; t += kBlock) {
-      int node = 0;
-      while (r.rec0[node + 1] <= t) ++node;
-      for (int b = 0; b < 4; ++b) atomicAdd(&cnt[r.first[node] + r.pos[4 * t + b]], 1);
-    }
-    __syncthreads();
-    for (int s = tid; s < nb4; s += kBlock) {
-      int c = s < nb ? cnt[s] : 0;
-      if (c) {
-        int node = 0;
-        while (r.first[node + 1] <= s) ++node;
-        const int64_t ga = r.nodes[node], gb = m.cols[m.row_ptr[4 * ga] + 4 * (s - r.first[node])] / 4;
-        if (m.place[gb] < m.place[ga]) c = cnt[s] = 0;  // the pair is b's run's
-        else atomicAdd(&total, 1 << cluster_log_lanes(c));
-      }
-      rank[s] = (uint8_t)cluster_rank(c);
-    }
-    __syncthreads();
-    if (!lanes) {
-      if (tid == 0) {
-        nlanes[run] = (total + 63) / 64 * 64;
-        nelems[run] = r.ne;
-      }
-      continue;
-    }
-    const int base = nlanes[run], end = nlanes[run + 1], e0 = nelems[run];
+    const int n = r.rec0[rn], base = nlanes[q], end = nlanes[q + 1], e0 = nelems[q];
     if (tid == 0) {
       runs[run] = int4{(int)a0, (int)a1, e0, r.ne};
       spans[run] = int2{base, end};
     }
     for (int t = tid; t < n; t += kBlock)
       if ((r.info[t] >> 2) == t) elems[e0 + r.slot[t]] = r.elem[t];
-    for (int t = base + total + tid; t < end; t += kBlock) lanes[t] = ClusterLane{0, 0};  // idle lanes: no visits
-    for (int s = tid; s < nb; s += kBlock) {
-      const int c = cnt[s];
+    for (int i = tid; i < 4 * n; i += kBlock) {
+      const int t = i >> 2, b = i & 3, node = r.node[t], pos = r.pos[i], s = r.first[node] + pos, c = cnt[s];
       if (!c) continue;
-      const int mine = rank[s], lg = cluster_log_lanes(c);
-      int lane = 0;  // lanes of the pairs before this one
-      for (int u = 0; u < nb; u += 4) {
-        const uint32_t four = *reinterpret_cast<const uint32_t*>(rank + u);
-#pragma unroll
-        for (int k = 0; k < 4; ++k) {
-          const int ru = (four >> (8 * k)) & 255;
-          if (ru < mine || (ru == mine && u + k < s)) lane += ru < 9 ? cluster_lanes_of_rank(ru) : 0;
-        }
+      int v = 0;  // visits of the pair before this one
+      for (int u = r.rec0[node]; u <= t; ++u) {
+        const ushort4 w = *reinterpret_cast<const ushort4*>(r.pos + 4 * u);
+        const bool all = u < t;
+        v += (w.x == pos && (all || b > 0)) + (w.y == pos && (all || b > 1)) + (w.z == pos && (all || b > 2)) +
+             (w.w == pos && all);
       }
-      int node = 0;
-      while (r.first[node + 1] <= s) ++node;
-      const int pos = s - r.first[node];
-      const int64_t ga = r.nodes[node], gb = m.cols[m.row_ptr[4 * ga] + 4 * pos] / 4;
-      const int64_t rb = m.row_ptr[4 * gb];
-      uint64_t pos_t = 0;
-      // lane j's visits, in incidence order: the pair's visits v = j, j + 2^lg, ..
-      for (int j = 0; j < (1 << lg); ++j) {
-        uint64_t w = 0;
-        int v = 0, k = 0;
-        for (int t = r.rec0[node]; t < r.rec0[node + 1]; ++t)
-          for (int b = 0; b < 4; ++b)
-            if (r.pos[4 * t + b] == pos) {
-              if ((v & ((1 << lg) - 1)) == j) {
-                const int a = r.info[t] & 3;
-                w |= (uint64_t)(r.slot[r.info[t] >> 2] | (a << 9) | (b << 11)) << (13 * k++);
-                pos_t = m.pos[((int64_t)r.elem[t] * 4 + b) * 4 + a];
-              }
-              ++v;
-            }
-        ClusterLane o;
-        o.x = w | ((uint64_t)k << kLaneCount) | ((uint64_t)pos << kLanePos) | ((uint64_t)node << kLaneNode) |
+      const int lg = cluster_log_lanes(c), lane = at[s] + (v & ((1 << lg) - 1));
+      const int code = r.slot[r.info[t] >> 2] | ((r.info[t] & 3) << 9) | (b << 11);
+      atomicOr(&work[lane], (unsigned long long)code << (13 * (v >> lg)));
+      if (!(v >> lg)) src[lane] = (uint16_t)i;
+    }
+    __syncthreads();
+    for (int l = tid; l < end - base; l += kBlock) {
+      ClusterLane o = {0, 0};  // idle lanes: no visits
+      if (l < total) {
+        const int i = src[l], t = i >> 2, b = i & 3, a = r.info[t] & 3, node = r.node[t], pos = r.pos[i];
+        const int s = r.first[node] + pos, lg = cluster_log_lanes(cnt[s]), j = l - at[s];
+        const int k = (cnt[s] - j + (1 << lg) - 1) >> lg;  // visits j, j + 2^lg, ..
+        const int64_t ga = r.nodes[node], gb = m.cols[m.row_ptr[4 * ga] + 4 * pos] / 4, rb = m.row_ptr[4 * gb];
+        const uint64_t pos_t = m.pos[((int64_t)r.elem[t] * 4 + b) * 4 + a];
+        o.x = work[l] | ((uint64_t)k << kLaneCount) | ((uint64_t)pos << kLanePos) | ((uint64_t)node << kLaneNode) |
               ((uint64_t)lg << kLaneLog) | kLaneFirst | (ga == gb ? kLaneDiag : 0);
         o.y = (uint64_t)(rb / 16) | ((uint64_t)((m.row_ptr[4 * gb + 1] - rb) / 4) << kLaneDegT) | (pos_t << kLanePosT);
-        lanes[base + lane + j] = o;
       }
+      lanes[base + l] = o;
     }
   }
 }
@@ -1273,7 +1366,7 @@ hipError_t morton_order(const double* coords, int64_t nn, void* temp, size_t tem
   hipError_t err = hipMemsetAsync(box, 0xff, 3 * sizeof(*box), s);
   if (err == hipSuccess) err = hipMemsetAsync(box + 3, 0, 3 * sizeof(*box), s);
   if (err != hipSuccess) return err;
-  hipLaunchKernelGGL(cluster_box_kernel, dim3(std::min(grid_for(nn), 1024u)), dim3(kBlock), 0, s, coords, nn, box);
+  hipLaunchKernelGGL(cluster_box_kernel, dim3(std::min(grid_for(nn), 256u)), dim3(kBlock), 0, s, coords, nn, box);
   hipLaunchKernelGGL(cluster_morton_kernel, dim3(grid_for(nn)), dim3(kBlock), 0, s, coords, nn, box, code, iota);
   err = hipGetLastError();
   if (err != hipSuccess) return err;
@@ -1306,7 +1399,7 @@ hipError_t cluster_order(const int32_t* conn, const double* coords, int64_t ne, 
 
 hipError_t cluster_count(const ClusterMesh& m, const int64_t* seg, int64_t nn, void* temp, size_t temp_bytes,
                          int32_t* runs, int32_t* more, int32_t* recs, int32_t* most, hipStream_t s) {
-  hipLaunchKernelGGL(cluster_count_kernel, dim3(grid_for(nn + 1)), dim3(kBlock), 0, s, m, seg, nn, runs, more, recs,
+  hipLaunchKernelGGL(cluster_count_kernel, dim3(grid_for(64 * (nn + 1))), dim3(kBlock), 0, s, m, seg, nn, runs, more, recs,
                      most);
   hipError_t err = hipGetLastError();
   for (int32_t* v : {runs, more, recs}) {
@@ -1317,10 +1410,16 @@ hipError_t cluster_count(const ClusterMesh& m, const int64_t* seg, int64_t nn, v
   return err;
 }
 
+hipError_t cluster_totals(const int32_t* a, const int32_t* b, const int32_t* c, const int32_t* d, int4* out,
+                          hipStream_t s) {
+  hipLaunchKernelGGL(cluster_totals_kernel, dim3(1), dim3(1), 0, s, a, b, c, d, out);
+  return hipGetLastError();
+}
+
 hipError_t cluster_fill(const ClusterMesh& m, const int64_t* seg, int64_t nn, const int32_t* runs,
                         const int32_t* more, const int32_t* recs, int64_t num_runs, int4* run_tab, int4* chunk_tab,
                         int2* span_tab, uint32_t* elem_tab, int2* rec_tab, hipStream_t s) {
-  hipLaunchKernelGGL(cluster_fill_kernel, dim3(grid_for(nn)), dim3(kBlock), 0, s, m, seg, nn, runs, more, recs,
+  hipLaunchKernelGGL(cluster_fill_kernel, dim3(grid_for(64 * nn)), dim3(kBlock), 0, s, m, seg, nn, runs, more, recs,
                      num_runs, run_tab, chunk_tab, span_tab, elem_tab, rec_tab);
   return hipGetLastError();
 }
@@ -1349,28 +1448,27 @@ hipError_t linear_order(const double* coords, int64_t nn, void* temp, size_t tem
   return morton_order(coords, nn, temp, temp_bytes, box, code, code_sorted, place, place, nodes, s);
 }
 
-hipError_t linear_split(const ClusterMesh& m, int64_t nn, void* temp, size_t temp_bytes, int32_t* parts, int32_t* bad,
-                        hipStream_t s) {
-  const int64_t groups = (nn + kLinearNodes - 1) / kLinearNodes;
-  hipLaunchKernelGGL(linear_split_kernel, dim3((unsigned)groups), dim3(kBlock), 0, s, m, nn, parts, bad);
+hipError_t linear_split(const ClusterMesh& m, int64_t nn, void* temp, size_t temp_bytes, int32_t* parts,
+                        int32_t* nlanes, int32_t* nelems, int32_t* bad, int4* totals, hipStream_t s) {
+  const int64_t groups = (nn + kLinearNodes - 1) / kLinearNodes, most = kLinearNodes * groups;
+  hipLaunchKernelGGL(linear_split_kernel, dim3((unsigned)groups), dim3(kBlock), 0, s, m, nn, parts, nlanes, nelems,
+                     bad);
   hipError_t err = hipGetLastError();
-  if (err != hipSuccess) return err;
-  return hipcub::DeviceScan::ExclusiveSum(temp, temp_bytes, parts, parts, (int)(groups + 1), s);
+  for (int32_t* v : {parts, nlanes, nelems}) {
+    if (err != hipSuccess) return err;
+    size_t tb = temp_bytes;
+    err = hipcub::DeviceScan::ExclusiveSum(temp, tb, v, v, (int)((v == parts ? groups : most) + 1), s);
+  }
+  return err != hipSuccess ? err : cluster_totals(parts + groups, nlanes + most, nelems + most, bad, totals, s);
 }
 
-hipError_t linear_tables(const ClusterMesh& m, int64_t nn, int64_t num_runs, const int32_t* parts, void* temp,
-                         size_t temp_bytes, int32_t* nlanes, int32_t* nelems, int4* runs, int2* spans, int32_t* elems,
-                         ClusterLane* lanes, hipStream_t s) {
+hipError_t linear_tables(const ClusterMesh& m, int64_t nn, const int32_t* parts, const int32_t* nlanes,
+                         const int32_t* nelems, int4* runs, int2* spans, int32_t* elems, ClusterLane* lanes,
+                         hipStream_t s) {
   const int64_t groups = (nn + kLinearNodes - 1) / kLinearNodes;
   hipLaunchKernelGGL(linear_tables_kernel, dim3((unsigned)groups), dim3(kBlock), 0, s, m, nn, parts, nlanes, nelems,
                      runs, spans, elems, lanes);
-  hipError_t err = hipGetLastError();
-  if (err != hipSuccess || lanes) return err;
-  size_t tb = temp_bytes;
-  err = hipcub::DeviceScan::ExclusiveSum(temp, tb, nlanes, nlanes, (int)(num_runs + 1), s);
-  if (err != hipSuccess) return err;
-  tb = temp_bytes;
-  return hipcub::DeviceScan::ExclusiveSum(temp, tb, nelems, nelems, (int)(num_runs + 1), s);
+  return hipGetLastError();
 }
 
 hipError_t launch_linear_points(const AsmArgs& a, hipStream_t s) {

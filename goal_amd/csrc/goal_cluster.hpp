@@ -41,76 +41,96 @@ struct ClusterMesh {
   const int32_t* place;    // [nodes] place in the ordered list
 };
 
-// Cuts the nodes [lo, hi) into runs and chunks, in order.  The sink's calls:
+// Cuts the nodes [lo, hi) into runs and chunks, in order; a wavefront's work (all
+// 64 lanes with the same arguments).  Lane s keeps the open chunk's element s, so
+// that looking an element up is one ballot; nodes and incidences come in 64 at a
+// time.  The sink's calls:
 //   run(node_lo)                            a run begins at this place of the list
 //   chunk()                                 a chunk begins
-//   elem(slot, e), own(slot)                the chunk's element in a slot; it writes the element's states
 //   rec(k, slot, a, node)                   an incidence: record k, element slot, local node, run-local node
-//   end_chunk(nelem), end_run(node_hi, blocks)
+//   end_chunk(nelem, elem, own)             its elements, one a lane, and which of them (bits) have their states
+//                                           written by this chunk
+//   end_run(node_hi, blocks)
 //   bare()                                  a node without elements
 template <typename Sink>
-__host__ __device__ inline void walk_cluster(const ClusterMesh& m, int64_t lo, int64_t hi, Sink& out) {
-  int32_t elems[kClusterElems];
+__device__ inline void walk_cluster(const ClusterMesh& m, int64_t lo, int64_t hi, Sink& out) {
+  const int lane = threadIdx.x & 63;
+  int32_t mine = -1;  // the open chunk's element in this lane's slot
+  uint32_t own = 0;
   int ne = 0, nn = 0;
   int64_t nb = 0;
   bool open_run = false, open_chunk = false;
-  for (int64_t i = lo; i < hi; ++i) {
-    const int64_t n = m.nodes[i];
-    const int64_t deg = (m.row_ptr[4 * n + 1] - m.row_ptr[4 * n]) / 4;
-    if (m.inc_ptr[n] == m.inc_ptr[n + 1]) out.bare();
-    if (open_run && (nn == kClusterNodes || nb + deg > kClusterSlots)) {
-      if (open_chunk) out.end_chunk(ne);
-      open_chunk = false;
-      out.end_run(i, nb);
-      open_run = false;
+  for (int64_t i0 = lo; i0 < hi; i0 += 64) {
+    int deg_l = 0;
+    int64_t k0_l = 0, k1_l = 0;
+    if (i0 + lane < hi) {
+      const int64_t n = m.nodes[i0 + lane];
+      deg_l = (int)((m.row_ptr[4 * n + 1] - m.row_ptr[4 * n]) / 4);
+      k0_l = m.inc_ptr[n];
+      k1_l = m.inc_ptr[n + 1];
     }
-    if (!open_run) {
-      out.run(i);
-      open_run = true;
-      nn = 0;
-      nb = 0;
-    }
-    for (int64_t k = m.inc_ptr[n]; k < m.inc_ptr[n + 1]; ++k) {
-      const int32_t e = m.inc[k] / 10, a = m.inc[k] % 10;
-      int s = 0;
-      if (open_chunk) {
-        while (s < ne && elems[s] != e) ++s;
-        if (s == kClusterElems) {
-          out.end_chunk(ne);
-          open_chunk = false;
+    const int some = hi - i0 < 64 ? (int)(hi - i0) : 64;
+    for (int l = 0; l < some; ++l) {
+      const int64_t i = i0 + l, k0 = __shfl(k0_l, l, 64), k1 = __shfl(k1_l, l, 64);
+      const int deg = __builtin_amdgcn_readlane(deg_l, l);
+      if (k0 == k1) out.bare();
+      if (open_run && (nn == kClusterNodes || nb + deg > kClusterSlots)) {
+        if (open_chunk) out.end_chunk(ne, mine, own);
+        open_chunk = false;
+        out.end_run(i, nb);
+        open_run = false;
+      }
+      if (!open_run) {
+        out.run(i);
+        open_run = true;
+        nn = 0;
+        nb = 0;
+      }
+      for (int64_t kb = k0; kb < k1; kb += 64) {
+        const int32_t inc_l = kb + lane < k1 ? m.inc[kb + lane] : 0;
+        const int incs = k1 - kb < 64 ? (int)(k1 - kb) : 64;
+        for (int j = 0; j < incs; ++j) {
+          const int32_t v = __builtin_amdgcn_readlane(inc_l, j), e = v / 10, a = v % 10;
+          int s = 0;
+          if (open_chunk) {
+            const unsigned long long same = __ballot(lane < ne && mine == e);
+            s = same ? __ffsll(same) - 1 : ne;
+            if (s == kClusterElems) {
+              out.end_chunk(ne, mine, own);
+              open_chunk = false;
+            }
+          }
+          if (!open_chunk) {
+            out.chunk();
+            open_chunk = true;
+            ne = s = 0;
+            own = 0;
+          }
+          if (s == ne) {
+            if (lane == s) mine = e;
+            ++ne;
+          }
+          if (a == 0) own |= 1u << s;
+          out.rec(kb + j, s, a, nn);
         }
       }
-      if (!open_chunk) {
-        out.chunk();
-        open_chunk = true;
-        ne = s = 0;
-      }
-      if (s == ne) {
-        elems[s] = e;
-        out.elem(s, e);
-        ++ne;
-      }
-      if (a == 0) out.own(s);
-      out.rec(k, s, a, nn);
+      nb += deg;
+      ++nn;
     }
-    nb += deg;
-    ++nn;
   }
-  if (open_chunk) out.end_chunk(ne);
+  if (open_chunk) out.end_chunk(ne, mine, own);
   if (open_run) out.end_run(hi, nb);
 }
 
-// Sinks: the sizes of one key's part, and the tables themselves.
+// Sinks: the sizes of one key's part, and the tables themselves (written by lane 0).
 struct ClusterCount {
   int runs = 0, chunks = 0, recs = 0, most = 0;  // most: blocks of the largest run, kClusterSlots + 1 with a bare node
-  __host__ __device__ void run(int64_t) { ++runs; }
-  __host__ __device__ void chunk() { ++chunks; }
-  __host__ __device__ void elem(int, int32_t) {}
-  __host__ __device__ void own(int) {}
-  __host__ __device__ void rec(int64_t, int, int, int) { ++recs; }
-  __host__ __device__ void end_chunk(int) {}
-  __host__ __device__ void end_run(int64_t, int64_t nb) { most = nb > most ? (int)nb : most; }
-  __host__ __device__ void bare() { most = most > kClusterSlots ? most : kClusterSlots + 1; }
+  __device__ void run(int64_t) { ++runs; }
+  __device__ void chunk() { ++chunks; }
+  __device__ void rec(int64_t, int, int, int) { ++recs; }
+  __device__ void end_chunk(int, int32_t, uint32_t) {}
+  __device__ void end_run(int64_t, int64_t nb) { most = nb > most ? (int)nb : most; }
+  __device__ void bare() { most = most > kClusterSlots ? most : kClusterSlots + 1; }
 };
 struct ClusterFill {
   // Chunk r is the first of run r; a run's further chunks follow all runs.
@@ -120,34 +140,36 @@ struct ClusterFill {
   uint32_t* elems;  // [chunks][kClusterElems] element | kClusterOwned
   int2* recs;       // [incidences] record, slot | local node << 8 | run-local node << 16
   int r, x, k;      // the next run, further chunk and incidence
+  bool writes;      // lane 0
   int c, in_run;
   int4 cur;
-  __host__ __device__ void run(int64_t node_lo) {
+  __device__ void run(int64_t node_lo) {
     cur.x = (int)node_lo;
     cur.z = x;
     in_run = 0;
   }
-  __host__ __device__ void chunk() {
+  __device__ void chunk() {
     c = in_run++ ? x++ : r;
-    spans[c].x = k;
+    if (writes) spans[c].x = k;
   }
-  __host__ __device__ void elem(int s, int32_t e) { elems[(int64_t)c * kClusterElems + s] = (uint32_t)e; }
-  __host__ __device__ void own(int s) { elems[(int64_t)c * kClusterElems + s] |= kClusterOwned; }
-  __host__ __device__ void rec(int64_t rk, int s, int a, int node) {
-    recs[k].x = (int)rk;
-    recs[k].y = s | (a << 8) | (node << 16);
+  __device__ void rec(int64_t rk, int s, int a, int node) {
+    if (writes) recs[k] = int2{(int)rk, s | (a << 8) | (node << 16)};
     ++k;
   }
-  __host__ __device__ void end_chunk(int ne) {
+  __device__ void end_chunk(int ne, int32_t elem, uint32_t own) {
+    const int lane = threadIdx.x & 63;
+    if (lane < ne) elems[(int64_t)c * kClusterElems + lane] = (uint32_t)elem | ((own >> lane) & 1u ? kClusterOwned : 0u);
+    if (!writes) return;
     spans[c].y = k;
     chunks[c] = int4{ne, 0, 0, 0};
   }
-  __host__ __device__ void end_run(int64_t node_hi, int64_t) {
+  __device__ void end_run(int64_t node_hi, int64_t) {
     cur.y = (int)node_hi;
     cur.w = x;
-    runs[r++] = cur;
+    if (writes) runs[r] = cur;
+    ++r;
   }
-  __host__ __device__ void bare() {}
+  __device__ void bare() {}
 };
 
 // Lanes (as a power of two) of a pair with n visits.
@@ -184,7 +206,7 @@ struct alignas(16) ClusterLane {
 // element slot 9, local a 2, local b 2.
 constexpr int kLinearElems = 160;   // elements per run
 constexpr int kLinearNodes = 8;     // vertices per run
-constexpr int kLinearRecs = 1024;   // incidences per run
+constexpr int kLinearRecs = 4 * kLinearElems;  // incidences per run
 constexpr int kLinearPoint = 32;    // doubles per element
 static_assert(kLinearElems <= 3 * 64 && kLinearElems < 512 && kLinearNodes <= kClusterNodes, "the fields of a lane's work");
 struct LinearArgs {
@@ -247,18 +269,22 @@ hipError_t cluster_lanes(const ClusterMesh& m, int64_t num_runs, int64_t num_chu
                          int32_t* nlanes, void* temp, size_t temp_bytes, ClusterLane* lanes, hipStream_t s);
 hipError_t cluster_conn(int64_t num_chunks, const int4* chunk_tab, const uint32_t* elem_tab, const int32_t* conn,
                         int32_t* chunk_conn, hipStream_t s);
+// out: the four values, for one read-back.
+hipError_t cluster_totals(const int32_t* a, const int32_t* b, const int32_t* c, const int32_t* d, int4* out,
+                          hipStream_t s);
 // linear_split: runs per group of kLinearNodes ordered nodes into parts
-// [groups + 1] (then scanned), or a number above kLinearNodes into *bad when a
-// node's incidences do not fit a run.  linear_tables: with lanes null the
-// lanes (whole wavefronts) and elements of every run into nlanes, nelems
-// [runs + 1] (then scanned); else the tables.
+// [groups + 1], lanes (whole wavefronts) and elements of each run into nlanes
+// and nelems [kLinearNodes groups + 1], all scanned into starts; a number above
+// zero into *bad (zero before) when a node's incidences do not fit a run; the
+// numbers of runs, lanes and elements, and *bad, into *totals.  linear_tables:
+// the tables.
 hipError_t linear_order(const double* coords, int64_t nn, void* temp, size_t temp_bytes, unsigned long long* box,
                         uint32_t* code, uint32_t* code_sorted, int32_t* place, int32_t* nodes, hipStream_t s);
-hipError_t linear_split(const ClusterMesh& m, int64_t nn, void* temp, size_t temp_bytes, int32_t* parts, int32_t* bad,
-                        hipStream_t s);
-hipError_t linear_tables(const ClusterMesh& m, int64_t nn, int64_t num_runs, const int32_t* parts, void* temp,
-                         size_t temp_bytes, int32_t* nlanes, int32_t* nelems, int4* runs, int2* spans, int32_t* elems,
-                         ClusterLane* lanes, hipStream_t s);
+hipError_t linear_split(const ClusterMesh& m, int64_t nn, void* temp, size_t temp_bytes, int32_t* parts,
+                        int32_t* nlanes, int32_t* nelems, int32_t* bad, int4* totals, hipStream_t s);
+hipError_t linear_tables(const ClusterMesh& m, int64_t nn, const int32_t* parts, const int32_t* nlanes,
+                         const int32_t* nelems, int4* runs, int2* spans, int32_t* elems, ClusterLane* lanes,
+                         hipStream_t s);
 // Point states of every element (model neo-Hookean or J2; states saved as asked) into a.pt.
 hipError_t launch_linear_points(const AsmArgs& a, hipStream_t s);
 hipError_t launch_linear_cluster(bool transpose, bool plastic, const LinearArgs& a, int blocks, hipStream_t s);

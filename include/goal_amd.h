@@ -286,7 +286,10 @@ int goal_asm_jacobian(goal_mech m, goal_solinfo s, int adjoint, int save_states)
  * library holds on each GPU until the process ends, so a mesh may have at most
  * 5,115 ten-node or 30,840 four-node tets (J2, whose point states take room
  * too: 3,748 ten-node four-point or 19,904 four-node one-point tets; larger
- * meshes: GOAL_ERR_INVALID, and nothing is launched).  Results are bitwise those of goal_asm_jacobian.  All
+ * meshes: GOAL_ERR_INVALID, and nothing is launched).  Results are bitwise those of goal_asm_jacobian.  The
+ * node clusters that FP64 Jacobians are summed over are made by a mesh's first
+ * goal_asm_jacobian, which allocates; where this entry point comes first, the
+ * mesh's Jacobians keep to the element matrices (slower: assemble once before).  All
  * calls on one GPU share the array: calls that overlap on one GPU (other
  * streams or threads) race.  Under capture, set the mechanics' "check" option
  * to 0 (the status read-back synchronizes). */
