@@ -24,7 +24,7 @@
 //   A  gather connectivity, vertex coordinates, DOFs        (element, DOF)
 //   B  shape functions                                       (element, point, node)
 //   C1 quadrature-point state: kinematics, model, states     (element, point)
-//   C2 one column of the 13x13 point tangent (J2, elastic)   (element, point, direction)
+//   C2 one column of the 13x13 point tangent (elastic)       (element, point, direction)
 //   D  residual rows                                         (element, row)
 //   E  Jacobian: a lane owns one column (b,k), forms C = D B
 //      and writes K(row, col) = B^T C for all rows           (element, column)
@@ -157,25 +157,25 @@ struct SPrefetch {
   double px[G][4 * NN];
 };
 struct SNoPrefetch {};
-// (FP64 element matrices and residuals, and the matrix-core kernels of either
+// (FP64 element matrices, and the matrix-core kernels of either
 // precision; the vector-ALU FP32-tangent kernels measured slightly slower
 // with it, 10.50 -> 10.55 ms, chunked beside the gather)
-template <int NN, int NQ, int MODEL, int KIND, typename TE>
+template <int NN, int NQ, int MODEL, typename TE>
 constexpr bool kPrefetch = MODEL == MODEL_NEOHOOKEAN && Layout<NN, NQ, MODEL>::T >= 128 &&
                            (std::is_same<TE, double>::value || Layout<NN, NQ, MODEL>::MF);
 
 // J2 assemblies take their point states from the thread-per-point pass
 // (j2_point_kernel) instead of phases C1 and C2.
-template <int MODEL, int KIND>
+template <int MODEL>
 constexpr bool kPointPass = MODEL == MODEL_J2;
 template <int NQ, int G>
 struct SJacD {
   double D[G][NQ][13][13];
 };
 
-template <int NN, int NQ, int MODEL, int KIND, int G, typename TE = double>
-struct Smem : std::conditional<kPrefetch<NN, NQ, MODEL, KIND, TE>, SPrefetch<NN, G>, SNoPrefetch>::type {
-  using Ext = typename std::conditional<kPointPass<MODEL, KIND>, SJacD<NQ, G>, SJac<NQ, MODEL, G, TE>>::type;
+template <int NN, int NQ, int MODEL, int G, typename TE = double>
+struct Smem : std::conditional<kPrefetch<NN, NQ, MODEL, TE>, SPrefetch<NN, G>, SNoPrefetch>::type {
+  using Ext = typename std::conditional<kPointPass<MODEL>, SJacD<NQ, G>, SJac<NQ, MODEL, G, TE>>::type;
   SBase<NN, NQ, G> b;
   Ext ext;
 };
@@ -183,11 +183,11 @@ struct Smem : std::conditional<kPrefetch<NN, NQ, MODEL, KIND, TE>, SPrefetch<NN,
 // (W, or GOAL_ELEM_WAVES for the J2 point-pass kinds), lowered to what the
 // workgroup's LDS allows (160 KB per CU), so the compiler is not held to an
 // occupancy the LDS rules out.
-template <int NN, int NQ, int MODEL, int KIND, typename TE>
+template <int NN, int NQ, int MODEL, typename TE>
 constexpr int elem_waves() {
   using Lay = Layout<NN, NQ, MODEL>;
-  constexpr int want = kPointPass<MODEL, KIND> ? GOAL_ELEM_WAVES : Lay::W;
-  constexpr int per_cu = 163840 / (int)sizeof(Smem<NN, NQ, MODEL, KIND, Lay::G, TE>);
+  constexpr int want = kPointPass<MODEL> ? GOAL_ELEM_WAVES : Lay::W;
+  constexpr int per_cu = 163840 / (int)sizeof(Smem<NN, NQ, MODEL, Lay::G, TE>);
   constexpr int lds = per_cu * (Lay::T / 64) / 4;
   return lds < 1 ? 1 : (lds < want ? lds : want);
 }
@@ -504,13 +504,13 @@ __device__ inline void mf_tile_product(const T* A, const T* C, const int32_t* re
 }
 
 template <int NN, int NQ, int MODEL, int KIND, typename TE>
-__global__ __launch_bounds__((Layout<NN, NQ, MODEL>::T), (elem_waves<NN, NQ, MODEL, KIND, TE>())) void element_kernel(
+__global__ __launch_bounds__((Layout<NN, NQ, MODEL>::T), (elem_waves<NN, NQ, MODEL, TE>())) void element_kernel(
     AsmArgs a) {
   using Lay = Layout<NN, NQ, MODEL>;
   using M = typename ModelOf<MODEL>::type;
   constexpr int G = Lay::G, ND = Lay::ND, T = Lay::T;
   static_assert(KIND == ASM_JACOBIAN || KIND == ASM_ADJOINT, "residuals have a kernel of their own");
-  __shared__ Smem<NN, NQ, MODEL, KIND, G, TE> sm;
+  __shared__ Smem<NN, NQ, MODEL, G, TE> sm;
   auto& s = sm.b;
   const int tid = threadIdx.x;
   const int64_t ne = a.num_elems;
@@ -526,7 +526,7 @@ __global__ __launch_bounds__((Layout<NN, NQ, MODEL>::T), (elem_waves<NN, NQ, MOD
   // J2 point-pass kinds: four-node tets load a group's point states into
   // registers one group ahead, so the loads are in flight during the previous
   // group's phases (ten-node tets have no registers to spare for it)
-  constexpr bool PP = kPointPass<MODEL, KIND>;
+  constexpr bool PP = kPointPass<MODEL>;
   constexpr int PPS = PP ? kPointTangent : 1;
   constexpr int NPF = PP ? (G * NQ * PPS + T - 1) / T : 1;
   constexpr bool PPF = PP && NN == 4 && NQ == 1;
@@ -543,7 +543,7 @@ __global__ __launch_bounds__((Layout<NN, NQ, MODEL>::T), (elem_waves<NN, NQ, MOD
     }
   };
   if constexpr (PPF) fetch_points(0);
-  if constexpr (kPointPass<MODEL, KIND>) {
+  if constexpr (kPointPass<MODEL>) {
     // the point tangent's structural zeros (s3 rows of the p column, P and r1
     // rows of the grad-p columns): never stored, never overwritten
     for (int t = tid; t < G * NQ * 33; t += T) {
@@ -562,7 +562,7 @@ __global__ __launch_bounds__((Layout<NN, NQ, MODEL>::T), (elem_waves<NN, NQ, MOD
     const int nv = (int)min((int64_t)G, ne - e0);  // elements of this group
 
     // ---- A: gather (Displacement/Pressure::gather, src/goal_displacement.cpp:139-156)
-    constexpr bool PF = kPrefetch<NN, NQ, MODEL, KIND, TE>;
+    constexpr bool PF = kPrefetch<NN, NQ, MODEL, TE>;
     if (PF && fetched) {
       // this group's data came in during the previous group's phase C1
       if constexpr (PF) {
@@ -583,7 +583,7 @@ __global__ __launch_bounds__((Layout<NN, NQ, MODEL>::T), (elem_waves<NN, NQ, MOD
       const int el = t / 12, c = t % 12;
       s.X[el][c / 3][c % 3] = a.coords[3 * (int64_t)s.conn[el][c / 3] + (c % 3)];
     }
-    if constexpr (!kPointPass<MODEL, KIND>)  // the point pass read the DOFs
+    if constexpr (!kPointPass<MODEL>)  // the point pass read the DOFs
       for (int t = tid; t < nv * ND; t += T) {
         const int el = t / ND, k = t % ND;
         const int64_t dof = 4 * (int64_t)s.conn[el][k >> 2] + (k & 3);
@@ -712,7 +712,7 @@ __global__ __launch_bounds__((Layout<NN, NQ, MODEL>::T), (elem_waves<NN, NQ, MOD
       }
       if constexpr (PPF) fetch_points(it + 1);
     }
-    if constexpr (!kPointPass<MODEL, KIND>) {
+    if constexpr (!kPointPass<MODEL>) {
       for (int t = tid; t < nv * NQ; t += T) {
         const int el = t / NQ, q = t % NQ;
         const int64_t e = e0 + el;
@@ -780,7 +780,7 @@ __global__ __launch_bounds__((Layout<NN, NQ, MODEL>::T), (elem_waves<NN, NQ, MOD
     __syncthreads();
 
     // ---- C2: tangent columns d sig / d F_kL, one (element, point, direction) per lane
-    if constexpr (MODEL != MODEL_NEOHOOKEAN && !kPointPass<MODEL, KIND>) {
+    if constexpr (MODEL != MODEL_NEOHOOKEAN && !kPointPass<MODEL>) {
       for (int t = tid; t < nv * NQ * 9; t += T) {
         const int el = t / (NQ * 9), r = t % (NQ * 9);
         const int q = r / 9, c = r % 9;
@@ -916,6 +916,10 @@ constexpr int kGatherThreads = 256;  // four waves: one per equation
 constexpr int kGatherRecords = 256;  // incidence records staged per chunk
 constexpr int kGatherNodes = 64;     // nodes per run, at most
 
+// g.vals and g.R are always given.  Their tests stay: without them the compiler
+// allocates the four-node instances' registers differently and the gather of 1.3 M
+// linear tets takes 0.83 ms instead of 0.70 (FP64), 0.51 instead of 0.48 (FP32); the
+// ten-node ones are the same either way.
 template <int NN, typename TE>
 __global__ __launch_bounds__(kGatherThreads) void gather_kernel(GatherArgs g) {
   constexpr int ND = 4 * NN, RB = 4 * ND, NT = kGatherThreads, RC = kGatherRecords, NC = kGatherNodes;
@@ -1168,7 +1172,7 @@ int resident_grid(int64_t ne) {
 
 template <int NN, int NQ, int MODEL, int KIND, typename TE>
 hipError_t launch4(const AsmArgs& a, int blocks, hipStream_t s) {
-  if constexpr (kPointPass<MODEL, KIND>) {
+  if constexpr (kPointPass<MODEL>) {
     if (!a.pt) return hipErrorInvalidValue;
     const int64_t npts = a.num_elems * NQ;
     const int pb = (int)std::min<int64_t>((npts + 255) / 256, 65536);

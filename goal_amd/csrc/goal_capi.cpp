@@ -290,8 +290,6 @@ struct goal_states_s {
   DevBuf<double> sigma, eqps, eqps_old, Fp, Fp_old;
 };
 
-// zero_* only mark a buffer as pending zero; the next assembly then writes
-// it instead of adding to it, and any other access fills it first.
 // Pinned host memory that a kernel writes results to, and the event after it:
 // the host waits for those results alone, with later work already queued.
 struct ReadBack {
@@ -318,6 +316,8 @@ struct ReadBack {
   void wait() { HIPCHK(hipEventSynchronize(done)); }
 };
 
+// zero_* only mark a buffer as pending zero; the next assembly then writes
+// it instead of adding to it, and any other access fills it first.
 struct goal_solinfo_s {
   goal_disc d = nullptr;
   DevBuf<double> R, dMdu, vals;
@@ -679,7 +679,8 @@ goal::AsmArgs asm_args(goal_mech m) {
   return a;
 }
 
-// 0 lets the launcher size a persistent grid from the kernel's occupancy.
+// 0 lets the launcher size the grid: the element pass a persistent one from the
+// kernel's occupancy, the cluster kernels one workgroup per run.
 int asm_blocks(goal_mech m) { return m->blocks; }
 
 
@@ -691,7 +692,6 @@ void materialize(goal_solinfo s) {
   s->zero_R = s->zero_dMdu = s->zero_vals = false;
 }
 
-// Element pass + node gather.  want_vals: Jacobian assembly.
 // Chunked assembly (neo-Hookean; option "overlap" = K chunks).  The element
 // groups are split into K consecutive chunks on the library stream; after
 // chunk c, the node runs whose incident elements all lie in chunks <= c are
@@ -783,9 +783,7 @@ void run_chunked(goal_mech m, goal_solinfo s, int kind, goal::AsmArgs a) {
   s->zero_R = s->zero_vals = false;
 }
 
-// Element buffers between the two passes: the mechanics' own (allocated on
-// first use), or, with emr_buf/em_buf given, the caller's.
-// Doubles of J2 point states an assembly of this kind needs (0: none).
+// Doubles of J2 point states between the point pass and the element pass (0: none).
 int64_t point_states(goal_mech m) {
   if (m->model != goal::MODEL_J2) return 0;
   return goal::point_state_doubles(m->d->mesh.num_elems * m->st->nq, goal::kPointTangent);
@@ -917,9 +915,11 @@ void run_residual(goal_mech m, goal_solinfo s, int kind, goal::AsmArgs a) {
   }
 }
 
-// Residual and Jacobian.  With emr_buf given (and pt_buf for J2) the assembly
-// also stays in one pass (the chunked path keeps a host-side table it builds on
-// first use); the two give the same bits.
+// Residual and Jacobian.  The element buffers between the two passes are the
+// mechanics' own (allocated on first use) or, with emr_buf and em_buf (and pt_buf
+// for J2) given, the caller's; the assembly then also stays in one pass (the
+// chunked path keeps a host-side table it builds on first use).  The same bits
+// either way.
 void run_assembly(goal_mech m, goal_solinfo s, int kind, goal::AsmArgs a, double* emr_buf = nullptr,
                   double* em_buf = nullptr, double* pt_buf = nullptr) {
   const bool own_buffers = emr_buf == nullptr;

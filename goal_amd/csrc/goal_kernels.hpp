@@ -40,7 +40,7 @@ struct AsmArgs {
   // a node sums are contiguous.  emr[k][4], em[k][4][4*npe] (for
   // ASM_ADJOINT the row blocks of the transposed element matrix).
   double* emr;
-  double* em;               // null: residual only
+  double* em;               // or em32
   float* em32;              // FP32 element matrices instead of em (FP32 tangent)
   // per quadrature point history, structure of arrays: comp * (ne*nq) + e*nq + q
   const double* Fp_old;
@@ -94,10 +94,10 @@ struct GatherArgs {
   const uint16_t* posi;     // [records][npe] position of each element node in adj(node)
   const int64_t* row_ptr;   // [num_dofs + 1]
   const double* emr;        // node-major, see AsmArgs
-  const double* em;         // null: residual only
+  const double* em;         // or em32
   const float* em32;        // FP32 element matrices instead of em
-  double* R;                // null: skip
-  double* vals;             // null: skip
+  double* R;
+  double* vals;
   int overwrite_R;          // 1: R = sum (R was pending zero), 0: R += sum
   int overwrite_vals;
 };

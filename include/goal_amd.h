@@ -340,7 +340,8 @@ int goal_batch_destroy(goal_batch b);
 /* Autotuner: for each mesh, time `reps` assemblies with each candidate
  * persistent-grid size (the occupancy-sized grid and multiples of the CU
  * count) and keep the fastest as its "blocks" option.  Outputs (may be NULL):
- * the chosen grid (0 = occupancy-sized) and its median time in ms per mesh.
+ * the chosen grid (0: occupancy-sized, over node clusters one workgroup per run)
+ * and its median time in ms per mesh.
  * A captured graph is dropped (capture again). */
 int goal_batch_tune(goal_batch b, int reps, int* blocks, float* ms);
 /* Capture the batch (one eager assembly per mesh first sizes the buffers).
