@@ -18,7 +18,7 @@
 //
 // Measured on the P2 64^3 cube (1.57 M tets; 7.8 GB of CSR values): 5.6 ms
 // against 12.7 ms for the element pass and the gather, whose 20.6 GB of element
-// matrices were written and read once.  HBM traffic 10.5 GB instead of 51.
+// matrices were written and read once.  HBM traffic 10.8 GB instead of 51.
 // Leaving out the blocks' sums takes 1.0-1.6 ms off, the point states 1.6-1.9,
 // the stores 1.4-1.7, and all three leave 1.1 ms: with four workgroups per CU
 // (LDS) the phases' latencies add up, the vector ALUs are busy for 2.7 ms.
