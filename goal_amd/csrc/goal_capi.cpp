@@ -232,11 +232,18 @@ struct Carve {
     return at;
   }
 };
+struct ArenaRef {
+  uint8_t* p = nullptr;
+  template <typename T>
+  T* at(size_t offset) const {
+    return reinterpret_cast<T*>(p + offset);
+  }
+};
 struct Arena : DevBuf<uint8_t> {
   void alloc(const Carve& c) { DevBuf<uint8_t>::alloc((int64_t)c.size); }
   template <typename T>
   T* at(size_t offset) const {
-    return reinterpret_cast<T*>(p + offset);
+    return ArenaRef{p}.at<T>(offset);
   }
 };
 
@@ -562,8 +569,10 @@ std::unique_ptr<ClusterPlan> cluster_build(goal_disc d) {
   return p;
 }
 
-// The same for linear elements.
-std::unique_ptr<ClusterPlan> linear_cluster_build(goal_disc d) {
+// The same for linear elements.  pt: the assembly's point states, not yet written,
+// whose memory serves as work space where it suffices (it does but for meshes of
+// few elements): an allocation and a release of some MB can take 0.3 ms each.
+std::unique_ptr<ClusterPlan> linear_cluster_build(goal_disc d, const DevBuf<double>& pt) {
   auto p = std::make_unique<ClusterPlan>();
   const int64_t nn = d->mesh.num_nodes, ne = d->mesh.num_elems;
   const int64_t groups = (nn + goal::kLinearNodes - 1) / goal::kLinearNodes, most = goal::kLinearNodes * groups;
@@ -576,8 +585,10 @@ std::unique_ptr<ClusterPlan> linear_cluster_build(goal_disc d) {
                o_totals = c.take<int4>(1), o_code = c.take<uint32_t>(2 * nn), o_place = c.take<int32_t>(nn),
                o_nodes = c.take<int32_t>(nn), o_parts = c.take<int32_t>(groups + 1),
                o_nlanes = c.take<int32_t>(most + 1), o_nelems = c.take<int32_t>(most + 1);
-  Arena work;
-  work.alloc(c);
+  Arena own;
+  const bool fits = c.size <= sizeof(double) * (size_t)pt.n;
+  if (!fits) own.alloc(c);
+  const ArenaRef work{fits ? reinterpret_cast<uint8_t*>(pt.p) : own.p};
   void* temp = work.at<void>(o_temp);
   uint32_t* code = work.at<uint32_t>(o_code);
   int32_t *place = work.at<int32_t>(o_place), *nodes = work.at<int32_t>(o_nodes), *parts = work.at<int32_t>(o_parts),
@@ -796,6 +807,13 @@ bool uses_clusters(const goal_mech_s* m) {
          (m->d->mesh.order == 2 ? m->quad_order == 2 && m->model == goal::MODEL_NEOHOOKEAN
                                 : m->quad_order == 1 && m->model != goal::MODEL_ELASTIC);
 }
+// Linear elements' point states: the mechanics' own, allocated on first use.
+double* linear_states(goal_mech m) {
+  const int64_t n = goal::kLinearPoint * m->d->mesh.num_elems;
+  if (m->linear_pt.n < n) m->linear_pt.alloc(n);
+  return m->linear_pt.p;
+}
+
 // The node clusters an assembly takes, or null: then it takes the element pass
 // and the gather.  Made by the disc's first Jacobian that can take them, so
 // that meshes which only assemble residuals, functionals or features never pay
@@ -806,8 +824,15 @@ const ClusterPlan* clusters_of(goal_mech m, bool may_alloc) {
   goal_disc d = m->d;
   std::lock_guard<std::mutex> one(d->cluster_mutex);  // several threads may assemble mechanics of one disc
   if (!d->cluster) {
-    if (!may_alloc) d->cluster = std::make_unique<ClusterPlan>();
-    else d->cluster = d->mesh.order == 2 ? cluster_build(d) : linear_cluster_build(d);
+    if (!may_alloc) {
+      d->cluster = std::make_unique<ClusterPlan>();
+    } else if (d->mesh.order == 2) {
+      d->cluster = cluster_build(d);
+    } else {
+      linear_states(m);
+      d->cluster = linear_cluster_build(d, m->linear_pt);
+      if (d->cluster->num_runs == 0) m->linear_pt.release();  // not needed after all
+    }
   }
   return d->cluster->num_runs > 0 ? d->cluster.get() : nullptr;
 }
@@ -815,11 +840,7 @@ const ClusterPlan* clusters_of(goal_mech m, bool may_alloc) {
 // Linear elements: the point states in pt (kLinearPoint doubles an element), then the blocks.
 void run_linear_clustered(goal_mech m, goal_solinfo s, int kind, const ClusterPlan& p, goal::AsmArgs a, double* pt) {
   goal_disc d = m->d;
-  if (!pt) {
-    const int64_t n = goal::kLinearPoint * d->mesh.num_elems;
-    if (m->linear_pt.n < n) m->linear_pt.alloc(n);
-    pt = m->linear_pt.p;
-  }
+  if (!pt) pt = linear_states(m);
   a.pt = pt;
   goal::LinearArgs c{};
   c.num_runs = p.num_runs;
