@@ -1216,7 +1216,7 @@ hipError_t launch2(int kind, const AsmArgs& a, int blocks, hipStream_t s) {
 // With emr set, the derivative of the element value w.r.t. the element DOFs
 // (what QoI<FADT>::scatter adds up, src/goal_qoi.cpp:63-76) goes to the
 // element's incidence records, to be summed by node.  1.57 M linear tets, von
-// Mises: 124 us and 42 for the sums, where FP64 atomics on the nodes took 1,097.
+// Mises: 123 us and 35 for the sums, where FP64 atomics on the nodes took 1,097.
 template <int NN, int NQ, int MODEL>
 __global__ __launch_bounds__(256) void qoi_kernel(QoiArgs a) {
   const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
