@@ -2330,7 +2330,8 @@ int goal_asm_jacobian_noalloc(goal_mech m, goal_solinfo s, int adjoint, int save
     goal::AsmArgs a = asm_args(m);  // ctx() is up: the mechanics was created through it
     const int64_t ne = m->d->mesh.num_elems, nd = 4 * (int64_t)m->d->mesh.nodes_per_elem;
     // element matrices (FP64; FP32 ones take half), element residuals, then
-    // (J2) the point states
+    // (J2) the point states; asked for over node clusters too, which need less:
+    // what is accepted does not depend on which of a mesh's Jacobians came first
     const int kind = adjoint ? goal::ASM_ADJOINT : goal::ASM_JACOBIAN;
     const bool pts = m->model == goal::MODEL_J2;
     auto need_of = [&](int64_t n) {
